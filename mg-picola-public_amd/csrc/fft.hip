@@ -42,19 +42,14 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_fft_col(float2 *__restric
   int bx, by;
   xcd_tile(bx, by);
   auto tile = [&](int i) { return buf + (size_t)(by * TPB + i) * outer_stride + (size_t)bx * T; };
-  if constexpr (TPB == 1) {
-    float2 *base = tile(0);
-    auto ld = [&](int c, int j, int o) { return (base + (size_t)j * line_stride + c)[(size_t)o * line_stride]; };
-    auto st = [&](int c, int j, int o, float2 v) { (base + (size_t)j * line_stride + c)[(size_t)o * line_stride] = v; };
-    fft_stages<L, T, NT, SIGN, 1, T, true, false, 1>(lds, tw, 1, tid, ld, st);
-    return;
-  }
+  StageTwiddles<L, T, NT> stw(tw, tid);
   float2 pre[E];
   {
     const float2 *base = tile(0);
     first_loads<L, T, NT, true>(
-        pre, tid, [&](int c, int j, int o) { return (base + (size_t)j * line_stride + c)[(size_t)o * line_stride]; });
+        pre, tid, [&](int c, int j, int o) { return col_at<L, T>(base, line_stride, c, j, o); });
   }
+  const float2 *twl = stw.to_lds(lds, tid);
 #pragma unroll
   for (int i = 0; i < TPB; ++i) {
     float2 cur[E];
@@ -63,12 +58,12 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_fft_col(float2 *__restric
     if (i + 1 < TPB) {
       const float2 *nb = tile(i + 1);
       first_loads<L, T, NT, true>(
-          pre, tid, [&](int c, int j, int o) { return (nb + (size_t)j * line_stride + c)[(size_t)o * line_stride]; });
+          pre, tid, [&](int c, int j, int o) { return col_at<L, T>(nb, line_stride, c, j, o); });
     }
     float2 *base = tile(i);
-    auto ld = [&](int c, int j, int o) { return (base + (size_t)j * line_stride + c)[(size_t)o * line_stride]; };
-    auto st = [&](int c, int j, int o, float2 v) { (base + (size_t)j * line_stride + c)[(size_t)o * line_stride] = v; };
-    fft_stages<L, T, NT, SIGN, 1, T, true, false, 1, false, true>(lds, tw, 1, tid, ld, st, cur);
+    auto ld = [&](int c, int j, int o) { return col_at<L, T>(base, line_stride, c, j, o); };
+    auto st = [&](int c, int j, int o, float2 v) { col_at<L, T>(base, line_stride, c, j, o) = v; };
+    fft_stages<L, T, NT, SIGN, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ld, st, cur);
     if (i + 1 < TPB) __syncthreads();  // the next tile's first exchange reuses the LDS
   }
 }
@@ -133,7 +128,7 @@ constexpr int col_tpb(int L) { return (L % 3 != 0 && L >= 256) ? MGPU_COL_TPB : 
 template <int L, int T, int SIGN>
 int launch_col(mgpu_ctx *ctx, float2 *buf, size_t line_stride, size_t outer_stride, int nouter, int ntiles,
                const float2 *tw) {
-  size_t lds = (size_t)L * T * sizeof(float2);
+  size_t lds = col_lds_elems(L, T) * sizeof(float2);
   constexpr int TPB = col_tpb(L);
   auto kern = k_fft_col<L, T, SIGN, TPB>;
   static_assert(L % TPB == 0, "outer count must be a multiple of the tiles per block");
@@ -194,9 +189,11 @@ bool fft_size_supported(int n) {
   }
 }
 
+size_t fft_col_lds(int n, int T) { return col_lds_elems(n, T) * sizeof(float2); }
+
 // 16-column tiles fit one workgroup's LDS and thread limit
 bool fft_tile16_fits(const mgpu_ctx *ctx, int n) {
-  const size_t need16 = (size_t)n * 16 * sizeof(float2);
+  const size_t need16 = fft_col_lds(n, 16);
   return need16 <= ctx->lds_max && n * 16 / elems_per_thread(n) <= 1024;
 }
 

@@ -151,7 +151,7 @@ constexpr int elems_per_thread(int L) {
 // same LDS buffer (every thread has read its last-stage operands by then).
 template <int L, int B, int NT, int SIGN, int BS, int ES, bool BFAST, bool IN_LDS, int Ns, bool SYNC_ST = false,
           bool PRE = false, class LD, class ST>
-__device__ __forceinline__ void fft_stages(float2 *lds, const float2 *__restrict__ tw, int twstride, int tid,
+__device__ __forceinline__ void fft_stages(float2 *lds, const float2 *tw, int twstride, int tid,
                                            const LD &ld, const ST &st, const float2 *pre = nullptr) {
   constexpr int E = L * B / NT;
   constexpr int R = pick_radix(L / Ns, E);
@@ -261,6 +261,61 @@ __device__ __forceinline__ void xcd_tile(int &bx, int &by) {
 // ---------------------------------------------------------------- strided column pass
 constexpr int col_ept(int L, int T) { return elems_per_thread(L); }
 constexpr int col_threads(int L, int T) { return L * T / col_ept(L, T); }
+
+// Element of a column tile: column c, line index j + o of the tile at base, ls
+// elements between lines.  base + o ls is the same for the whole workgroup (o is
+// a compile-time constant of the stage), so it lives in scalar registers and the
+// lanes hold one byte offset for all of a stage's accesses: 32 bits wide, except
+// where a stage reaches past 4 GiB (the 1536 and 2048 meshes, whose last radix is
+// 3 or 8: j up to L/3 or L/8 lines of L HP elements).
+constexpr int col_last_radix(int L, int T) {
+  int n = 1, e = col_ept(L, T), r = 0;
+  while (n < L) r = pick_radix(L / n, e), n *= r;
+  return r;
+}
+template <int L, int T>
+struct ColOff {
+  static constexpr unsigned long long kReach = (unsigned long long)(L / col_last_radix(L, T)) * L * (L / 2 + 16) * 8;
+  using type = typename std::conditional<(kReach >> 32) == 0, unsigned, size_t>::type;
+};
+// Twiddle table of the column passes: in LDS after the tile, so that the stages'
+// twiddles do not queue behind the tile loads and stores in flight (the vector-memory
+// counter is waited on in order), and every pass needs fewer registers.  Measured with
+// the table in global memory / in LDS: plain x pass 2.20 / 2.02 ms and y pass 1.76 /
+// 1.70 ms at 1024 (16 columns), dual y pass 178 / 155 us and density pair 229 / 188 us
+// at 384.  From 1536 on the table stays in global memory: the tile and the P(k) bins
+// take the LDS.
+constexpr bool tw_in_lds(int L) { return L < 1536; }
+constexpr size_t col_lds_elems(int L, int T) { return (size_t)L * T + (tw_in_lds(L) ? L : 0); }
+// Construct before the tile's loads (so the table's loads are the older ones), then
+// to_lds() after them: the table's LDS writes wait for its own loads only.
+template <int L, int T, int NT>
+struct StageTwiddles {
+  static constexpr int K = tw_in_lds(L) ? (L + NT - 1) / NT : 1;
+  float2 r[K];
+  const float2 *tw;
+  __device__ __forceinline__ StageTwiddles(const float2 *t, int tid) : tw(t) {
+    if constexpr (tw_in_lds(L))
+#pragma unroll
+      for (int i = 0; i < K; ++i) r[i] = tw[tid + i * NT < L ? tid + i * NT : 0];
+  }
+  __device__ __forceinline__ const float2 *to_lds(float2 *lds, int tid) {
+    if constexpr (!tw_in_lds(L)) return tw;
+    float2 *t = lds + (size_t)L * T;
+#pragma unroll
+    for (int i = 0; i < K; ++i)
+      if (tid + i * NT < L) t[tid + i * NT] = r[i];
+    __syncthreads();
+    return t;
+  }
+};
+template <int L, int T, class P>
+__device__ __forceinline__ P &col_at(P *base, size_t ls, int c, int j, int o) {
+  using O = typename ColOff<L, T>::type;
+  using B = typename std::conditional<std::is_const<P>::value, const char, char>::type;
+  B *u = reinterpret_cast<B *>(base + (size_t)o * ls);
+  return *reinterpret_cast<P *>(u + ((O)j * (O)(ls * sizeof(P)) + (O)((unsigned)c * sizeof(P))));
+}
 
 // ---------------------------------------------------------------- contiguous z pass
 // threads per block of the z passes (rows per block = this / (N/2) x elements per thread):

@@ -87,16 +87,15 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_green(const float2 *_
   xcd_tile(bx, ky);
   const int kz0 = bx * T;
   const size_t tile = (size_t)ky * os + kz0;
+  StageTwiddles<L, T, NT> stw(tw, tid);
   float2 p1[E], p2[E];
 #pragma unroll
   for (int q = 0; q < NB0; ++q) {
     const int g = tid + q * NT, c = g % T, j = g / T;
-    const float2 *pa = a + tile + (size_t)j * ls + c;
-    const float2 *pb = b ? b + tile + (size_t)j * ls + c : nullptr;
 #pragma unroll
     for (int r = 0; r < R0; ++r) {
-      float2 v = pa[(size_t)(r * M0) * ls];
-      if (pb) v = cadd(v, pb[(size_t)(r * M0) * ls]);
+      float2 v = col_at<L, T>(a + tile, ls, c, j, r * M0);
+      if (b) v = cadd(v, col_at<L, T>(b + tile, ls, c, j, r * M0));
       p1[q * R0 + r] = v;
     }
   }
@@ -113,12 +112,13 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_green(const float2 *_
     }
   }
   auto ld = [&](int, int, int) { return make_float2(0.f, 0.f); };
-  auto st0 = [&](int c, int j, int o, float2 v) { out0[tile + (size_t)j * ls + c + (size_t)o * ls] = v; };
-  fft_stages<L, T, NT, +1, 1, T, true, false, 1, false, true>(lds, tw, 1, tid, ld, st0, p1);
+  auto st0 = [&](int c, int j, int o, float2 v) { col_at<L, T>(out0 + tile, ls, c, j, o) = v; };
+  const float2 *twl = stw.to_lds(lds, tid);
+  fft_stages<L, T, NT, +1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ld, st0, p1);
   if (MODE == GREEN_FORCE) {
     __syncthreads();
-    auto st1 = [&](int c, int j, int o, float2 v) { out1[tile + (size_t)j * ls + c + (size_t)o * ls] = v; };
-    fft_stages<L, T, NT, +1, 1, T, true, false, 1, false, true>(lds, tw, 1, tid, ld, st1, p2);
+    auto st1 = [&](int c, int j, int o, float2 v) { col_at<L, T>(out1 + tile, ls, c, j, o) = v; };
+    fft_stages<L, T, NT, +1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ld, st1, p2);
   }
 }
 
@@ -136,24 +136,25 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_dual(float2 *buf, flo
   int bx, by;
   xcd_tile(bx, by);
   const size_t tile = (size_t)by * os + (size_t)bx * T;
+  StageTwiddles<L, T, NT> stw(tw, tid);
   float2 p1[E], p2[E];
 #pragma unroll
   for (int q = 0; q < NB0; ++q) {
     const int g = tid + q * NT, c = g % T, j = g / T;
-    const float2 *pa = buf + tile + (size_t)j * ls + c;
 #pragma unroll
     for (int r = 0; r < R0; ++r) {
-      const float2 v = pa[(size_t)(r * M0) * ls];
+      const float2 v = col_at<L, T>((const float2 *)buf + tile, ls, c, j, r * M0);
       p2[q * R0 + r] = v;
       p1[q * R0 + r] = cscale(mul_i<+1>(v), (float)nsgn(j + r * M0, L));
     }
   }
   auto ld = [&](int, int, int) { return make_float2(0.f, 0.f); };
-  auto st0 = [&](int c, int j, int o, float2 v) { oy[tile + (size_t)j * ls + c + (size_t)o * ls] = v; };
-  fft_stages<L, T, NT, +1, 1, T, true, false, 1, false, true>(lds, tw, 1, tid, ld, st0, p1);
+  auto st0 = [&](int c, int j, int o, float2 v) { col_at<L, T>(oy + tile, ls, c, j, o) = v; };
+  const float2 *twl = stw.to_lds(lds, tid);
+  fft_stages<L, T, NT, +1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ld, st0, p1);
   __syncthreads();
-  auto st1 = [&](int c, int j, int o, float2 v) { buf[tile + (size_t)j * ls + c + (size_t)o * ls] = v; };
-  fft_stages<L, T, NT, +1, 1, T, true, false, 1, false, true>(lds, tw, 1, tid, ld, st1, p2);
+  auto st1 = [&](int c, int j, int o, float2 v) { col_at<L, T>(buf + tile, ls, c, j, o) = v; };
+  fft_stages<L, T, NT, +1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ld, st1, p2);
 }
 
 // x pass, forward, then phi = coupling n^2/(n^2 + m2) X (0 at n = 0): EffDensitykToPhiofk
@@ -171,14 +172,18 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_epi(float2 *buf, size
   const int kz0 = bx * T;
   const size_t tile = (size_t)ky * os + kz0;
   const int ny = nsgn(ky, N);
-  auto ld = [&](int c, int j, int o) { return buf[tile + (size_t)j * ls + c + (size_t)o * ls]; };
+  auto ld = [&](int c, int j, int o) { return col_at<L, T>((const float2 *)buf + tile, ls, c, j, o); };
   auto st = [&](int c, int j, int o, float2 v) {
     const int kz = kz0 + c, nx = nsgn(j + o, N);
     const int n2 = nx * nx + ny * ny + kz * kz;
     const float f = (kz <= N / 2 && n2 > 0) ? coupling * ((float)n2 / ((float)n2 + m2)) : 0.f;
-    buf[tile + (size_t)j * ls + c + (size_t)o * ls] = cscale(v, f);
+    col_at<L, T>(buf + tile, ls, c, j, o) = cscale(v, f);
   };
-  fft_stages<L, T, NT, -1, 1, T, true, false, 1>(lds, tw, 1, tid, ld, st);
+  StageTwiddles<L, T, NT> stw(tw, tid);
+  float2 pre[col_ept(L, T)];
+  first_loads<L, T, NT, true>(pre, tid, ld);
+  const float2 *twl = stw.to_lds(lds, tid);
+  fft_stages<L, T, NT, -1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ld, st, pre);
 }
 
 // x pass, forward, accumulating compute_power_spectrum's binned power
@@ -195,7 +200,7 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_pofk(float2 *buf, siz
   extern __shared__ float2 lds[];
   constexpr int NT = col_threads(L, T);
   constexpr int N = L;
-  double *bins = (double *)(lds + (size_t)L * T);
+  double *bins = (double *)(lds + col_lds_elems(L, T));
   float *wv = (float *)(bins + nbins);
   const int tid = threadIdx.x;
   for (int b = tid; b < nbins; b += NT) bins[b] = 0.0;
@@ -206,9 +211,9 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_pofk(float2 *buf, siz
   const int kz0 = bx * T;
   const size_t tile = (size_t)ky * os + kz0;
   const int d1 = ky > N / 2 ? N - ky : ky;
-  auto ld = [&](int c, int j, int o) { return buf[tile + (size_t)j * ls + c + (size_t)o * ls]; };
+  auto ld = [&](int c, int j, int o) { return col_at<L, T>((const float2 *)buf + tile, ls, c, j, o); };
   auto st = [&](int c, int j, int o, float2 v) {
-    buf[tile + (size_t)j * ls + c + (size_t)o * ls] = v;
+    col_at<L, T>(buf + tile, ls, c, j, o) = v;
     const int kz = kz0 + c, kx = j + o;
     if (kz > N / 2) return;
     const int d0 = kx > N / 2 ? N - kx : kx;
@@ -218,7 +223,11 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_pofk(float2 *buf, siz
     const float w = (kz == 0 || kz == N / 2) ? 1.f : 2.f;
     atomicAdd(&bins[nk], (double)((v.x * v.x + v.y * v.y) * (w * wv[d0] * wv[d1] * wv[kz])));
   };
-  fft_stages<L, T, NT, -1, 1, T, true, false, 1>(lds, tw, 1, tid, ld, st);
+  StageTwiddles<L, T, NT> stw(tw, tid);
+  float2 pre[col_ept(L, T)];
+  first_loads<L, T, NT, true>(pre, tid, ld);
+  const float2 *twl = stw.to_lds(lds, tid);
+  fft_stages<L, T, NT, -1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ld, st, pre);
   __syncthreads();
   for (int b = tid; b < nbins; b += NT)
     if (bins[b] != 0.0) atomicAdd(&pk[b], bins[b]);
@@ -238,9 +247,15 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_pofk(float2 *buf, siz
 // k_col_green.  The forward's last stage stores its outputs into LDS in the
 // tile layout (after a barrier), from where each thread takes its first-stage
 // operands of the inverse.
+// What bounds it: with one workgroup per CU its load, transform and store phases add
+// up.  At most 128 VGPRs (four waves per SIMD, two 512-thread workgroups per CU at
+// 1024) let one tile's loads and stores run under another's transforms; the stage
+// twiddles in LDS free the registers and the vector-memory queue for that.  Force
+// pair 6.45 -> 4.68 ms at 1024 (2.8 -> 3.8 TB/s), 316 -> 254 us at 384; density pair
+// with the Green's force (LCDM) 7.2 -> 5.2 ms at 1024, 340 -> 293 us at 384.
 enum { FWD_DENSITY = 0, FWD_EPI = 1, FWD_PLAIN = 2 };
 template <int L, int T, int FWD, int MODE>
-__global__ __launch_bounds__(col_threads(L, T)) void k_col_fused(
+__global__ __launch_bounds__(col_threads(L, T), tw_in_lds(L) ? 4 : 1) void k_col_fused(
     const float2 *in, float2 *kout, const float2 *__restrict__ dk, float2 *out0, float2 *out1, size_t ls, size_t os,
     const float2 *__restrict__ tw, GreenArgs ga, float coupling, float m2, const float *__restrict__ winv,
     const int16_t *__restrict__ pbin, int nbins, double *__restrict__ pk, size_t zs) {
@@ -261,7 +276,7 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_fused(
   const size_t tile = (size_t)ky * os + kz0;
   const int ny = nsgn(ky, N), d1 = ky > N / 2 ? N - ky : ky;
   const bool bin = FWD == FWD_DENSITY && pk != nullptr;
-  double *bins = (double *)(lds + (size_t)L * T);
+  double *bins = (double *)(lds + col_lds_elems(L, T));
   float *wv = (float *)(bins + nbins);
   if (bin) {
     for (int b = tid; b < nbins; b += NT) bins[b] = 0.0;
@@ -269,11 +284,11 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_fused(
     __syncthreads();
   }
   // forward transform; its outputs (row kx of column c) go to lds[c + kx T]
-  auto ld = [&](int c, int j, int o) { return in[tile + (size_t)j * ls + c + (size_t)o * ls]; };
+  auto ld = [&](int c, int j, int o) { return col_at<L, T>(in + tile, ls, c, j, o); };
   auto st = [&](int c, int j, int o, float2 v) {
     const int kx = j + o, kz = kz0 + c;
     if (FWD == FWD_DENSITY) {
-      if (kout) kout[tile + (size_t)kx * ls + c] = v;
+      if (kout) col_at<L, T>(kout + tile, ls, c, j, o) = v;
       if (bin && kz <= N / 2) {
         const int d0 = kx > N / 2 ? N - kx : kx;
         const int nk = pbin[d0 * d0 + d1 * d1 + kz * kz];
@@ -290,19 +305,20 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_fused(
     }
     lds[c + kx * T] = v;
   };
-  fft_stages<L, T, NT, -1, 1, T, true, false, 1, true>(lds, tw, 1, tid, ld, st);
-  // delta(k) to add, in the inverse's first-stage layout (requested after the
-  // forward's loads: the vector-memory counter is waited on in order, so loads
-  // issued earlier would delay the forward's first stage)
+  StageTwiddles<L, T, NT> stw(tw, tid);
   float2 p1[E], p2[E];
-  if (FWD != FWD_DENSITY) {
-#pragma unroll
-    for (int q = 0; q < NB0; ++q) {
-      const int g = tid + q * NT, c = g % T, j = g / T;
-#pragma unroll
-      for (int r = 0; r < R0; ++r) p2[q * R0 + r] = dk[tile + (size_t)(j + r * M0) * ls + c];
-    }
-  }
+  first_loads<L, T, NT, true>(p1, tid, ld);
+  // delta(k) to add, in the inverse's first-stage layout.  With 12 elements per thread
+  // it is requested behind the forward's loads and arrives while the forward
+  // transform runs (384: 254 against 262 us for the pair); with 16 the registers it
+  // would hold spill, so it is requested after the forward transform (1024: 4.68
+  // against 4.85 ms).
+  constexpr bool kDkEarly = E <= 12;
+  auto ldk = [&](int c, int j, int o) { return col_at<L, T>(dk + tile, ls, c, j, o); };
+  if constexpr (FWD != FWD_DENSITY && kDkEarly) first_loads<L, T, NT, true>(p2, tid, ldk);
+  const float2 *twl = stw.to_lds(lds, tid);
+  fft_stages<L, T, NT, -1, 1, T, true, false, 1, true, true>(lds, twl, 1, tid, ld, st, p1);
+  if constexpr (FWD != FWD_DENSITY && !kDkEarly) first_loads<L, T, NT, true>(p2, tid, ldk);
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < NB0; ++q) {
@@ -326,12 +342,12 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_fused(
     }
   }
   auto ldz = [&](int, int, int) { return make_float2(0.f, 0.f); };
-  auto st0 = [&](int c, int j, int o, float2 v) { out0[tile + (size_t)j * ls + c + (size_t)o * ls] = v; };
-  fft_stages<L, T, NT, +1, 1, T, true, false, 1, false, true>(lds, tw, 1, tid, ldz, st0, p1);
+  auto st0 = [&](int c, int j, int o, float2 v) { col_at<L, T>(out0 + tile, ls, c, j, o) = v; };
+  fft_stages<L, T, NT, +1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ldz, st0, p1);
   if (MODE == GREEN_FORCE) {
     __syncthreads();
-    auto st1 = [&](int c, int j, int o, float2 v) { out1[tile + (size_t)j * ls + c + (size_t)o * ls] = v; };
-    fft_stages<L, T, NT, +1, 1, T, true, false, 1, false, true>(lds, tw, 1, tid, ldz, st1, p2);
+    auto st1 = [&](int c, int j, int o, float2 v) { col_at<L, T>(out1 + tile, ls, c, j, o) = v; };
+    fft_stages<L, T, NT, +1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ldz, st1, p2);
   }
   if (bin) {
     __syncthreads();
@@ -409,7 +425,7 @@ int set_lds(mgpu_ctx *ctx, K kern, size_t lds) {
 template <int N, int T>
 int green_launch(mgpu_ctx *ctx, int mode, const float2 *a, const float2 *b, float2 *o0, float2 *o1, GreenArgs ga) {
   const size_t HP = ctx->fft.hp, ls = (size_t)N * HP, os = HP;
-  const size_t lds = (size_t)N * T * sizeof(float2);
+  const size_t lds = col_lds_elems(N, T) * sizeof(float2);
   dim3 grid(HP / T, N), block(col_threads(N, T));
   int rc;
   if (mode == GREEN_FORCE) {
@@ -444,7 +460,7 @@ template <int N, int T, int FWD, int MODE>
 int fused_x_launch_k(mgpu_ctx *ctx, const FusedXArgs &a) {
   const size_t HP = ctx->fft.hp, ls = (size_t)N * HP, os = HP;
   const int nbins = a.pk ? ctx->p.pofk_nbins : 0;
-  const size_t lds = (size_t)N * T * sizeof(float2) + (a.pk ? sizeof(double) * nbins + sizeof(float) * (N / 2 + 1) : 0);
+  const size_t lds = col_lds_elems(N, T) * sizeof(float2) + (a.pk ? sizeof(double) * nbins + sizeof(float) * (N / 2 + 1) : 0);
   if (lds > ctx->lds_max) return mgpu_fail(ctx, MGPU_E_INVALID, "P(k) bins do not fit the LDS of the x pass");
   if (a.pk && !ctx->pk_bin) return mgpu_fail(ctx, MGPU_E_INVALID, "no P(k) bin table");
   int rc;
@@ -473,7 +489,7 @@ int fused_x_launch(mgpu_ctx *ctx, const FusedXArgs &a) {
 template <int N, int T>
 int dual_launch(mgpu_ctx *ctx, float2 *buf, float2 *oy) {
   const size_t HP = ctx->fft.hp, ls = HP, os = (size_t)N * HP;
-  const size_t lds = (size_t)N * T * sizeof(float2);
+  const size_t lds = col_lds_elems(N, T) * sizeof(float2);
   int rc;
   if ((rc = set_lds(ctx, k_col_dual<N, T>, lds))) return rc;
   hipLaunchKernelGGL((k_col_dual<N, T>), dim3(HP / T, N, ctx->bz), dim3(col_threads(N, T)), lds, ctx->stream, buf, oy,
@@ -485,7 +501,7 @@ int dual_launch(mgpu_ctx *ctx, float2 *buf, float2 *oy) {
 template <int N, int T>
 int epi_launch(mgpu_ctx *ctx, float2 *buf, float coupling, float m2) {
   const size_t HP = ctx->fft.hp, ls = (size_t)N * HP, os = HP;
-  const size_t lds = (size_t)N * T * sizeof(float2);
+  const size_t lds = col_lds_elems(N, T) * sizeof(float2);
   int rc;
   if ((rc = set_lds(ctx, k_col_epi<N, T>, lds))) return rc;
   hipLaunchKernelGGL((k_col_epi<N, T>), dim3(HP / T, N), dim3(col_threads(N, T)), lds, ctx->stream, buf, ls, os,
@@ -498,7 +514,7 @@ template <int N, int T>
 int pofk_launch(mgpu_ctx *ctx, float2 *buf, double *pk) {
   const size_t HP = ctx->fft.hp, ls = (size_t)N * HP, os = HP;
   const int nbins = ctx->p.pofk_nbins;
-  const size_t lds = (size_t)N * T * sizeof(float2) + sizeof(double) * nbins + sizeof(float) * (N / 2 + 1);
+  const size_t lds = col_lds_elems(N, T) * sizeof(float2) + sizeof(double) * nbins + sizeof(float) * (N / 2 + 1);
   if (lds > ctx->lds_max) return mgpu_fail(ctx, MGPU_E_INVALID, "P(k) bins do not fit the LDS of the x pass");
   if (!ctx->pk_bin) return mgpu_fail(ctx, MGPU_E_INVALID, "no P(k) bin table");
   int rc;

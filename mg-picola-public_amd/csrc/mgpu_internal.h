@@ -207,6 +207,8 @@ struct PhaseTimer {
 int fft_plan_init(mgpu_ctx *ctx, FFTPlan *plan, int n, int tcols = 16);
 void fft_plan_free(FFTPlan *plan);
 bool fft_tile16_fits(const mgpu_ctx *ctx, int n);
+// LDS bytes of a column pass of T columns (the tile, and the stage twiddles where they are held there)
+size_t fft_col_lds(int n, int T);
 int fft_autotune(mgpu_ctx *ctx, FFTPlan *plan, float2 *buf, double ms[2]);
 bool fft_size_supported(int n);
 // in-place 3D transforms on a slot with the padded layout above

@@ -476,7 +476,7 @@ int pm_pofk(mgpu_ctx *ctx, const float2 *dk, mgpu_pofk *out) {
 
 // The x pass that bins P(k) holds its tile of T columns and the bins in LDS.
 static bool pofk_fused_fits(const mgpu_ctx *ctx, int T) {
-  const size_t need = (size_t)ctx->N * T * sizeof(float2) + sizeof(double) * (size_t)ctx->p.pofk_nbins +
+  const size_t need = fft_col_lds(ctx->N, T) + sizeof(double) * (size_t)ctx->p.pofk_nbins +
                       sizeof(float) * (size_t)(ctx->N / 2 + 1);
   return need <= ctx->lds_max;
 }
