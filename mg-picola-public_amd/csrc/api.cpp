@@ -178,7 +178,7 @@ static void memory_plan(const mgpu_params *p, size_t part[MGPU_MEM_PARTS]) {
   }
   const size_t nb = (size_t)std::max(1, p->pofk_nbins);
   part[MGPU_MEM_TABLES] = (3 * std::max<size_t>((np + 255) / 256, N) + 3 * 1024) * sizeof(double) +
-                          4 * nb * sizeof(double) + (N / 2 + 1) * 12 + 2 * N * sizeof(float2) +
+                          MGPU_PK_SETS * nb * sizeof(double) + (nb + 1) * sizeof(int) + (N / 2 + 1) * 12 + 2 * N * sizeof(float2) +
                           mgpu_n2_table_len((int)N) * (2 * sizeof(double) + 2 * sizeof(float) + sizeof(int16_t));
   part[MGPU_MEM_RSD] = np * sizeof(float4);
 }
@@ -293,7 +293,7 @@ int create_ctx(const mgpu_params *p, mgpu_ctx **out, mgpu_arena *arena, char *sh
   if ((rc = alloc(ctx, (void **)&ctx->partial, ctx->partial_len * sizeof(double), "reduction scratch"))) return fail(rc);
   if ((rc = alloc(ctx, (void **)&ctx->dsum, 8 * sizeof(double), "sums"))) return fail(rc);
   const int nb = std::max(1, p->pofk_nbins);
-  if ((rc = alloc(ctx, (void **)&ctx->pk, 4 * (size_t)nb * sizeof(double), "P(k) bins"))) return fail(rc);
+  if ((rc = alloc(ctx, (void **)&ctx->pk, MGPU_PK_SETS * (size_t)nb * sizeof(double), "P(k) bins"))) return fail(rc);
   {
     // compute_power_spectrum's CIC deconvolution 1/(W_x W_y W_z)^4 with the 1/N^6 of the
     // transform split over the three axes (src/compute_pofk.c:128-134)
@@ -327,6 +327,36 @@ int create_ctx(const mgpu_params *p, mgpu_ctx **out, mgpu_arena *arena, char *sh
     if ((rc = alloc(ctx, (void **)&ctx->pk_bin, tab.size() * sizeof(int16_t), "P(k) bin table"))) return fail(rc);
     if (hipMemcpy(ctx->pk_bin, tab.data(), tab.size() * sizeof(int16_t), hipMemcpyHostToDevice) != hipSuccess)
       return fail(mgpu_fail(ctx, MGPU_E_HIP, "bin table upload failed"));
+    // the bins by their first |n|^2: below the first bin and past the last one the table
+    // holds -1 (bins of unusual kmin, kmax that do not rise with |n|^2 keep the table)
+    const int nbk = p->pofk_nbins;
+    std::vector<int> edge((size_t)nbk + 1, (int)ctx->n2len);
+    size_t lo = 0, hi = ctx->n2len;
+    while (lo < hi && tab[lo] < 0) lo++;
+    while (hi > lo && tab[hi - 1] < 0) hi--;
+    bool rises = lo < hi;
+    for (size_t n2 = lo, b = 0; n2 < hi && rises; n2++) {
+      rises = tab[n2] >= 0 && (n2 == lo || tab[n2] >= tab[n2 - 1]);
+      for (; rises && b <= (size_t)tab[n2]; b++) edge[b] = (int)n2;
+    }
+    if (rises) {
+      // bins past the last occupied one start where the table ends
+      for (size_t b = (size_t)tab[hi - 1] + 1; b <= (size_t)nbk; b++) edge[b] = (int)hi;
+      int *dev = nullptr;
+      if ((rc = alloc(ctx, (void **)&dev, edge.size() * sizeof(int), "P(k) bin edges"))) return fail(rc);
+      ctx->pk_fn.edge = dev;
+      if (hipMemcpy(dev, edge.data(), edge.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess)
+        return fail(mgpu_fail(ctx, MGPU_E_HIP, "bin edge upload failed"));
+      ctx->pk_fn.nbins = nbk;
+      ctx->pk_fn.logbins = p->pofk_bintype == 1;
+      if (p->pofk_bintype == 1) {
+        ctx->pk_fn.a = (float)(0.5 * std::log(2.0) * nbk / lnrange);
+        ctx->pk_fn.b = (float)(0.5 - std::log(kmin) / lnrange * nbk);
+      } else {
+        ctx->pk_fn.a = (float)(nbk / (kmax - kmin));
+        ctx->pk_fn.b = (float)(0.5 - kmin / (kmax - kmin) * nbk);
+      }
+    }
   }
   for (int s = 0; s < 2; s++) {
     if ((rc = alloc(ctx, (void **)&ctx->n2tab[s], ctx->n2len * sizeof(double), "n2 table"))) return fail(rc);
@@ -370,7 +400,7 @@ void mgpu_destroy(mgpu_ctx *ctx) {
                   ctx->cdelta[1], ctx->partial,  ctx->dsum,      ctx->pk,        ctx->n2tab[0],
                   ctx->n2tab[1], ctx->n2tabf[0], ctx->n2tabf[1], ctx->lattice_slot, ctx->slice_buf,
                   ctx->dep_scratch, ctx->winv,    ctx->winvf,     ctx->pk_bin,    ctx->rsd_crd,
-                  ctx->nu_slice, ctx->nu_fac,  ctx->feat_part, ctx->feat,     ctx->green_mult};
+                  ctx->nu_slice, ctx->nu_fac,  ctx->feat_part, ctx->feat,     ctx->green_mult, (void *)ctx->pk_fn.edge};
   for (void *q : ptrs)
     if (q && !((const char *)q >= a0 && (const char *)q < a1)) (void)hipFree(q);
   if (ctx->slice_host) (void)hipHostFree(ctx->slice_host);

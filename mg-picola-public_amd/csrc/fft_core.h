@@ -120,13 +120,70 @@ struct Bfly<16, SIGN> {
   }
 };
 
+// 12 points as 4 x 3: n = n1 + 4 n2, k = k2 + 3 k1;
+// A[n1][k2] = DFT3_n2(v[n1 + 4 n2]) * W12^(n1 k2), X[k2 + 3 k1] = DFT4_n1(A[n1][k2]).
+template <int SIGN>
+struct Bfly<12, SIGN> {
+  __device__ __forceinline__ static void run(float2 *v) {
+    const float h = 0.5f, s3 = 0.86602540378443864676f, sg = (float)SIGN;
+    float2 a[4][3];
+#pragma unroll
+    for (int n1 = 0; n1 < 4; ++n1) {
+      a[n1][0] = v[n1];
+      a[n1][1] = v[n1 + 4];
+      a[n1][2] = v[n1 + 8];
+      Bfly<3, SIGN>::run(a[n1]);
+    }
+    // twiddles W12^(n1 k2) = exp(SIGN 2 pi i n1 k2 / 12)
+    const float2 w1 = make_float2(s3, sg * h), w2 = make_float2(h, sg * s3), w4 = make_float2(-h, sg * s3);
+    a[1][1] = cmul(a[1][1], w1);
+    a[1][2] = cmul(a[1][2], w2);
+    a[2][1] = cmul(a[2][1], w2);
+    a[2][2] = cmul(a[2][2], w4);
+    a[3][1] = mul_i<SIGN>(a[3][1]);
+    a[3][2] = make_float2(-a[3][2].x, -a[3][2].y);
+#pragma unroll
+    for (int k2 = 0; k2 < 3; ++k2) {
+      float2 b[4] = {a[0][k2], a[1][k2], a[2][k2], a[3][k2]};
+      Bfly<4, SIGN>::run(b);
+      v[k2] = b[0];
+      v[k2 + 3] = b[1];
+      v[k2 + 6] = b[2];
+      v[k2 + 9] = b[3];
+    }
+  }
+};
+
+// largest radix first; 12 elements per thread start with a radix 12, so that 192, 384
+// and 768 points take 3, 4 and 4 stages (12 4 4, 12 4 4 2, 12 4 4 4) instead of the
+// 4, 5 and 5 of radices 4, 2 and 3
 constexpr int pick_radix(int rem, int e) {
-  return (rem % 16 == 0 && e % 16 == 0)  ? 16
-         : (rem % 8 == 0 && e % 8 == 0)  ? 8
-         : (rem % 4 == 0 && e % 4 == 0)  ? 4
-         : (rem % 2 == 0 && e % 2 == 0)  ? 2
-         : (rem % 3 == 0 && e % 3 == 0)  ? 3
-                                         : 0;
+  return (rem % 12 == 0 && e == 12)      ? 12
+         : (rem % 16 == 0 && e % 16 == 0) ? 16
+         : (rem % 8 == 0 && e % 8 == 0)   ? 8
+         : (rem % 4 == 0 && e % 4 == 0)   ? 4
+         : (rem % 2 == 0 && e % 2 == 0)   ? 2
+         : (rem % 3 == 0 && e % 3 == 0)   ? 3
+                                          : 0;
+}
+// The last stage's radix, and the radix of the stage at sub-length Ns: in the order of
+// pick_radix, or (rev) in the opposite order.  Two transforms that follow each other
+// with only a multiplier between run the second one reversed: its first radix is then
+// the first one's last, so each thread already holds its operands in registers.
+constexpr int last_radix(int L, int E) {
+  int n = 1, r = 0;
+  while (n < L) r = pick_radix(L / n, E), n *= r;
+  return r;
+}
+constexpr int stage_radix(int L, int E, int Ns, bool rev) {
+  if (!rev) return pick_radix(L / Ns, E);
+  int list[16] = {}, k = 0;
+  for (int n = 1; n < L; n *= list[k++]) list[k] = pick_radix(L / n, E);
+  for (int n = 1; k > 0; n *= list[k]) {
+    --k;
+    if (n == Ns) return list[k];
+  }
+  return 0;
 }
 // elements held per thread for a length-L transform
 // (radix-3 lengths: 12 up to 768, so the z passes and the fused column passes of
@@ -149,16 +206,25 @@ constexpr int elems_per_thread(int L) {
 // through a pointer at run time (which would place it in scratch memory).
 // With SYNC_ST a barrier precedes the last stage's stores, so st may write the
 // same LDS buffer (every thread has read its last-stage operands by then).
+// REV: the stages' radices in the opposite order (see stage_radix).
+// hook() is called once, before the last stage reads its operands, when the data are
+// in LDS and few registers are live: the place to issue loads that the caller needs
+// right after the transform.
+struct NoHook {
+  __device__ __forceinline__ void operator()() const {}
+};
 template <int L, int B, int NT, int SIGN, int BS, int ES, bool BFAST, bool IN_LDS, int Ns, bool SYNC_ST = false,
-          bool PRE = false, class LD, class ST>
+          bool PRE = false, bool REV = false, class LD, class ST, class HOOK = NoHook>
 __device__ __forceinline__ void fft_stages(float2 *lds, const float2 *tw, int twstride, int tid,
-                                           const LD &ld, const ST &st, const float2 *pre = nullptr) {
+                                           const LD &ld, const ST &st, const float2 *pre = nullptr,
+                                           const HOOK &hook = HOOK()) {
   constexpr int E = L * B / NT;
-  constexpr int R = pick_radix(L / Ns, E);
+  constexpr int R = stage_radix(L, E, Ns, REV);
   static_assert(R > 0, "size not factorable with the per-thread element count");
   constexpr int NB = E / R;
   constexpr int M = L / R;
   constexpr bool FIRST = (Ns == 1), LAST = (Ns * R == L);
+  if constexpr (FIRST && LAST) hook();
   float2 v[NB][R];
 #pragma unroll
   for (int q = 0; q < NB; ++q) {
@@ -166,10 +232,10 @@ __device__ __forceinline__ void fft_stages(float2 *lds, const float2 *tw, int tw
     int b, j;
     if constexpr (BFAST) { b = g % B; j = g / B; } else { j = g % M; b = g / M; }
     const int k = j % Ns;
-    // twiddles W^(r k) of this stage: for radix 8 and 16, r = r1 + 4 r2 and
+    // twiddles W^(r k) of this stage: for radix 8, 12 and 16, r = r1 + 4 r2 and
     // W^(r k) = W^(r1 k) W^(4 r2 k), so only W^(k), W^(2k), W^(3k) and the
     // W^(4 r2 k) are loaded (one extra rounding for the products)
-    constexpr int R2 = (R == 16 || R == 8) ? R / 4 : 1;
+    constexpr int R2 = (R == 16 || R == 12 || R == 8) ? R / 4 : 1;
     constexpr int R1 = R / R2;
     float2 wa[R1], wb[R2];
     if constexpr (!FIRST) {
@@ -226,16 +292,19 @@ __device__ __forceinline__ void fft_stages(float2 *lds, const float2 *tw, int tw
 #pragma unroll
       for (int r = 0; r < R; ++r) lds[b * BS + (d + r * Ns) * ES] = v[q][r];
     }
+    if constexpr (Ns * R * stage_radix(L, E, Ns * R, REV) == L) hook();
     __syncthreads();
-    fft_stages<L, B, NT, SIGN, BS, ES, BFAST, false, Ns * R, SYNC_ST>(lds, tw, twstride, tid, ld, st);
+    fft_stages<L, B, NT, SIGN, BS, ES, BFAST, false, Ns * R, SYNC_ST, false, REV>(lds, tw, twstride, tid, ld, st,
+                                                                                  nullptr, hook);
   }
 }
 
-// The first stage's operand loads of fft_stages, into registers.
-template <int L, int B, int NT, bool BFAST, class LD>
+// The first stage's operand loads of fft_stages (of the reversed order with REV: the
+// layout of the last stage's outputs), into registers.
+template <int L, int B, int NT, bool BFAST, bool REV = false, class LD>
 __device__ __forceinline__ void first_loads(float2 *pre, int tid, const LD &ld) {
   constexpr int E = L * B / NT;
-  constexpr int R = pick_radix(L, E);
+  constexpr int R = stage_radix(L, E, 1, REV);
   constexpr int NB = E / R;
   constexpr int M = L / R;
 #pragma unroll
@@ -268,11 +337,7 @@ constexpr int col_threads(int L, int T) { return L * T / col_ept(L, T); }
 // lanes hold one byte offset for all of a stage's accesses: 32 bits wide, except
 // where a stage reaches past 4 GiB (the 1536 and 2048 meshes, whose last radix is
 // 3 or 8: j up to L/3 or L/8 lines of L HP elements).
-constexpr int col_last_radix(int L, int T) {
-  int n = 1, e = col_ept(L, T), r = 0;
-  while (n < L) r = pick_radix(L / n, e), n *= r;
-  return r;
-}
+constexpr int col_last_radix(int L, int T) { return last_radix(L, col_ept(L, T)); }
 template <int L, int T>
 struct ColOff {
   static constexpr unsigned long long kReach = (unsigned long long)(L / col_last_radix(L, T)) * L * (L / 2 + 16) * 8;

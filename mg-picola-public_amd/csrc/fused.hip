@@ -186,6 +186,49 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_epi(float2 *buf, size
   fft_stages<L, T, NT, -1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ld, st, pre);
 }
 
+// P(k) sums of an x pass in LDS: copies sets of bin sums (lanes take them in turn, so
+// fewer lanes of a wave add to one address: most of a wave's modes share a few bins),
+// the per-axis window and the bin edges.
+template <int L, int NT>
+struct PofkLds {
+  double *bins;
+  float *wv;
+  int *edge;
+  int e0, e1;
+  __device__ __forceinline__ void init(void *lds, const PkBinFn &f, int copies, const float *__restrict__ winv,
+                                       int tid) {
+    bins = (double *)lds;
+    wv = (float *)(bins + copies * f.nbins);
+    edge = (int *)(wv + L / 2 + 1);
+    for (int b = tid; b < copies * f.nbins; b += NT) bins[b] = 0.0;
+    for (int d = tid; d <= L / 2; d += NT) wv[d] = winv[d];
+    for (int b = tid; b <= f.nbins; b += NT) edge[b] = f.edge[b];
+    e0 = f.edge[0];
+    e1 = f.edge[f.nbins];
+    __syncthreads();
+  }
+  // mode (kx, d1 = |ky|, kz) of power |v|^2: weight 1 (kz = 0, N/2) or 2, CIC deconvolution
+  __device__ __forceinline__ void add(float2 v, int kx, int d1, int kz, const PkBinFn &f, int copies, int tid) const {
+    if (kz > L / 2) return;
+    const int d0 = kx > L / 2 ? L - kx : kx;
+    const int nk = pk_bin_of(d0 * d0 + d1 * d1 + kz * kz, f, edge, e0, e1);
+    if (nk < 0) return;
+    const float w = (kz == 0 || kz == L / 2) ? 1.f : 2.f;
+    atomicAdd(&bins[nk + f.nbins * (tid & (copies - 1))],
+              (double)((v.x * v.x + v.y * v.y) * (w * wv[d0] * wv[d1] * wv[kz])));
+  }
+  // into the workgroup's set of MGPU_PK_SETS global sums (adds to one address are
+  // serialised: with one set the 1344 workgroups of a 192 mesh cost 18 us)
+  __device__ __forceinline__ void flush(double *__restrict__ pk, const PkBinFn &f, int copies, int tid) const {
+    pk += ((blockIdx.x + blockIdx.y * gridDim.x) % MGPU_PK_SETS) * f.nbins;
+    for (int b = tid; b < f.nbins; b += NT) {
+      double s = bins[b];
+      for (int c = 1; c < copies; ++c) s += bins[b + c * f.nbins];
+      if (s != 0.0) atomicAdd(&pk[b], s);
+    }
+  }
+};
+
 // x pass, forward, accumulating compute_power_spectrum's binned power
 // (src/compute_pofk.c:71-236) from the transform's output as it is stored:
 // weight 1 (kz = 0, N/2) or 2, CIC deconvolution winv[d0] winv[d1] winv[d2]
@@ -194,18 +237,14 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_epi(float2 *buf, size
 template <int L, int T>
 __global__ __launch_bounds__(col_threads(L, T)) void k_col_pofk(float2 *buf, size_t ls, size_t os,
                                                                   const float2 *__restrict__ tw,
-                                                                  const float *__restrict__ winv,
-                                                                  const int16_t *__restrict__ pbin, int nbins,
-                                                                  double *__restrict__ pk) {
+                                                                  const float *__restrict__ winv, PkBinFn fn,
+                                                                  int copies, double *__restrict__ pk) {
   extern __shared__ float2 lds[];
   constexpr int NT = col_threads(L, T);
   constexpr int N = L;
-  double *bins = (double *)(lds + col_lds_elems(L, T));
-  float *wv = (float *)(bins + nbins);
   const int tid = threadIdx.x;
-  for (int b = tid; b < nbins; b += NT) bins[b] = 0.0;
-  for (int d = tid; d <= N / 2; d += NT) wv[d] = winv[d];
-  __syncthreads();
+  PofkLds<L, NT> pl;
+  pl.init(lds + col_lds_elems(L, T), fn, copies, winv, tid);
   int bx, ky;
   xcd_tile(bx, ky);
   const int kz0 = bx * T;
@@ -214,14 +253,7 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_pofk(float2 *buf, siz
   auto ld = [&](int c, int j, int o) { return col_at<L, T>((const float2 *)buf + tile, ls, c, j, o); };
   auto st = [&](int c, int j, int o, float2 v) {
     col_at<L, T>(buf + tile, ls, c, j, o) = v;
-    const int kz = kz0 + c, kx = j + o;
-    if (kz > N / 2) return;
-    const int d0 = kx > N / 2 ? N - kx : kx;
-    // the bin of |n|^2 comes from the table the host fills with the FP64 formula
-    const int nk = pbin[d0 * d0 + d1 * d1 + kz * kz];
-    if (nk < 0) return;
-    const float w = (kz == 0 || kz == N / 2) ? 1.f : 2.f;
-    atomicAdd(&bins[nk], (double)((v.x * v.x + v.y * v.y) * (w * wv[d0] * wv[d1] * wv[kz])));
+    pl.add(v, j + o, d1, kz0 + c, fn, copies, tid);
   };
   StageTwiddles<L, T, NT> stw(tw, tid);
   float2 pre[col_ept(L, T)];
@@ -229,8 +261,7 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_pofk(float2 *buf, siz
   const float2 *twl = stw.to_lds(lds, tid);
   fft_stages<L, T, NT, -1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ld, st, pre);
   __syncthreads();
-  for (int b = tid; b < nbins; b += NT)
-    if (bins[b] != 0.0) atomicAdd(&pk[b], bins[b]);
+  pl.flush(pk, fn, copies, tid);
 }
 
 // x pass pair: a forward x transform and, from its output in LDS, an inverse
@@ -258,7 +289,7 @@ template <int L, int T, int FWD, int MODE>
 __global__ __launch_bounds__(col_threads(L, T), tw_in_lds(L) ? 4 : 1) void k_col_fused(
     const float2 *in, float2 *kout, const float2 *__restrict__ dk, float2 *out0, float2 *out1, size_t ls, size_t os,
     const float2 *__restrict__ tw, GreenArgs ga, float coupling, float m2, const float *__restrict__ winv,
-    const int16_t *__restrict__ pbin, int nbins, double *__restrict__ pk, size_t zs) {
+    PkBinFn fn, int copies, double *__restrict__ pk, size_t zs) {
   in = zbuf(in, zs);
   kout = zbuf(kout, zs);
   dk = zbuf(dk, zs);
@@ -267,7 +298,11 @@ __global__ __launch_bounds__(col_threads(L, T), tw_in_lds(L) ? 4 : 1) void k_col
   pk = zbuf(pk, zs);
   extern __shared__ float2 lds[];
   constexpr int NT = col_threads(L, T), E = col_ept(L, T);
-  constexpr int R0 = pick_radix(L, E), NB0 = E / R0, M0 = L / R0;
+  // The forward's outputs are handed to the inverse in registers (its stages reversed);
+  // with delta(k) to add at 16 elements per thread those registers spill (1024: 4.94
+  // against 4.69 ms, 256: 96 against 82 us), and the outputs go through LDS instead.
+  constexpr bool kHand = FWD == FWD_DENSITY || E <= 12;
+  constexpr int RX = stage_radix(L, E, 1, kHand), MX = L / RX;  // the inverse's first stage
   constexpr int N = L;
   const int tid = threadIdx.x;
   int bx, ky;
@@ -276,83 +311,63 @@ __global__ __launch_bounds__(col_threads(L, T), tw_in_lds(L) ? 4 : 1) void k_col
   const size_t tile = (size_t)ky * os + kz0;
   const int ny = nsgn(ky, N), d1 = ky > N / 2 ? N - ky : ky;
   const bool bin = FWD == FWD_DENSITY && pk != nullptr;
-  double *bins = (double *)(lds + col_lds_elems(L, T));
-  float *wv = (float *)(bins + nbins);
-  if (bin) {
-    for (int b = tid; b < nbins; b += NT) bins[b] = 0.0;
-    for (int d = tid; d <= N / 2; d += NT) wv[d] = winv[d];
-    __syncthreads();
-  }
-  // forward transform; its outputs (row kx of column c) go to lds[c + kx T]
+  PofkLds<L, NT> pl;
+  if (bin) pl.init(lds + col_lds_elems(L, T), fn, copies, winv, tid);
+  // forward transform; its outputs stay in the registers of the threads that form them
+  float2 p1[E], p2[E];
   auto ld = [&](int c, int j, int o) { return col_at<L, T>(in + tile, ls, c, j, o); };
+  int oi = 0;  // output index of the store (a constant of the unrolled last stage)
   auto st = [&](int c, int j, int o, float2 v) {
     const int kx = j + o, kz = kz0 + c;
     if (FWD == FWD_DENSITY) {
       if (kout) col_at<L, T>(kout + tile, ls, c, j, o) = v;
-      if (bin && kz <= N / 2) {
-        const int d0 = kx > N / 2 ? N - kx : kx;
-        const int nk = pbin[d0 * d0 + d1 * d1 + kz * kz];
-        if (nk >= 0) {
-          const float w = (kz == 0 || kz == N / 2) ? 1.f : 2.f;
-          atomicAdd(&bins[nk], (double)((v.x * v.x + v.y * v.y) * (w * wv[d0] * wv[d1] * wv[kz])));
-        }
-      }
+      if (bin) pl.add(v, kx, d1, kz, fn, copies, tid);
     }
     if (FWD == FWD_EPI) {
       const int nx = nsgn(kx, N), n2 = nx * nx + ny * ny + kz * kz;
       const float f = (kz <= N / 2 && n2 > 0) ? coupling * ((float)n2 / ((float)n2 + m2)) : 0.f;
       v = cscale(v, f);
     }
-    lds[c + kx * T] = v;
+    if constexpr (kHand) p1[oi++] = v;
+    else lds[c + kx * T] = v;
   };
   StageTwiddles<L, T, NT> stw(tw, tid);
-  float2 p1[E], p2[E];
   first_loads<L, T, NT, true>(p1, tid, ld);
-  // delta(k) to add, in the inverse's first-stage layout.  With 12 elements per thread
-  // it is requested behind the forward's loads and arrives while the forward
-  // transform runs (384: 254 against 262 us for the pair); with 16 the registers it
-  // would hold spill, so it is requested after the forward transform (1024: 4.68
-  // against 4.85 ms).
-  constexpr bool kDkEarly = E <= 12;
-  auto ldk = [&](int c, int j, int o) { return col_at<L, T>(dk + tile, ls, c, j, o); };
-  if constexpr (FWD != FWD_DENSITY && kDkEarly) first_loads<L, T, NT, true>(p2, tid, ldk);
   const float2 *twl = stw.to_lds(lds, tid);
-  fft_stages<L, T, NT, -1, 1, T, true, false, 1, true, true>(lds, twl, 1, tid, ld, st, p1);
-  if constexpr (FWD != FWD_DENSITY && !kDkEarly) first_loads<L, T, NT, true>(p2, tid, ldk);
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < NB0; ++q) {
-    const int g = tid + q * NT, c = g % T, j = g / T;
-#pragma unroll
-    for (int r = 0; r < R0; ++r) {
-      const float2 v = lds[c + (j + r * M0) * T];
-      p1[q * R0 + r] = FWD == FWD_DENSITY ? v : cadd(p2[q * R0 + r], v);
-    }
+  // delta(k) to add, in the layout of the inverse's first stage: requested before the
+  // forward's last stage, or after it where the registers are short
+  auto ldk = [&](int c, int j, int o) { return col_at<L, T>(dk + tile, ls, c, j, o); };
+  auto hook = [&]() {
+    if constexpr (FWD != FWD_DENSITY && kHand) first_loads<L, T, NT, true, kHand>(p2, tid, ldk);
+  };
+  fft_stages<L, T, NT, -1, 1, T, true, false, 1, !kHand, true>(lds, twl, 1, tid, ld, st, p1, hook);
+  if constexpr (!kHand) {
+    first_loads<L, T, NT, true, kHand>(p2, tid, ldk);
+    __syncthreads();
+    first_loads<L, T, NT, true, kHand>(p1, tid, [&](int c, int j, int o) { return lds[c + (j + o) * T]; });
   }
-  __syncthreads();
 #pragma unroll
-  for (int q = 0; q < NB0; ++q) {
+  for (int q = 0; q < E / RX; ++q) {
     const int g = tid + q * NT, c = g % T, j = g / T;
     const int kz = kz0 + c;
 #pragma unroll
-    for (int r = 0; r < R0; ++r) {
-      const int nx = nsgn(j + r * M0, N);
+    for (int r = 0; r < RX; ++r) {
+      const int i = q * RX + r, nx = nsgn(j + r * MX, N);
       const int n2 = nx * nx + ny * ny + kz * kz;
-      green_mul<MODE>(p1[q * R0 + r], nx, n2, kz <= N / 2, ga, p1[q * R0 + r], p2[q * R0 + r]);
+      const float2 S = FWD == FWD_DENSITY ? p1[i] : cadd(p2[i], p1[i]);
+      green_mul<MODE>(S, nx, n2, kz <= N / 2, ga, p1[i], p2[i]);
     }
   }
   auto ldz = [&](int, int, int) { return make_float2(0.f, 0.f); };
   auto st0 = [&](int c, int j, int o, float2 v) { col_at<L, T>(out0 + tile, ls, c, j, o) = v; };
-  fft_stages<L, T, NT, +1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ldz, st0, p1);
+  fft_stages<L, T, NT, +1, 1, T, true, true, 1, false, true, kHand>(lds, twl, 1, tid, ldz, st0, p1);
   if (MODE == GREEN_FORCE) {
-    __syncthreads();
     auto st1 = [&](int c, int j, int o, float2 v) { col_at<L, T>(out1 + tile, ls, c, j, o) = v; };
-    fft_stages<L, T, NT, +1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ldz, st1, p2);
+    fft_stages<L, T, NT, +1, 1, T, true, true, 1, false, true, kHand>(lds, twl, 1, tid, ldz, st1, p2);
   }
   if (bin) {
     __syncthreads();
-    for (int b = tid; b < nbins; b += NT)
-      if (bins[b] != 0.0) atomicAdd(&pk[b], bins[b]);
+    pl.flush(pk, fn, copies, tid);
   }
 }
 
@@ -367,51 +382,47 @@ enum { SCREEN_POTENTIAL = 0, SCREEN_DENSITY = 1 };
 //       delta_eff = delta * p0 * 2 (sqrt(1 + f) - 1) / f, f = p1 (1 + delta_R), 1 if f < 1e-5
 //                                                                   (p0 = coupling, p1 = dgp_fac)
 template <int N, int KIND>
-__global__ __launch_bounds__(RowCfg<N>::NT) void k_z_screen(float2 *buf, const float2 *__restrict__ dx, int HP,
+__global__ __launch_bounds__(RowCfg<N>::NT, N <= 1024 ? 4 : 1) void k_z_screen(float2 *buf, const float2 *__restrict__ dx, int HP,
                                                              size_t nrows, const float2 *__restrict__ tw, float p0,
                                                              float p1, size_t zs) {
   buf = zbuf(buf, zs);
   dx = zbuf(dx, zs);
   using C = RowCfg<N>;
-  constexpr int ITER = C::RB * C::M / C::NT;
-  static_assert(C::RB * C::M % C::NT == 0, "row block not a multiple of the block size");
+  constexpr int E = C::M * C::RB / C::NT, RL = last_radix(C::M, E), ML = C::M / RL;
   extern __shared__ float2 lds[];
   const int tid = threadIdx.x;
   const size_t row0 = (size_t)blockIdx.x * C::RB;
   // the delta(x) pairs this thread screens, loaded first so they arrive during the c2r
-  float2 dv[ITER];
+  float2 dv[E], f[E];
 #pragma unroll
-  for (int it = 0; it < ITER; ++it) {
-    const int e = tid + it * C::NT, r = e / C::M, n = e % C::M;
-    const size_t row = row0 + r < nrows ? row0 + r : nrows - 1;
-    dv[it] = dx[row * HP + n];
+  for (int q = 0; q < E / RL; ++q) {
+    const int g = tid + q * C::NT, j = g % ML;
+    const size_t row = row0 + g / ML < nrows ? row0 + g / ML : nrows - 1;
+#pragma unroll
+    for (int r = 0; r < RL; ++r) dv[q * RL + r] = dx[row * HP + j + r * ML];
   }
   z_merge<N, false>(lds, buf, HP, row0, nrows, tw, tid);
   __syncthreads();
   auto ldl = [&](int r, int j, int o) { return lds[r * C::LS + j + o]; };
   auto stl = [&](int r, int j, int o, float2 v) { lds[r * C::LS + j + o] = v; };
-  fft_stages<C::M, C::RB, C::NT, +1, C::LS, 1, false, true, 1>(lds, tw, 2, tid, ldl, stl);
-  __syncthreads();
-#pragma unroll
-  for (int it = 0; it < ITER; ++it) {
-    const int e = tid + it * C::NT, r = e / C::M, n = e % C::M;
-    const float2 f = lds[r * C::LS + n];
-    const float2 d = dv[it];
+  int oi = 0;  // output index of the store (a constant of the unrolled last stage)
+  auto sts = [&](int, int, int, float2 v) {
+    const float2 d = dv[oi];
     float s0, s1;
     if (KIND == SCREEN_POTENTIAL) {
-      s0 = f.x < 0.f ? fminf(1.f, fabsf(p0 / f.x)) : 1.f;
-      s1 = f.y < 0.f ? fminf(1.f, fabsf(p0 / f.y)) : 1.f;
+      s0 = v.x < 0.f ? fminf(1.f, fabsf(p0 / v.x)) : 1.f;
+      s1 = v.y < 0.f ? fminf(1.f, fabsf(p0 / v.y)) : 1.f;
     } else {
-      const float a0 = p1 * (1.f + f.x), a1 = p1 * (1.f + f.y);
+      const float a0 = p1 * (1.f + v.x), a1 = p1 * (1.f + v.y);
       s0 = p0 * (a0 < 1e-5f ? 1.f : 2.f * (sqrtf(1.f + a0) - 1.f) / a0);
       s1 = p0 * (a1 < 1e-5f ? 1.f : 2.f * (sqrtf(1.f + a1) - 1.f) / a1);
     }
-    lds[r * C::LS + n] = make_float2(d.x * s0, d.y * s1);
-  }
-  __syncthreads();
+    f[oi++] = make_float2(d.x * s0, d.y * s1);
+  };
+  fft_stages<C::M, C::RB, C::NT, +1, C::LS, 1, false, true, 1>(lds, tw, 2, tid, ldl, sts);
   float2 w[ZSplit<N>::ITER];
   z_split_twiddles<N>(w, tw, tid);
-  fft_stages<C::M, C::RB, C::NT, -1, C::LS, 1, false, true, 1>(lds, tw, 2, tid, ldl, stl);
+  fft_stages<C::M, C::RB, C::NT, -1, C::LS, 1, false, true, 1, false, true, true>(lds, tw, 2, tid, ldl, stl, f);
   __syncthreads();
   z_split<N>(lds, w, buf, HP, row0, nrows, tid);
 }
@@ -456,18 +467,27 @@ struct FusedXArgs {
   double *pk;
 };
 
+// two copies of the P(k) sums where the LDS has room for both (a third and fourth
+// gained nothing more)
+int pofk_copies(const mgpu_ctx *ctx, size_t tile_lds) {
+  const size_t l1 = tile_lds + pofk_lds(ctx->N, ctx->p.pofk_nbins, 1), l2 = tile_lds + pofk_lds(ctx->N, ctx->p.pofk_nbins, 2);
+  // not at the price of a workgroup per CU
+  return l2 <= ctx->lds_max && (ctx->lds_max / l2 == ctx->lds_max / l1 || ctx->lds_max / l2 >= 4) ? 2 : 1;
+}
+
 template <int N, int T, int FWD, int MODE>
 int fused_x_launch_k(mgpu_ctx *ctx, const FusedXArgs &a) {
   const size_t HP = ctx->fft.hp, ls = (size_t)N * HP, os = HP;
-  const int nbins = a.pk ? ctx->p.pofk_nbins : 0;
-  const size_t lds = col_lds_elems(N, T) * sizeof(float2) + (a.pk ? sizeof(double) * nbins + sizeof(float) * (N / 2 + 1) : 0);
+  const size_t tile_lds = col_lds_elems(N, T) * sizeof(float2);
+  const int copies = a.pk ? pofk_copies(ctx, tile_lds) : 1;
+  const size_t lds = tile_lds + (a.pk ? pofk_lds(N, ctx->p.pofk_nbins, copies) : 0);
   if (lds > ctx->lds_max) return mgpu_fail(ctx, MGPU_E_INVALID, "P(k) bins do not fit the LDS of the x pass");
-  if (a.pk && !ctx->pk_bin) return mgpu_fail(ctx, MGPU_E_INVALID, "no P(k) bin table");
+  if (a.pk && !ctx->pk_fn.edge) return mgpu_fail(ctx, MGPU_E_INVALID, "no P(k) bin table");
   int rc;
   auto kern = k_col_fused<N, T, FWD, MODE>;
   if ((rc = set_lds(ctx, kern, lds))) return rc;
   hipLaunchKernelGGL(kern, dim3(HP / T, N, ctx->bz), dim3(col_threads(N, T)), lds, ctx->stream, a.in, a.kout, a.dk,
-                     a.o0, a.o1, ls, os, ctx->fft.tw, a.ga, a.coupling, a.m2, ctx->winvf, ctx->pk_bin, nbins, a.pk,
+                     a.o0, a.o1, ls, os, ctx->fft.tw, a.ga, a.coupling, a.m2, ctx->winvf, ctx->pk_fn, copies, a.pk,
                      ctx->zs);
   MGPU_HIP(ctx, hipGetLastError());
   return MGPU_OK;
@@ -513,14 +533,15 @@ int epi_launch(mgpu_ctx *ctx, float2 *buf, float coupling, float m2) {
 template <int N, int T>
 int pofk_launch(mgpu_ctx *ctx, float2 *buf, double *pk) {
   const size_t HP = ctx->fft.hp, ls = (size_t)N * HP, os = HP;
-  const int nbins = ctx->p.pofk_nbins;
-  const size_t lds = col_lds_elems(N, T) * sizeof(float2) + sizeof(double) * nbins + sizeof(float) * (N / 2 + 1);
+  const size_t tile_lds = col_lds_elems(N, T) * sizeof(float2);
+  const int copies = pofk_copies(ctx, tile_lds);
+  const size_t lds = tile_lds + pofk_lds(N, ctx->p.pofk_nbins, copies);
   if (lds > ctx->lds_max) return mgpu_fail(ctx, MGPU_E_INVALID, "P(k) bins do not fit the LDS of the x pass");
-  if (!ctx->pk_bin) return mgpu_fail(ctx, MGPU_E_INVALID, "no P(k) bin table");
+  if (!ctx->pk_fn.edge) return mgpu_fail(ctx, MGPU_E_INVALID, "no P(k) bin table");
   int rc;
   if ((rc = set_lds(ctx, k_col_pofk<N, T>, lds))) return rc;
   hipLaunchKernelGGL((k_col_pofk<N, T>), dim3(HP / T, N), dim3(col_threads(N, T)), lds, ctx->stream, buf, ls, os,
-                     ctx->fft.tw, ctx->winvf, ctx->pk_bin, nbins, pk);
+                     ctx->fft.tw, ctx->winvf, ctx->pk_fn, copies, pk);
   MGPU_HIP(ctx, hipGetLastError());
   return MGPU_OK;
 }

@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../../include/mgpu.h"
+#include "pofk_bins.h"
 
 #define MGPU_PI 3.14159265358979323846
 #define MGPU_INVERSE_H0_MPCH 2997.92458
@@ -24,6 +25,8 @@
 #define MGPU_NSLOTS 4
 // seed-table entries of the allocation-free IC scratch: the Nmesh^2 columns of Nmesh = 2048
 #define MGPU_IC_SCRATCH_SEEDS (2048 * 2048)
+// sets of P(k) sums the x passes add into (the host adds the sets)
+#define MGPU_PK_SETS 8
 // columns per tile of the strided FFT passes (16: 128-byte row segments, 8: 64-byte)
 #ifndef MGPU_FFT_TCOLS
 #define MGPU_FFT_TCOLS 16
@@ -90,10 +93,11 @@ struct mgpu_ctx {
   double *partial = nullptr;  // per-block partial sums
   size_t partial_len = 0;
   double *dsum = nullptr;     // final sums
-  double *pk = nullptr;       // 3 * nbins
+  double *pk = nullptr;       // MGPU_PK_SETS * nbins
   double *winv = nullptr;     // P(k) deconvolution per axis: 1/sinc(pi d/N)^4 N^-2, d = 0..N/2
   float *winvf = nullptr;     // FP32 copy of winv
   int16_t *pk_bin = nullptr;  // P(k) bin of each |n|^2 (-1: outside the bins); null when nbins > 32767
+  PkBinFn pk_fn;              // the same bins by their edges; edge null when pk_bin is, or does not rise with |n|^2
   float4 *rsd_crd = nullptr;  // redshift-space particle records (allocated on the first RSD call)
   // massive neutrinos: PtoMesh's term delta = cdmfac delta + fac(|n|^2) cdelta_IC while nu_on
   bool nu_on = false;
@@ -209,6 +213,10 @@ void fft_plan_free(FFTPlan *plan);
 bool fft_tile16_fits(const mgpu_ctx *ctx, int n);
 // LDS bytes of a column pass of T columns (the tile, and the stage twiddles where they are held there)
 size_t fft_col_lds(int n, int T);
+// LDS bytes an x pass needs to bin P(k): copies sets of bin sums, the window of an axis, the bin edges
+static inline size_t pofk_lds(int n, int nbins, int copies) {
+  return copies * sizeof(double) * (size_t)nbins + sizeof(float) * (size_t)(n / 2 + 1) + sizeof(int) * (size_t)(nbins + 1);
+}
 int fft_autotune(mgpu_ctx *ctx, FFTPlan *plan, float2 *buf, double ms[2]);
 bool fft_size_supported(int n);
 // in-place 3D transforms on a slot with the padded layout above

@@ -20,7 +20,8 @@ constexpr int kBlock = 256;
 // the LDS takes several launches over bin ranges.
 __global__ __launch_bounds__(kBlock) void k_pofk(const float2 *__restrict__ dk, int N, int HP,
                                                  const double *__restrict__ winv, const int16_t *__restrict__ pbin,
-                                                 int nbins, int bintype, double kmin, double kmax, int b0, int nb,
+                                                 PkBinFn fn, int nbins, int bintype, double kmin, double kmax, int b0,
+                                                 int nb,
                                                  double *__restrict__ out) {
   extern __shared__ double sh[];  // 3*nb
   for (int b = threadIdx.x; b < 3 * nb; b += blockDim.x) sh[b] = 0.0;
@@ -28,6 +29,7 @@ __global__ __launch_bounds__(kBlock) void k_pofk(const float2 *__restrict__ dk, 
   const int H = N / 2 + 1;
   const size_t total = (size_t)N * N * H;
   const double lnrange = bintype == 1 ? log(kmax / kmin) : 1.0;
+  const int e0 = fn.edge ? fn.edge[0] : 0, e1 = fn.edge ? fn.edge[nbins] : 0;
   for (size_t m = (size_t)blockIdx.x * blockDim.x + threadIdx.x; m < total; m += (size_t)gridDim.x * blockDim.x) {
     const int k = (int)(m % H);
     const size_t rowi = m / H;
@@ -36,7 +38,8 @@ __global__ __launch_bounds__(kBlock) void k_pofk(const float2 *__restrict__ dk, 
     const int n2 = d0 * d0 + d1 * d1 + d2 * d2;
     const double kmag = sqrt((double)n2);
     int nk;
-    if (pbin) nk = pbin[n2];  // the same formula, evaluated by the host
+    if (fn.edge) nk = pk_bin_of(n2, fn, fn.edge, e0, e1);
+    else if (pbin) nk = pbin[n2];  // the same formula, evaluated by the host
     else if (bintype == 0) nk = (int)((kmag - kmin) / (kmax - kmin) * nbins + 0.5);
     else nk = kmag <= 0.0 ? -1 : (int)(log(kmag / kmin) / lnrange * nbins + 0.5);
     if (nk < 0 || nk >= nbins || nk < b0 || nk >= b0 + nb) continue;
@@ -88,20 +91,21 @@ __global__ __launch_bounds__(kBlock) void k_rsd_coords(const float *__restrict__
 // mu^2 = n_z^2/n^2, and the mode count; weights 1 (kz = 0, N/2) or 2.
 __global__ __launch_bounds__(kBlock) void k_rsd_bins(const float2 *__restrict__ dk, int N, int HP,
                                                      const double *__restrict__ winv,
-                                                     const int16_t *__restrict__ pbin, int nbins,
+                                                     const int16_t *__restrict__ pbin, PkBinFn fn, int nbins,
                                                      double *__restrict__ out) {
   extern __shared__ double sh[];  // 4*nbins
   for (int b = threadIdx.x; b < 4 * nbins; b += blockDim.x) sh[b] = 0.0;
   __syncthreads();
   const int H = N / 2 + 1;
   const size_t total = (size_t)N * N * H;
+  const int e0 = fn.edge ? fn.edge[0] : 0, e1 = fn.edge ? fn.edge[nbins] : 0;
   for (size_t m = (size_t)blockIdx.x * blockDim.x + threadIdx.x; m < total; m += (size_t)gridDim.x * blockDim.x) {
     const int k = (int)(m % H);
     const size_t rowi = m / H;
     const int j = (int)(rowi % N), i = (int)(rowi / N);
     const int d0 = i > N / 2 ? N - i : i, d1 = j > N / 2 ? N - j : j;
     const int n2 = d0 * d0 + d1 * d1 + k * k;
-    const int nk = pbin[n2];
+    const int nk = fn.edge ? pk_bin_of(n2, fn, fn.edge, e0, e1) : pbin[n2];
     if (nk < 0) continue;
     const double kmag = sqrt((double)n2);
     const double mu2 = k == 0 ? 0.0 : (double)(k * k) / kmag / kmag;
@@ -417,7 +421,7 @@ int pofk_setup(mgpu_ctx *ctx, double **dwin) {
   const int nbins = ctx->p.pofk_nbins;
   if (nbins <= 0) return mgpu_fail(ctx, MGPU_E_INVALID, "pofk_nbins must be positive");
   *dwin = ctx->winv;
-  MGPU_HIP(ctx, hipMemsetAsync(ctx->pk, 0, 3 * nbins * sizeof(double), ctx->stream));
+  MGPU_HIP(ctx, hipMemsetAsync(ctx->pk, 0, MGPU_PK_SETS * (size_t)nbins * sizeof(double), ctx->stream));
   return MGPU_OK;
 }
 
@@ -425,12 +429,15 @@ int pofk_setup(mgpu_ctx *ctx, double **dwin) {
 // |n| sums and mode counts come from ctx->pk_geom and only the power from the device
 int pofk_finish(mgpu_ctx *ctx, mgpu_pofk *out, bool geometry_from_ctx) {
   const int nbins = ctx->p.pofk_nbins;
-  std::vector<double> h(3 * nbins);
-  MGPU_HIP(ctx, hipMemcpyAsync(h.data(), ctx->pk, (geometry_from_ctx ? 1 : 3) * nbins * sizeof(double),
+  std::vector<double> h(MGPU_PK_SETS * (size_t)nbins);
+  MGPU_HIP(ctx, hipMemcpyAsync(h.data(), ctx->pk, (geometry_from_ctx ? MGPU_PK_SETS : 3) * (size_t)nbins * sizeof(double),
                                hipMemcpyDeviceToHost, ctx->stream));
   MGPU_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  // the x pass adds into MGPU_PK_SETS sets of sums; k_pofk into the first, with the |n| sums and counts behind it
+  for (int c = 1; geometry_from_ctx && c < MGPU_PK_SETS; c++)
+    for (int b = 0; b < nbins; b++) h[b] += h[(size_t)c * nbins + b];
   if (geometry_from_ctx) std::copy(ctx->pk_geom.begin(), ctx->pk_geom.end(), h.begin() + nbins);
-  else ctx->pk_geom.assign(h.begin() + nbins, h.end());
+  else ctx->pk_geom.assign(h.begin() + nbins, h.begin() + 3 * (size_t)nbins);
   const double box3 = std::pow(ctx->p.box, 3);
   const double shot = std::pow(ctx->p.box / (double)ctx->Np, 3);
   for (int b = 0; b < nbins; b++) {
@@ -467,7 +474,7 @@ int pm_pofk(mgpu_ctx *ctx, const float2 *dk, mgpu_pofk *out) {
     const int nb = std::min(chunk, nbins - b0);
     KScope ks(ctx, MGPU_K_POFK, 8.0 * modes);
     hipLaunchKernelGGL(k_pofk, dim3(grid), dim3(kBlock), 3 * (size_t)nb * sizeof(double), ctx->stream, dk, N, ctx->HP,
-                       dwin, ctx->pk_bin, nbins, ctx->p.pofk_bintype, ctx->p.pofk_kmin, ctx->p.pofk_kmax, b0, nb,
+                       dwin, ctx->pk_bin, ctx->pk_fn, nbins, ctx->p.pofk_bintype, ctx->p.pofk_kmin, ctx->p.pofk_kmax, b0, nb,
                        ctx->pk);
     MGPU_HIP(ctx, hipGetLastError());
   }
@@ -476,9 +483,7 @@ int pm_pofk(mgpu_ctx *ctx, const float2 *dk, mgpu_pofk *out) {
 
 // The x pass that bins P(k) holds its tile of T columns and the bins in LDS.
 static bool pofk_fused_fits(const mgpu_ctx *ctx, int T) {
-  const size_t need = fft_col_lds(ctx->N, T) + sizeof(double) * (size_t)ctx->p.pofk_nbins +
-                      sizeof(float) * (size_t)(ctx->N / 2 + 1);
-  return need <= ctx->lds_max;
+  return ctx->pk_fn.edge && fft_col_lds(ctx->N, T) + pofk_lds(ctx->N, ctx->p.pofk_nbins, 1) <= ctx->lds_max;
 }
 
 // PtoMesh's r2c of delta(x) (slot dx_slot) into slot 0, with P(k) when out != NULL.
@@ -488,7 +493,7 @@ int pm_transform(mgpu_ctx *ctx, mgpu_pofk *out) {
   float2 *dk = ctx->slot[0];
   const float *dx = (const float *)ctx->slot[ctx->dx_slot];
   int rc;
-  if (!out || !ctx->pk_bin || ctx->pk_geom.size() != 2 * (size_t)ctx->p.pofk_nbins ||
+  if (!out || ctx->pk_geom.size() != 2 * (size_t)ctx->p.pofk_nbins ||
       !pofk_fused_fits(ctx, ctx->fft.tcols)) {
     {
       PhaseTimer pt(ctx, &ctx->t.ptomesh);
@@ -613,7 +618,7 @@ static int forces_tail(mgpu_ctx *ctx) {
 
 bool pm_step_fusable(const mgpu_ctx *ctx, const mgpu_mg *mg, const mgpu_pofk *out) {
   if (ctx->nu_on) return false;  // the neutrino term sits between the density's x pass and the next
-  if (out && (!ctx->pk_bin || ctx->pk_geom.size() != 2 * (size_t)ctx->p.pofk_nbins)) return false;
+  if (out && ctx->pk_geom.size() != 2 * (size_t)ctx->p.pofk_nbins) return false;
   // the density pair bins P(k) in LDS: 8-column tiles with the Green's force (LCDM), else the plan's width
   const bool lcdm = !ctx->p.mg_active || ctx->p.model == MGPU_LCDM;
   if (out && !pofk_fused_fits(ctx, lcdm ? 8 : ctx->fft.tcols)) return false;
@@ -843,7 +848,7 @@ int pm_rsd_pofk(mgpu_ctx *ctx, int axis, double vnorm, double s1, double s2, mgp
   {
     KScope ks(ctx, MGPU_K_POFK, 8.0 * modes);
     hipLaunchKernelGGL(k_rsd_bins, dim3(std::min<size_t>(cdiv(modes, kBlock), 4096)), dim3(kBlock), shmem, ctx->stream,
-                       dk, N, ctx->HP, ctx->winv, ctx->pk_bin, nbins, ctx->pk);
+                       dk, N, ctx->HP, ctx->winv, ctx->pk_bin, ctx->pk_fn, nbins, ctx->pk);
   }
   MGPU_HIP(ctx, hipGetLastError());
   std::vector<double> h(4 * (size_t)nbins);

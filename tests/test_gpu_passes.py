@@ -1,0 +1,72 @@
+"""The FFT passes' radix schedules and the P(k) bin edges at the sizes where they change:
+one radix (8-16), a radix 12 first or reversed (12-192), no LDS stage, odd bin counts."""
+import numpy as np
+import pytest
+
+import mgpicola as M
+import oracle as O
+from helpers import lattice_particles, rel_err
+
+pytestmark = pytest.mark.gpu
+BOX, OM = 64.0, 0.3
+
+
+@pytest.mark.parametrize("model", ["lcdm", "fofr", "dgp"])
+@pytest.mark.parametrize("n", [8, 12, 16, 24, 64, 96, 192])
+@pytest.mark.parametrize("tcols", [8, 16])
+def test_x_pass_pairs_and_screening_row(model, n, tcols):
+    """GetDisplacements' paired x passes and screening rows against the oracle.  The force
+    meshes hold FP32 rounding of 3 log2(n)-stage transforms: 3e-5 of the field maximum, the
+    bound of the oracle comparisons of the separate passes."""
+    ns = n // 2
+    pos = lattice_particles(ns, BOX, amp=1.5, seed=n)
+    kw, okw, mg, omg = {}, {}, None, None
+    if model != "lcdm":
+        d = dict(a=0.7, coupling=1 / 3 if model == "fofr" else 0.12, mass2=2e4, phi_crit=3e-8, dgp_fac=0.05,
+                 rsmooth=2.0, geff=1.0)
+        okw = dict(model=O.FOFR if model == "fofr" else O.DGP, mg_active=1, include_screening=1,
+                   filter=O.FILTER_GAUSSIAN if model == "dgp" else O.FILTER_NONE)
+        kw, mg, omg = dict(okw), M.MG(**d), O.MG(**d)
+    print("model, n, tcols =", model, n, tcols, flush=True)
+    g = M.MGPU(n, ns, BOX, OM, pofk_nbins=n // 2 + 1, pofk_subtract_shotnoise=0, **kw)
+    g.set_fft_tile(0, tcols)
+    g.set_particles(pos)
+    g.get_displacements(mg=mg, pofk=True)  # records the mode counts
+    _, (pk, _, nm) = g.get_displacements(mg=mg, pofk=True)
+    c = O.cfg(n, ns, BOX, OM, **okw)
+    dk = O.deposit(c, pos)
+    dx = dk.copy()
+    O.fft_r2c_3d(n, dk)
+    rp, _, rn = O.pofk(c, dk, n // 2 + 1, 0, 0.0, float(n), 0)
+    f = O.forces(c, dk, O.fifth_force(c, omg, dk, dx) if omg is not None else None)
+    for a, mid in enumerate((M.MESH_FORCE_X, M.MESH_FORCE_Y, M.MESH_FORCE_Z)):
+        assert rel_err(g.get_mesh(mid), O.real_view(f[a], n)) < 3e-5
+    assert np.array_equal(nm, rn)
+    ok = (rn > 0) & (np.arange(rn.size) > 0)
+    np.testing.assert_allclose(pk[ok], rp[ok], rtol=1e-3)
+    g.close()
+
+
+@pytest.mark.parametrize("nbins,bintype,kmin,kmax", [(1, 0, 0.0, 48.0), (7, 0, 3.0, 11.5), (48, 1, 1.0, 48.0),
+                                                     (333, 0, 0.0, 48.0), (500, 1, 2.5, 30.0)])
+def test_pofk_bins_by_edges(nbins, bintype, kmin, kmax):
+    """Every mode in the bin of the FP64 formula: mode counts equal the oracle's, for bins
+    wider and finer than a mode, with modes below the first bin and past the last, in
+    k_pofk (first call), the density x pass (second call) and the fused pair."""
+    n, ns = 48, 24
+    pos = lattice_particles(ns, BOX, amp=1.5, seed=5)
+    g = M.MGPU(n, ns, BOX, OM, pofk_nbins=nbins, pofk_bintype=bintype, pofk_kmin=kmin, pofk_kmax=kmax,
+               pofk_subtract_shotnoise=0)
+    g.set_particles(pos)
+    got = [g.pm_density(pofk=True), g.pm_density(pofk=True), g.get_displacements(pofk=True)[1]]
+    c = O.cfg(n, ns, BOX, OM)
+    dk = O.deposit(c, pos)
+    O.fft_r2c_3d(n, dk)
+    rp, rk, rn = O.pofk(c, dk, nbins, bintype, kmin, kmax, 0)
+    ok = (rn > 0) & (rk > 0)
+    for pk, kk, nm in got:
+        assert np.array_equal(nm, rn)
+        np.testing.assert_allclose(kk[ok], rk[ok], rtol=1e-12)
+        # one lost or misplaced mode changes a sparse bin by its share of the power
+        np.testing.assert_allclose(pk[ok], rp[ok], rtol=1e-3)
+    g.close()
