@@ -294,6 +294,14 @@ int create_ctx(const mgpu_params *p, mgpu_ctx **out, mgpu_arena *arena, char *sh
   if ((rc = alloc(ctx, (void **)&ctx->dsum, 8 * sizeof(double), "sums"))) return fail(rc);
   const int nb = std::max(1, p->pofk_nbins);
   if ((rc = alloc(ctx, (void **)&ctx->pk, MGPU_PK_SETS * (size_t)nb * sizeof(double), "P(k) bins"))) return fail(rc);
+  // device-visible host memory: a kernel's stores are complete when the stream has been waited for
+  if (hipHostMalloc((void **)&ctx->host_sums, (8 + MGPU_PK_SETS * (size_t)nb) * sizeof(double), hipHostMallocDefault) !=
+      hipSuccess) {
+    (void)hipGetLastError();
+    ctx->host_sums = nullptr;
+    return fail(mgpu_fail(ctx, MGPU_E_NOMEM, "host allocation of the sums failed"));
+  }
+  ctx->host_pk = ctx->host_sums + 8;
   {
     // compute_power_spectrum's CIC deconvolution 1/(W_x W_y W_z)^4 with the 1/N^6 of the
     // transform split over the three axes (src/compute_pofk.c:128-134)
@@ -404,6 +412,7 @@ void mgpu_destroy(mgpu_ctx *ctx) {
   for (void *q : ptrs)
     if (q && !((const char *)q >= a0 && (const char *)q < a1)) (void)hipFree(q);
   if (ctx->slice_host) (void)hipHostFree(ctx->slice_host);
+  if (ctx->host_sums) (void)hipHostFree(ctx->host_sums);
   if (ctx->slice_ev) (void)hipEventDestroy(ctx->slice_ev);
   fft_plan_free(&ctx->fft);
   fft_plan_free(&ctx->fft_lattice);
@@ -749,6 +758,7 @@ int run_step(mgpu_ctx *ctx, const mgpu_mg *mg, double dda, double A, double s1k,
     if (rc || e != hipSuccess || !g) {
       if (g) (void)hipGraphDestroy(g);
       (void)hipGetLastError();
+      ctx->dep_counts_zero = false;  // nothing of the capture has run
       return rc ? rc : mgpu_fail(ctx, MGPU_E_HIP, std::string("step capture failed: ") + hipGetErrorString(e));
     }
     if (ctx->step_exec) {
@@ -764,6 +774,7 @@ int run_step(mgpu_ctx *ctx, const mgpu_mg *mg, double dda, double A, double s1k,
     if (!ctx->step_exec && hipGraphInstantiate(&ctx->step_exec, g, nullptr, nullptr, 0) != hipSuccess) {
       ctx->step_exec = nullptr;
       (void)hipGraphDestroy(g);
+      ctx->dep_counts_zero = false;
       return mgpu_fail(ctx, MGPU_E_HIP, "step graph instantiation failed");
     }
     (void)hipGraphDestroy(g);
@@ -891,10 +902,14 @@ int mgpu_batch_step(mgpu_ctx *const *members, int count, const mgpu_mg *mg, doub
     if (m->fft.tcols != m0->fft.tcols) return mgpu_fail(m0, MGPU_E_STATE, "the members' FFT tile widths differ");
   }
   // realization 0's launches with grid z = count reach every member
+  for (int r = 1; r < count; r++) m0->dep_counts_zero = m0->dep_counts_zero && members[r]->dep_counts_zero;
   m0->bz = (unsigned)count;
   rc = run_step(m0, mg, dda, A, s1k, s2k, dyyy, s1d, s2d, graph);
   m0->bz = 1;
-  if (rc) return rc;
+  if (rc) {
+    for (int r = 0; r < count; r++) members[r]->dep_counts_zero = false;
+    return rc;
+  }
   const size_t rec_off = (const char *)m0->dep_rec - (const char *)m0->dep_scratch;
   const size_t off_off = (const char *)m0->dep_off - (const char *)m0->dep_scratch;
   for (int r = 1; r < count; r++) {
@@ -911,6 +926,7 @@ int mgpu_batch_step(mgpu_ctx *const *members, int count, const mgpu_mg *mg, doub
     m->dep_rec = (float4 *)((char *)m->dep_scratch + rec_off);
     m->dep_off = (unsigned *)((char *)m->dep_scratch + off_off);
     m->sorted_valid = m0->sorted_valid;
+    m->dep_counts_zero = m0->dep_counts_zero;
     m->vsum_valid = m0->vsum_valid;
     m->dep_tiles_grid = m0->dep_tiles_grid;
   }

@@ -96,19 +96,16 @@ __global__ __launch_bounds__(RowCfg<N>::NT) void k_fft_z_r2c(const float2 *in, f
 
 // c2r along z: X[0..N/2] (Im of ends dropped) -> real row.  The row is written
 // to out with a row stride of orow float2 (out = buf, orow = HP in place; or a
-// compact [N^2][N] real array, orow = N/2).  IKZ multiplies X[k] by i k first
+// compact [N^2][N] real array, orow = N/2).  ikz multiplies X[k] by i k first
 // (the z force component, k the kz index).
-template <int N, bool IKZ>
-__global__ __launch_bounds__(RowCfg<N>::NT) void k_fft_z_c2r(const float2 *buf, int HP, size_t nrows,
-                                                              const float2 *__restrict__ tw, float2 *out, int orow,
-                                                              size_t zs) {
-  buf = zbuf(buf, zs);
-  out = zbuf(out, zs);
+template <int N>
+__device__ __forceinline__ void z_c2r_rows(const float2 *buf, int HP, size_t nrows, const float2 *__restrict__ tw,
+                                           float2 *out, int orow, bool ikz) {
   using C = RowCfg<N>;
   extern __shared__ float2 lds[];
   const int tid = threadIdx.x;
   const size_t row0 = (size_t)blockIdx.x * C::RB;
-  z_merge<N, IKZ>(lds, buf, HP, row0, nrows, tw, tid);
+  z_merge<N>(lds, buf, HP, row0, nrows, tw, tid, ikz);
   __syncthreads();
   auto ld = [&](int r, int j, int o) { return lds[r * C::LS + j + o]; };
   auto st = [&](int r, int j, int o, float2 v) {
@@ -116,6 +113,22 @@ __global__ __launch_bounds__(RowCfg<N>::NT) void k_fft_z_c2r(const float2 *buf, 
     if (row < nrows) out[row * orow + j + o] = v;
   };
   fft_stages<C::M, C::RB, C::NT, +1, C::LS, 1, false, true, 1>(lds, tw, 2, tid, ld, st);
+}
+template <int N>
+__global__ __launch_bounds__(RowCfg<N>::NT) void k_fft_z_c2r(const float2 *buf, int HP, size_t nrows,
+                                                              const float2 *__restrict__ tw, float2 *out, int orow,
+                                                              size_t zs) {
+  z_c2r_rows<N>(zbuf(buf, zs), HP, nrows, tw, zbuf(out, zs), orow, false);
+}
+// The three force components in one launch (grid y = component; the z component with
+// i k): one mesh after the other in the order of the blocks, as three launches would
+// run, without the gaps and the part-filled ends of three (128: 24.9 us for the three).
+template <int N>
+__global__ __launch_bounds__(RowCfg<N>::NT) void k_fft_z_c2r3(float2 *f0, float2 *f1, float2 *f2, int HP,
+                                                               size_t nrows, const float2 *__restrict__ tw,
+                                                               size_t zs) {
+  float2 *buf = zbuf(blockIdx.y == 0 ? f0 : blockIdx.y == 1 ? f1 : f2, zs);
+  z_c2r_rows<N>(buf, HP, nrows, tw, buf, HP, blockIdx.y == 2);
 }
 
 // tiles per block of the column passes: two (software-pipelined) for the
@@ -152,7 +165,7 @@ int launch_z(mgpu_ctx *ctx, float2 *buf, int HP, const float2 *tw, int forward, 
     hipLaunchKernelGGL(kern, grid, dim3(C::NT), lds, ctx->stream, in ? in : (const float2 *)buf, buf, HP, nrows, tw,
                        ctx->zs);
   } else {
-    auto kern = k_fft_z_c2r<N, false>;
+    auto kern = k_fft_z_c2r<N>;
     if (lds > 65536) MGPU_HIP(ctx, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(kern, grid, dim3(C::NT), lds, ctx->stream, (const float2 *)buf, HP, nrows, tw,
                        out ? out : buf, out ? N / 2 : HP, ctx->zs);
@@ -287,19 +300,19 @@ int fft_pass_col(mgpu_ctx *ctx, const FFTPlan *plan, float2 *buf, int axis, int 
   }
 }
 
-int fft_pass_z_ikz(mgpu_ctx *ctx, const FFTPlan *plan, float2 *buf) {
+int fft_pass_z_force(mgpu_ctx *ctx, const FFTPlan *plan, float2 *f0, float2 *f1, float2 *f2) {
   const double rows = (double)plan->n * plan->n;
-  KScope ks(ctx, MGPU_K_FFT_C2R, rows * (plan->n * 4.0 + (plan->n / 2 + 1) * 8.0));
+  KScope ks(ctx, MGPU_K_FFT_C2R, 3.0 * rows * (plan->n * 4.0 + (plan->n / 2 + 1) * 8.0));
   switch (plan->n) {
 #define X(S)                                                                                                    \
   case S: {                                                                                                     \
     using C = RowCfg<S>;                                                                                        \
     const size_t nrows = (size_t)S * S, lds = (size_t)C::RB * C::LS * sizeof(float2);                           \
-    auto kern = k_fft_z_c2r<S, true>;                                                                           \
+    auto kern = k_fft_z_c2r3<S>;                                                                                \
     if (lds > 65536)                                                                                            \
       MGPU_HIP(ctx, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
-    hipLaunchKernelGGL(kern, dim3(cdiv(nrows, C::RB), 1, ctx->bz), dim3(C::NT), lds, ctx->stream,              \
-                       (const float2 *)buf, plan->hp, nrows, plan->tw, buf, plan->hp, ctx->zs);                 \
+    hipLaunchKernelGGL(kern, dim3(cdiv(nrows, C::RB), 3, ctx->bz), dim3(C::NT), lds, ctx->stream, f0, f1, f2,   \
+                       plan->hp, nrows, plan->tw, ctx->zs);                                                     \
     MGPU_HIP(ctx, hipGetLastError());                                                                           \
     return MGPU_OK;                                                                                             \
   }

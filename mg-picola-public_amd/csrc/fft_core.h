@@ -438,10 +438,11 @@ __device__ __forceinline__ void z_split(const float2 *lds, const float2 *w, floa
 }
 // merge: Z[k] = (X_k + X*_{M-k}) + i w^k (X_k - X*_{M-k}), w = e^{+2 pi i/N}, from
 // the rows of buf (Im of X_0 and X_M dropped) into LDS.  Every global load of
-// the block's rows is issued before any is used.  IKZ: X_k -> i k X_k first.
-template <int N, bool IKZ>
+// the block's rows is issued before any is used.  ikz (the same for the whole
+// workgroup): X_k -> i k X_k first.
+template <int N>
 __device__ __forceinline__ void z_merge(float2 *lds, const float2 *buf, int HP, size_t row0, size_t nrows,
-                                        const float2 *__restrict__ tw, int tid) {
+                                        const float2 *__restrict__ tw, int tid, bool ikz = false) {
   using C = RowCfg<N>;
   constexpr int HALF = C::M / 2 + 1;
   constexpr int ITER = (C::RB * HALF + C::NT - 1) / C::NT;
@@ -465,7 +466,7 @@ __device__ __forceinline__ void z_merge(float2 *lds, const float2 *buf, int HP, 
     const int r = e / HALF, k = e % HALF;
     const int kk = C::M - k;
     float2 a = xk[it], b = xm[it];
-    if (IKZ) {
+    if (ikz) {
       a = cscale(mul_i<+1>(a), (float)k);
       b = cscale(mul_i<+1>(b), (float)kk);
     }

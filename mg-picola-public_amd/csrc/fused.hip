@@ -157,6 +157,48 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_dual(float2 *buf, flo
   fft_stages<L, T, NT, +1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ld, st1, p2);
 }
 
+// The y passes of the force tail in one launch, for meshes whose launches are short:
+// even rows of the grid take k_col_dual's tiles, odd rows the inverse y pass of other.
+// Each row of the grid is one kx (see k_col_dual).
+constexpr int kForceYOne = 256;
+template <int L, int T>
+__global__ __launch_bounds__(col_threads(L, T)) void k_col_force_y(float2 *buf, float2 *__restrict__ oy, float2 *other,
+                                                                     size_t ls, size_t os,
+                                                                     const float2 *__restrict__ tw, size_t zs) {
+  buf = zbuf(buf, zs);
+  oy = zbuf(oy, zs);
+  other = zbuf(other, zs);
+  extern __shared__ float2 lds[];
+  constexpr int NT = col_threads(L, T), E = col_ept(L, T);
+  constexpr int R0 = pick_radix(L, E), NB0 = E / R0, M0 = L / R0;
+  const int tid = threadIdx.x;
+  int bx, by;
+  xcd_tile(bx, by);
+  const bool dual = (by & 1) == 0;  // the same for the whole workgroup
+  const size_t tile = (size_t)(by >> 1) * os + (size_t)bx * T;
+  const float2 *src = dual ? buf : other;
+  StageTwiddles<L, T, NT> stw(tw, tid);
+  float2 p1[E], p2[E];
+  first_loads<L, T, NT, true>(p2, tid, [&](int c, int j, int o) { return col_at<L, T>(src + tile, ls, c, j, o); });
+  const float2 *twl = stw.to_lds(lds, tid);
+  auto ld = [&](int, int, int) { return make_float2(0.f, 0.f); };
+  if (dual) {
+#pragma unroll
+    for (int q = 0; q < NB0; ++q) {
+      const int j = (tid + q * NT) / T;
+#pragma unroll
+      for (int r = 0; r < R0; ++r)
+        p1[q * R0 + r] = cscale(mul_i<+1>(p2[q * R0 + r]), (float)nsgn(j + r * M0, L));
+    }
+    auto st0 = [&](int c, int j, int o, float2 v) { col_at<L, T>(oy + tile, ls, c, j, o) = v; };
+    fft_stages<L, T, NT, +1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ld, st0, p1);
+    __syncthreads();
+  }
+  float2 *dst = dual ? buf : other;
+  auto st1 = [&](int c, int j, int o, float2 v) { col_at<L, T>(dst + tile, ls, c, j, o) = v; };
+  fft_stages<L, T, NT, +1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ld, st1, p2);
+}
+
 // x pass, forward, then phi = coupling n^2/(n^2 + m2) X (0 at n = 0): EffDensitykToPhiofk
 // (src/mg.h:74-116) on the transform's output.  Tile: columns kz, outer ky, line kx.
 template <int L, int T>
@@ -188,7 +230,9 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_epi(float2 *buf, size
 
 // P(k) sums of an x pass in LDS: copies sets of bin sums (lanes take them in turn, so
 // fewer lanes of a wave add to one address: most of a wave's modes share a few bins),
-// the per-axis window and the bin edges.
+// the per-axis window and the bin edges.  init() goes behind the tile's loads, so that
+// it costs no latency of its own, and in front of the twiddles' barrier (or, without
+// one, of the stages' barriers).
 template <int L, int NT>
 struct PofkLds {
   double *bins;
@@ -203,9 +247,11 @@ struct PofkLds {
     for (int b = tid; b < copies * f.nbins; b += NT) bins[b] = 0.0;
     for (int d = tid; d <= L / 2; d += NT) wv[d] = winv[d];
     for (int b = tid; b <= f.nbins; b += NT) edge[b] = f.edge[b];
-    e0 = f.edge[0];
-    e1 = f.edge[f.nbins];
-    __syncthreads();
+  }
+  // after a barrier
+  __device__ __forceinline__ void begin(const PkBinFn &f) {
+    e0 = edge[0];
+    e1 = edge[f.nbins];
   }
   // mode (kx, d1 = |ky|, kz) of power |v|^2: weight 1 (kz = 0, N/2) or 2, CIC deconvolution
   __device__ __forceinline__ void add(float2 v, int kx, int d1, int kz, const PkBinFn &f, int copies, int tid) const {
@@ -244,7 +290,6 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_pofk(float2 *buf, siz
   constexpr int N = L;
   const int tid = threadIdx.x;
   PofkLds<L, NT> pl;
-  pl.init(lds + col_lds_elems(L, T), fn, copies, winv, tid);
   int bx, ky;
   xcd_tile(bx, ky);
   const int kz0 = bx * T;
@@ -258,8 +303,9 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_pofk(float2 *buf, siz
   StageTwiddles<L, T, NT> stw(tw, tid);
   float2 pre[col_ept(L, T)];
   first_loads<L, T, NT, true>(pre, tid, ld);
+  pl.init(lds + col_lds_elems(L, T), fn, copies, winv, tid);
   const float2 *twl = stw.to_lds(lds, tid);
-  fft_stages<L, T, NT, -1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ld, st, pre);
+  fft_stages<L, T, NT, -1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ld, st, pre, [&]() { pl.begin(fn); });
   __syncthreads();
   pl.flush(pk, fn, copies, tid);
 }
@@ -312,7 +358,6 @@ __global__ __launch_bounds__(col_threads(L, T), tw_in_lds(L) ? 4 : 1) void k_col
   const int ny = nsgn(ky, N), d1 = ky > N / 2 ? N - ky : ky;
   const bool bin = FWD == FWD_DENSITY && pk != nullptr;
   PofkLds<L, NT> pl;
-  if (bin) pl.init(lds + col_lds_elems(L, T), fn, copies, winv, tid);
   // forward transform; its outputs stay in the registers of the threads that form them
   float2 p1[E], p2[E];
   auto ld = [&](int c, int j, int o) { return col_at<L, T>(in + tile, ls, c, j, o); };
@@ -333,12 +378,14 @@ __global__ __launch_bounds__(col_threads(L, T), tw_in_lds(L) ? 4 : 1) void k_col
   };
   StageTwiddles<L, T, NT> stw(tw, tid);
   first_loads<L, T, NT, true>(p1, tid, ld);
+  if (bin) pl.init(lds + col_lds_elems(L, T), fn, copies, winv, tid);
   const float2 *twl = stw.to_lds(lds, tid);
   // delta(k) to add, in the layout of the inverse's first stage: requested before the
   // forward's last stage, or after it where the registers are short
   auto ldk = [&](int c, int j, int o) { return col_at<L, T>(dk + tile, ls, c, j, o); };
   auto hook = [&]() {
     if constexpr (FWD != FWD_DENSITY && kHand) first_loads<L, T, NT, true, kHand>(p2, tid, ldk);
+    if (bin) pl.begin(fn);
   };
   fft_stages<L, T, NT, -1, 1, T, true, false, 1, !kHand, true>(lds, twl, 1, tid, ld, st, p1, hook);
   if constexpr (!kHand) {
@@ -401,7 +448,7 @@ __global__ __launch_bounds__(RowCfg<N>::NT, N <= 1024 ? 4 : 1) void k_z_screen(f
 #pragma unroll
     for (int r = 0; r < RL; ++r) dv[q * RL + r] = dx[row * HP + j + r * ML];
   }
-  z_merge<N, false>(lds, buf, HP, row0, nrows, tw, tid);
+  z_merge<N>(lds, buf, HP, row0, nrows, tw, tid);
   __syncthreads();
   auto ldl = [&](int r, int j, int o) { return lds[r * C::LS + j + o]; };
   auto stl = [&](int r, int j, int o, float2 v) { lds[r * C::LS + j + o] = v; };
@@ -519,6 +566,18 @@ int dual_launch(mgpu_ctx *ctx, float2 *buf, float2 *oy) {
 }
 
 template <int N, int T>
+int force_y_launch(mgpu_ctx *ctx, float2 *buf, float2 *oy, float2 *other) {
+  const size_t HP = ctx->fft.hp, ls = HP, os = (size_t)N * HP;
+  const size_t lds = col_lds_elems(N, T) * sizeof(float2);
+  int rc;
+  if ((rc = set_lds(ctx, k_col_force_y<N, T>, lds))) return rc;
+  hipLaunchKernelGGL((k_col_force_y<N, T>), dim3(HP / T, 2 * N, ctx->bz), dim3(col_threads(N, T)), lds, ctx->stream, buf,
+                     oy, other, ls, os, ctx->fft.tw, ctx->zs);
+  MGPU_HIP(ctx, hipGetLastError());
+  return MGPU_OK;
+}
+
+template <int N, int T>
 int epi_launch(mgpu_ctx *ctx, float2 *buf, float coupling, float m2) {
   const size_t HP = ctx->fft.hp, ls = (size_t)N * HP, os = HP;
   const size_t lds = col_lds_elems(N, T) * sizeof(float2);
@@ -583,6 +642,10 @@ struct GreenF {
 template <int N, int T>
 struct DualF {
   static int run(mgpu_ctx *c, float2 *buf, float2 *oy) { return dual_launch<N, T>(c, buf, oy); }
+};
+template <int N, int T>
+struct ForceYF {
+  static int run(mgpu_ctx *c, float2 *buf, float2 *oy, float2 *other) { return force_y_launch<N, T>(c, buf, oy, other); }
 };
 template <int N, int T>
 struct PofkF {
@@ -668,6 +731,26 @@ int fused_dual_y(mgpu_ctx *ctx, float2 *buf, float2 *oy) {
     default:
       return mgpu_fail(ctx, MGPU_E_INVALID, "unsupported FFT size");
   }
+}
+
+int fused_force_y(mgpu_ctx *ctx, float2 *buf, float2 *oy, float2 *other) {
+  // one launch up to 256, where a pass is short against a launch (128: 16.6 us for the
+  // two launches); beyond, the plain pass keeps its own kernel's occupancy
+  if (ctx->N <= kForceYOne) {
+    const double modes = (double)ctx->N * ctx->N * (ctx->N / 2 + 1);
+    KScope ks(ctx, MGPU_K_FFT_DUAL, 8.0 * modes * 5);
+    switch (ctx->N) {
+#define X(S) \
+  case S:    \
+    if constexpr (S <= kForceYOne) return by_tile<S, ForceYF>(ctx, buf, oy, other);
+      MGPU_FFT_SIZES(X)
+#undef X
+      default:
+        return mgpu_fail(ctx, MGPU_E_INVALID, "unsupported FFT size");
+    }
+  }
+  int rc = fused_dual_y(ctx, buf, oy);
+  return rc ? rc : fft_pass_col(ctx, &ctx->fft, other, 1, 0);
 }
 
 int fused_epi_phi_x(mgpu_ctx *ctx, float2 *buf, double coupling, double massterm2) {

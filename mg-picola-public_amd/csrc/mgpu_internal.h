@@ -93,6 +93,8 @@ struct mgpu_ctx {
   double *partial = nullptr;  // per-block partial sums
   size_t partial_len = 0;
   double *dsum = nullptr;     // final sums
+  double *host_sums = nullptr;  // pinned: the last sums that went to the host
+  double *host_pk = nullptr;    // pinned: MGPU_PK_SETS * nbins P(k) or RSD sums (part of host_sums' allocation)
   double *pk = nullptr;       // MGPU_PK_SETS * nbins
   double *winv = nullptr;     // P(k) deconvolution per axis: 1/sinc(pi d/N)^4 N^-2, d = 0..N/2
   float *winvf = nullptr;     // FP32 copy of winv
@@ -131,6 +133,7 @@ struct mgpu_ctx {
   float4 *dep_rec = nullptr;       // particle records (x, y, z, index bits) in bin order (inside dep_scratch)
   unsigned *dep_off = nullptr;     // bin offsets of dep_rec, 8 bins (face classes) per tile
   bool sorted_valid = false;       // dep_rec holds the current positions
+  bool dep_counts_zero = false;    // the bin counters are zero (the scan leaves them so)
   unsigned dep_tiles_grid = 0;     // workgroups of the persistent tile deposit (0: not yet measured)
   // device-resident step (mgpu_step): dsum[0..2] the Disp sums of the last gather, dsum[3..5] the velocity
   // sums of the last kick; vsum_valid when dsum[3..5] matches the velocities
@@ -229,8 +232,8 @@ int fft_pass_z(mgpu_ctx *ctx, const FFTPlan *plan, float2 *buf, int forward, flo
                const float *in = nullptr);
 int fft_pass_col(mgpu_ctx *ctx, const FFTPlan *plan, float2 *buf, int axis, int forward);
 
-// z c2r of the force's z component: X(k) -> i kz X(k) before the transform (in place)
-int fft_pass_z_ikz(mgpu_ctx *ctx, const FFTPlan *plan, float2 *buf);
+// z c2r of the three force components in place, of the third with X(k) -> i kz X(k) first
+int fft_pass_z_force(mgpu_ctx *ctx, const FFTPlan *plan, float2 *f0, float2 *f1, float2 *f2);
 
 // ---------------------------------------------------------------- fused spectral passes (fused.hip)
 enum { FUSED_GREEN_FORCE = 0, FUSED_GREEN_LAPLACE = 1, FUSED_GREEN_SMOOTH = 2 };
@@ -242,6 +245,8 @@ int fused_green_x(mgpu_ctx *ctx, int mode, const float2 *a, const float2 *b, flo
                   double p1, int filter);
 // inverse y pass: buf <- Y[buf], oy <- Y[i n_y buf]
 int fused_dual_y(mgpu_ctx *ctx, float2 *buf, float2 *oy);
+// fused_dual_y and the inverse y pass of other
+int fused_force_y(mgpu_ctx *ctx, float2 *buf, float2 *oy, float2 *other);
 // forward x pass then times coupling n^2/(n^2 + massterm2)
 int fused_epi_phi_x(mgpu_ctx *ctx, float2 *buf, double coupling, double massterm2);
 // forward x pass of the density r2c, accumulating the binned P(k) power into pk[nbins]

@@ -162,12 +162,19 @@ __global__ __launch_bounds__(kBlock) void k_scale(const float2 *__restrict__ in,
 }
 
 // ------------------------------------------------------------------ gather
-// Sums of 3 per-particle values in a fixed order: each block takes kChunk
-// consecutive particles, each thread kRed of them at stride kBlock (in order),
+// Sums of 3 per-particle values in a fixed order: each block takes kBlock RED
+// consecutive particles, each thread RED of them at stride kBlock (in order),
 // then a shuffle tree per wave and the waves in order.  The partials
 // [block][3] are reduced by k_reduce3, so the means do not depend on launch
-// order or timing.
-constexpr int kRed = 8, kChunk = kBlock * kRed;
+// order or timing.  RED (1, 2, 4 or 8) is the smallest that leaves at most 1024
+// blocks, four per CU: with 8 always, 64^3 particles were 128 blocks of eight
+// particles in sequence per thread on 256 CUs (k_kick_drift 25 us).
+constexpr int kRedBlocks = 1024;
+int red_of(size_t np) {
+  int r = 1;
+  while (r < 8 && cdiv(np, (size_t)kBlock * r) > (unsigned)kRedBlocks) r *= 2;
+  return r;
+}
 
 __device__ __forceinline__ void block_sum3(double s[3], double *__restrict__ partial) {
   __shared__ double red[3][kBlock / 64];
@@ -222,29 +229,31 @@ __global__ __launch_bounds__(kBlock) void k_gather(const float *__restrict__ pos
 }
 
 // sums of Disp for the mean, in particle order (see block_sum3)
+template <int RED>
 __global__ __launch_bounds__(kBlock) void k_sum3(const float *__restrict__ disp, size_t np,
                                                  double *__restrict__ partial, size_t zs) {
   disp = zbuf(disp, zs);
   partial = zbuf(partial, zs);
-  const size_t base = (size_t)blockIdx.x * kChunk + threadIdx.x;
+  const size_t base = (size_t)blockIdx.x * (kBlock * RED) + threadIdx.x;
   double s[3] = {0, 0, 0};
 #pragma unroll
   for (int a = 0; a < 3; a++) {
-    float v[kRed];
+    float v[RED];
 #pragma unroll
-    for (int r = 0; r < kRed; r++) {
+    for (int r = 0; r < RED; r++) {
       const size_t i = base + (size_t)r * kBlock;
       v[r] = i < np ? disp[(size_t)a * np + i] : 0.f;
     }
 #pragma unroll
-    for (int r = 0; r < kRed; r++) s[a] += (double)v[r];
+    for (int r = 0; r < RED; r++) s[a] += (double)v[r];
   }
   block_sum3(s, partial);
 }
 
 // fixed-order reduction of per-block partials [nb][3] -> out[3]
+// (host: pinned memory that takes the sums too, or none)
 __global__ __launch_bounds__(1024) void k_reduce3(const double *__restrict__ partial, int nb, double *__restrict__ out,
-                                                  size_t zs) {
+                                                  double *host, size_t zs) {
   partial = zbuf(partial, zs);
   out = zbuf(out, zs);
   __shared__ double red[3][1024];
@@ -259,7 +268,10 @@ __global__ __launch_bounds__(1024) void k_reduce3(const double *__restrict__ par
     __syncthreads();
   }
   if (threadIdx.x == 0)
-    for (int a = 0; a < 3; a++) out[a] = red[a][0];
+    for (int a = 0; a < 3; a++) {
+      out[a] = red[a][0];
+      if (host) host[a] = red[a][0];
+    }
 }
 
 // ------------------------------------------------------------------ Kick / Drift
@@ -274,17 +286,18 @@ __device__ __forceinline__ double lpt_term(const float *__restrict__ l0, const f
 }
 
 // Kick (src/main.c:688-742)
+template <int RED>
 __global__ __launch_bounds__(kBlock) void k_kick(float *__restrict__ vel, float *__restrict__ disp,
                                                  const float *__restrict__ l0, const float *__restrict__ l1,
                                                  size_t np, double s1, double s2, int sd, double omega, double dda,
                                                  double A, int use_cola, double sD0, double sD1, double sD2,
                                                  double *__restrict__ partial) {
 #pragma clang fp contract(off)  // same rounding sequence as the CPU reference
-  const size_t base = (size_t)blockIdx.x * kChunk + threadIdx.x;
+  const size_t base = (size_t)blockIdx.x * (kBlock * RED) + threadIdx.x;
   double s[3] = {0, 0, 0};
   const double sD[3] = {sD0, sD1, sD2};
 #pragma unroll 2
-  for (int r = 0; r < kRed; r++) {
+  for (int r = 0; r < RED; r++) {
     const size_t i = base + (size_t)r * kBlock;
     if (i >= np) break;
 #pragma unroll
@@ -339,6 +352,7 @@ __global__ __launch_bounds__(kBlock) void k_drift(float *__restrict__ pos, const
 // LPT fields, whose k = 0 mode is zero), so it is the mean after the kick up to
 // rounding.  Disp is not written back (only a second kick at an output step
 // needs Disp - sumD, and that takes the separate passes).
+template <int RED>
 __global__ __launch_bounds__(kBlock) void k_kick_drift(float *__restrict__ vel, float *__restrict__ pos,
                                                        const float *__restrict__ disp, const float *__restrict__ l0,
                                                        const float *__restrict__ l1, size_t np, int sdk, double s1k,
@@ -355,7 +369,7 @@ __global__ __launch_bounds__(kBlock) void k_kick_drift(float *__restrict__ vel, 
   l1 = zbuf(l1, zs);
   dsum = zbuf(dsum, zs);
   partial = zbuf(partial, zs);
-  const size_t base = (size_t)blockIdx.x * kChunk + threadIdx.x;
+  const size_t base = (size_t)blockIdx.x * (kBlock * RED) + threadIdx.x;
   double s[3] = {0, 0, 0};
   double sD[3] = {sD0, sD1, sD2}, sV[3] = {sV0, sV1, sV2};
   if (dsum) {
@@ -368,7 +382,7 @@ __global__ __launch_bounds__(kBlock) void k_kick_drift(float *__restrict__ vel, 
     }
   }
 #pragma unroll 2
-  for (int r = 0; r < kRed; r++) {
+  for (int r = 0; r < RED; r++) {
     const size_t i = base + (size_t)r * kBlock;
     if (i >= np) break;
 #pragma unroll
@@ -392,15 +406,19 @@ __global__ __launch_bounds__(kBlock) void k_kick_drift(float *__restrict__ vel, 
 
 // =================================================================== host side
 
+#define BY_RED(kern, r) ((r) == 1 ? kern<1> : (r) == 2 ? kern<2> : (r) == 4 ? kern<4> : kern<8>)
+
 // the per-block partials reduced into dst (3 doubles on the device: ctx->dsum
-// for Disp, ctx->dsum + 3 for the velocities), and copied to out unless out is
-// nullptr (then nothing waits for the device)
+// for Disp, ctx->dsum + 3 for the velocities), and into out unless out is
+// nullptr (then nothing waits for the device): the kernel writes the context's
+// pinned host sums, so one wait for the stream and no copy brings them back
 int pm_reduce3(mgpu_ctx *ctx, int nblocks, double out[3], double *dst) {
-  hipLaunchKernelGGL(k_reduce3, dim3(1, 1, ctx->bz), dim3(1024), 0, ctx->stream, ctx->partial, nblocks, dst, ctx->zs);
+  hipLaunchKernelGGL(k_reduce3, dim3(1, 1, ctx->bz), dim3(1024), 0, ctx->stream, ctx->partial, nblocks, dst,
+                     out ? ctx->host_sums : nullptr, ctx->zs);
   MGPU_HIP(ctx, hipGetLastError());
   if (!out) return MGPU_OK;
-  MGPU_HIP(ctx, hipMemcpyAsync(out, dst, 3 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
   MGPU_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  std::copy(ctx->host_sums, ctx->host_sums + 3, out);
   return MGPU_OK;
 }
 
@@ -427,17 +445,21 @@ int pofk_setup(mgpu_ctx *ctx, double **dwin) {
 
 // normalisation of the bin sums (src/compute_pofk.c:200-236); with geometry the
 // |n| sums and mode counts come from ctx->pk_geom and only the power from the device
+// (queue starts the copy into the context's pinned buffer; finish, after a wait for the
+// stream, reads it)
+int pofk_queue(mgpu_ctx *ctx, bool geometry_from_ctx) {
+  const size_t n = (geometry_from_ctx ? MGPU_PK_SETS : 3) * (size_t)ctx->p.pofk_nbins;
+  MGPU_HIP(ctx, hipMemcpyAsync(ctx->host_pk, ctx->pk, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+  return MGPU_OK;
+}
 int pofk_finish(mgpu_ctx *ctx, mgpu_pofk *out, bool geometry_from_ctx) {
   const int nbins = ctx->p.pofk_nbins;
-  std::vector<double> h(MGPU_PK_SETS * (size_t)nbins);
-  MGPU_HIP(ctx, hipMemcpyAsync(h.data(), ctx->pk, (geometry_from_ctx ? MGPU_PK_SETS : 3) * (size_t)nbins * sizeof(double),
-                               hipMemcpyDeviceToHost, ctx->stream));
-  MGPU_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  double *h = ctx->host_pk;
   // the x pass adds into MGPU_PK_SETS sets of sums; k_pofk into the first, with the |n| sums and counts behind it
   for (int c = 1; geometry_from_ctx && c < MGPU_PK_SETS; c++)
     for (int b = 0; b < nbins; b++) h[b] += h[(size_t)c * nbins + b];
-  if (geometry_from_ctx) std::copy(ctx->pk_geom.begin(), ctx->pk_geom.end(), h.begin() + nbins);
-  else ctx->pk_geom.assign(h.begin() + nbins, h.begin() + 3 * (size_t)nbins);
+  if (geometry_from_ctx) std::copy(ctx->pk_geom.begin(), ctx->pk_geom.end(), h + nbins);
+  else ctx->pk_geom.assign(h + nbins, h + 3 * (size_t)nbins);
   const double box3 = std::pow(ctx->p.box, 3);
   const double shot = std::pow(ctx->p.box / (double)ctx->Np, 3);
   for (int b = 0; b < nbins; b++) {
@@ -478,6 +500,8 @@ int pm_pofk(mgpu_ctx *ctx, const float2 *dk, mgpu_pofk *out) {
                        ctx->pk);
     MGPU_HIP(ctx, hipGetLastError());
   }
+  if ((rc = pofk_queue(ctx, false))) return rc;
+  MGPU_HIP(ctx, hipStreamSynchronize(ctx->stream));
   return pofk_finish(ctx, out, false);
 }
 
@@ -511,6 +535,8 @@ int pm_transform(mgpu_ctx *ctx, mgpu_pofk *out) {
     if ((rc = fused_pofk_x(ctx, dk, ctx->pk))) return rc;
   }
   PhaseTimer pt(ctx, &ctx->t.pofk);
+  if ((rc = pofk_queue(ctx, true))) return rc;
+  MGPU_HIP(ctx, hipStreamSynchronize(ctx->stream));
   return pofk_finish(ctx, out, true);
 }
 
@@ -605,11 +631,8 @@ int pm_fifth_force(mgpu_ctx *ctx, const mgpu_mg *mg) {
 static int forces_tail(mgpu_ctx *ctx) {
   int rc;
   ctx->have_phik = false;
-  if ((rc = fused_dual_y(ctx, ctx->slot[1], ctx->slot[2]))) return rc;
-  if ((rc = fft_pass_col(ctx, &ctx->fft, ctx->slot[3], 1, 0))) return rc;
-  if ((rc = fft_pass_z(ctx, &ctx->fft, ctx->slot[3], 0, nullptr))) return rc;
-  if ((rc = fft_pass_z(ctx, &ctx->fft, ctx->slot[2], 0, nullptr))) return rc;
-  if ((rc = fft_pass_z_ikz(ctx, &ctx->fft, ctx->slot[1]))) return rc;
+  if ((rc = fused_force_y(ctx, ctx->slot[1], ctx->slot[2], ctx->slot[3]))) return rc;
+  if ((rc = fft_pass_z_force(ctx, &ctx->fft, ctx->slot[3], ctx->slot[2], ctx->slot[1]))) return rc;
   ctx->force_slot[0] = 3;
   ctx->force_slot[1] = 2;
   ctx->force_slot[2] = 1;
@@ -683,11 +706,13 @@ int pm_step_fused(mgpu_ctx *ctx, const mgpu_mg *mg, mgpu_pofk *out, double sumD[
     PhaseTimer pt(ctx, &ctx->t.forces);
     if ((rc = forces_tail(ctx))) return rc;
   }
-  if (out) {
-    PhaseTimer pt(ctx, &ctx->t.pofk);
-    if ((rc = pofk_finish(ctx, out, true))) return rc;
-  }
-  return pm_gather(ctx, sumD);
+  // P(k) comes back with the gather's sums: one wait
+  if (out && (rc = pofk_queue(ctx, true))) return rc;
+  if ((rc = pm_gather(ctx, sumD))) return rc;
+  if (!out) return MGPU_OK;
+  PhaseTimer pt(ctx, &ctx->t.pofk);
+  MGPU_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  return pofk_finish(ctx, out, true);
 }
 
 // Forces (src/auxPM.c:437-555): F_a = c2r(i n_a (-1/n^2) P / (N^3 2pi/Box)), P = delta(k) (+ phi(k)).
@@ -710,7 +735,8 @@ int pm_gather(mgpu_ctx *ctx, double sumD[3]) {
     return MGPU_OK;
   }
   const int N = ctx->N;
-  const unsigned nb = cdiv(ctx->np, kChunk);
+  const int red = red_of(ctx->np);
+  const unsigned nb = cdiv(ctx->np, (size_t)kBlock * red);
   const float *f0 = (const float *)ctx->slot[ctx->force_slot[0]], *f1 = (const float *)ctx->slot[ctx->force_slot[1]],
               *f2 = (const float *)ctx->slot[ctx->force_slot[2]];
   // compulsory: positions and Disp (12 B each per particle) and the three force meshes once
@@ -731,7 +757,7 @@ int pm_gather(mgpu_ctx *ctx, double sumD[3]) {
   MGPU_HIP(ctx, hipGetLastError());
   {
     KScope ks(ctx, MGPU_K_MEAN, 12.0 * ctx->np);
-    hipLaunchKernelGGL(k_sum3, dim3(nb, 1, ctx->bz), dim3(kBlock), 0, ctx->stream, ctx->disp, ctx->np, ctx->partial,
+    hipLaunchKernelGGL(BY_RED(k_sum3, red), dim3(nb, 1, ctx->bz), dim3(kBlock), 0, ctx->stream, ctx->disp, ctx->np, ctx->partial,
                        ctx->zs);
   }
   MGPU_HIP(ctx, hipGetLastError());
@@ -748,12 +774,13 @@ int pm_kick(mgpu_ctx *ctx, double dda, double A, double s1, double s2, const dou
     sumV[0] = sumV[1] = sumV[2] = 0;
     return MGPU_OK;
   }
-  const unsigned nb = cdiv(ctx->np, kChunk);
+  const int red = red_of(ctx->np);
+  const unsigned nb = cdiv(ctx->np, (size_t)kBlock * red);
   const int sd = ctx->p.scale_dependent ? 1 : 0;
   {
     // vel, Disp read + written, one (scale-dependent) or two LPT vectors read
     KScope ks(ctx, MGPU_K_KICK, (48.0 + (sd ? 12.0 : 24.0)) * ctx->np);
-    hipLaunchKernelGGL(k_kick, dim3(nb), dim3(kBlock), 0, ctx->stream, ctx->vel, ctx->disp, ctx->lpt[0], ctx->lpt[1],
+    hipLaunchKernelGGL(BY_RED(k_kick, red), dim3(nb), dim3(kBlock), 0, ctx->stream, ctx->vel, ctx->disp, ctx->lpt[0], ctx->lpt[1],
                        ctx->np, s1, s2, sd, ctx->p.omega, dda, A, ctx->p.use_cola, sumD[0], sumD[1], sumD[2],
                        ctx->partial);
   }
@@ -795,12 +822,13 @@ int pm_kick_drift(mgpu_ctx *ctx, double dda, double A, double s1k, double s2k, c
   }
   const double z3[3] = {0.0, 0.0, 0.0};
   const double *hD = dev ? z3 : sumD, *hV = dev ? z3 : sumV;
-  const unsigned nb = cdiv(ctx->np, kChunk);
+  const int red = red_of(ctx->np);
+  const unsigned nb = cdiv(ctx->np, (size_t)kBlock * red);
   const bool sdep = ctx->p.scale_dependent;
   {
     // vel, pos read + written, Disp and the LPT vectors read
     KScope ks(ctx, MGPU_K_KICK, 84.0 * ctx->np);
-    hipLaunchKernelGGL(k_kick_drift, dim3(nb, 1, ctx->bz), dim3(kBlock), 0, ctx->stream, ctx->vel, ctx->pos,
+    hipLaunchKernelGGL(BY_RED(k_kick_drift, red), dim3(nb, 1, ctx->bz), dim3(kBlock), 0, ctx->stream, ctx->vel, ctx->pos,
                        (const float *)ctx->disp, (const float *)ctx->lpt[0], (const float *)ctx->lpt[1], ctx->np,
                        sdep ? 1 : 0, s1k, s2k, sdep ? 2 : 0, s1d, s2d, ctx->p.omega, dda, A, dyyy,
                        (float)ctx->p.box, ctx->p.use_cola, hD[0], hD[1], hD[2], hV[0], hV[1], hV[2],
@@ -851,8 +879,9 @@ int pm_rsd_pofk(mgpu_ctx *ctx, int axis, double vnorm, double s1, double s2, mgp
                        dk, N, ctx->HP, ctx->winv, ctx->pk_bin, ctx->pk_fn, nbins, ctx->pk);
   }
   MGPU_HIP(ctx, hipGetLastError());
-  std::vector<double> h(4 * (size_t)nbins);
-  MGPU_HIP(ctx, hipMemcpyAsync(h.data(), ctx->pk, h.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+  const double *h = ctx->host_pk;
+  MGPU_HIP(ctx, hipMemcpyAsync(ctx->host_pk, ctx->pk, 4 * (size_t)nbins * sizeof(double), hipMemcpyDeviceToHost,
+                               ctx->stream));
   MGPU_HIP(ctx, hipStreamSynchronize(ctx->stream));
   const double box3 = std::pow(ctx->p.box, 3), shot = std::pow(ctx->p.box / (double)ctx->Np, 3);
   const double kmin = ctx->p.pofk_kmin, kmax = ctx->p.pofk_kmax;
