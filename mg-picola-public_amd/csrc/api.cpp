@@ -638,8 +638,8 @@ int mgpu_get_fft_tile(mgpu_ctx *ctx, int which, int *tcols) {
 int mgpu_autotune_fft(mgpu_ctx *ctx, double ms[4]) {
   if (check_ctx(ctx) || !ms) return MGPU_E_INVALID;
   ms[0] = ms[1] = ms[2] = ms[3] = -1.0;
-  int rc = fft_autotune(ctx, &ctx->fft, ctx->slot[3], ms);
-  if (!rc && ctx->fft_lattice.n > 0 && ctx->lattice_slot) rc = fft_autotune(ctx, &ctx->fft_lattice, ctx->lattice_slot, ms + 2);
+  int rc = fft_autotune(ctx, &ctx->fft, ctx->slot[3], true, ms);
+  if (!rc && ctx->fft_lattice.n > 0 && ctx->lattice_slot) rc = fft_autotune(ctx, &ctx->fft_lattice, ctx->lattice_slot, false, ms + 2);
   return rc;
 }
 

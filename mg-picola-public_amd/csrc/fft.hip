@@ -117,8 +117,8 @@ __device__ __forceinline__ void z_c2r_rows(const float2 *buf, int HP, size_t nro
 template <int N>
 __global__ __launch_bounds__(RowCfg<N>::NT) void k_fft_z_c2r(const float2 *buf, int HP, size_t nrows,
                                                               const float2 *__restrict__ tw, float2 *out, int orow,
-                                                              size_t zs) {
-  z_c2r_rows<N>(zbuf(buf, zs), HP, nrows, tw, zbuf(out, zs), orow, false);
+                                                              size_t zs, size_t ozs) {
+  z_c2r_rows<N>(zbuf(buf, zs), HP, nrows, tw, zbuf(out, ozs), orow, false);
 }
 // The three force components in one launch (grid y = component; the z component with
 // i k): one mesh after the other in the order of the blocks, as three launches would
@@ -154,7 +154,7 @@ int launch_col(mgpu_ctx *ctx, float2 *buf, size_t line_stride, size_t outer_stri
 
 template <int N>
 int launch_z(mgpu_ctx *ctx, float2 *buf, int HP, const float2 *tw, int forward, float2 *out = nullptr,
-             const float2 *in = nullptr) {
+             const float2 *in = nullptr, size_t ozs = 0) {
   using C = RowCfg<N>;
   size_t nrows = (size_t)N * N;
   size_t lds = (size_t)C::RB * C::LS * sizeof(float2);
@@ -168,7 +168,7 @@ int launch_z(mgpu_ctx *ctx, float2 *buf, int HP, const float2 *tw, int forward, 
     auto kern = k_fft_z_c2r<N>;
     if (lds > 65536) MGPU_HIP(ctx, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(kern, grid, dim3(C::NT), lds, ctx->stream, (const float2 *)buf, HP, nrows, tw,
-                       out ? out : buf, out ? N / 2 : HP, ctx->zs);
+                       out ? out : buf, out ? N / 2 : HP, ctx->zs, ozs ? ozs : ctx->zs);
   }
   MGPU_HIP(ctx, hipGetLastError());
   return MGPU_OK;
@@ -225,11 +225,15 @@ int fft_plan_init(mgpu_ctx *ctx, FFTPlan *plan, int n, int tcols) {
   return MGPU_OK;
 }
 
-// The column passes' tile width measured on this device: the forward and the
-// inverse y pass over buf (a scratch mesh of the plan's size) with each width
-// that fits, one warm-up and the best of three; the faster becomes
-// plan->tcols.  The width changes no column's arithmetic, only the schedule.
-int fft_autotune(mgpu_ctx *ctx, FFTPlan *plan, float2 *buf, double ms[2]) {
+// The column passes' tile width measured on this device: a forward and an
+// inverse y pass, a forward x pass and (force: the Nmesh plan) the y passes of
+// the force tail, over buf (a scratch mesh of the plan's size) and the force
+// slots, with each width that fits, one warm-up and the best of three; the
+// faster becomes plan->tcols.  The width changes no column's arithmetic, only
+// the schedule.  The y pair alone does not tell the widths apart at 1024 (3.51
+// against 3.47 ms for 8 and 16), where the dual pass takes 3.18 against 2.75 ms
+// and the density pair with P(k) 6.0 against 4.1 ms.
+int fft_autotune(mgpu_ctx *ctx, FFTPlan *plan, float2 *buf, bool force, double ms[2]) {
   const bool can16 = fft_tile16_fits(ctx, plan->n);
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
@@ -246,6 +250,8 @@ int fft_autotune(mgpu_ctx *ctx, FFTPlan *plan, float2 *buf, double ms[2]) {
       if (hipEventRecord(e0, ctx->stream) != hipSuccess) rc = MGPU_E_HIP;
       if (!rc) rc = fft_pass_col(ctx, plan, buf, 1, 1);
       if (!rc) rc = fft_pass_col(ctx, plan, buf, 1, 0);
+      if (!rc) rc = fft_pass_col(ctx, plan, buf, 0, 1);
+      if (!rc && force) rc = fused_force_y(ctx, ctx->slot[1], ctx->slot[2], ctx->slot[3]);
       float t = 0.f;
       if (!rc && (hipEventRecord(e1, ctx->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
                   hipEventElapsedTime(&t, e0, e1) != hipSuccess))
@@ -265,15 +271,15 @@ void fft_plan_free(FFTPlan *plan) {
   plan->tw = nullptr;
 }
 
-int fft_pass_z(mgpu_ctx *ctx, const FFTPlan *plan, float2 *buf, int forward, float *out, const float *in) {
+int fft_pass_z(mgpu_ctx *ctx, const FFTPlan *plan, float2 *buf, int forward, float *out, const float *in, size_t ozs) {
   // compulsory traffic: N^2 rows of N reals one way and N/2+1 complex the other
   const double rows = (double)plan->n * plan->n;
   const int cat = plan->kcat >= 0 ? plan->kcat : (forward ? MGPU_K_FFT_R2C : MGPU_K_FFT_C2R);
-  KScope ks(ctx, cat, rows * (plan->n * 4.0 + (plan->n / 2 + 1) * 8.0));
+  KScope ks(ctx, cat, ctx->bz * rows * (plan->n * 4.0 + (plan->n / 2 + 1) * 8.0));
   switch (plan->n) {
 #define X(S) \
   case S:    \
-    return launch_z<S>(ctx, buf, plan->hp, plan->tw, forward, (float2 *)out, (const float2 *)in);
+    return launch_z<S>(ctx, buf, plan->hp, plan->tw, forward, (float2 *)out, (const float2 *)in, ozs);
     MGPU_FFT_SIZES(X)
 #undef X
     default:
@@ -288,7 +294,7 @@ int fft_pass_col(mgpu_ctx *ctx, const FFTPlan *plan, float2 *buf, int axis, int 
   const size_t os = axis == 1 ? N * HP : HP;
   // compulsory traffic: read + write of the N*N*(N/2+1) half spectrum
   const int cat = plan->kcat >= 0 ? plan->kcat : (forward ? MGPU_K_FFT_COL_FWD : MGPU_K_FFT_COL_INV);
-  KScope ks(ctx, cat, 2.0 * 8.0 * (double)N * N * (N / 2 + 1));
+  KScope ks(ctx, cat, ctx->bz * 2.0 * 8.0 * (double)N * N * (N / 2 + 1));
   switch (plan->n) {
 #define X(S) \
   case S:    \
@@ -337,4 +343,27 @@ int fft_c2r_3d(mgpu_ctx *ctx, const FFTPlan *plan, float2 *buf, float *out) {
   if ((rc = fft_pass_col(ctx, plan, buf, 0, 0))) return rc;
   if ((rc = fft_pass_col(ctx, plan, buf, 1, 0))) return rc;
   return fft_pass_z(ctx, plan, buf, 0, out);
+}
+
+// The launches of one pass over several fields are one launch with grid z = field, the
+// way a batch's realizations are: the fields lie nl elements apart in buf, field
+// (s, a)'s result goes to out[s] + a np.  Six 128 lattice fields take 18 launches of
+// 7 us otherwise.
+int fft_c2r_fields(mgpu_ctx *ctx, const FFTPlan *plan, float2 *buf, size_t nl, int ns, float *const out[2], size_t np) {
+  if (ctx->bz != 1) return mgpu_fail(ctx, MGPU_E_STATE, "lattice fields of a batched launch");
+  PhaseTimer pt(ctx, &ctx->t.fft);
+  struct Restore {
+    mgpu_ctx *c;
+    size_t zs;
+    ~Restore() { c->bz = 1, c->zs = zs; }
+  } restore{ctx, ctx->zs};
+  int rc;
+  ctx->zs = nl * sizeof(float2);
+  ctx->bz = 3u * (unsigned)ns;
+  if ((rc = fft_pass_col(ctx, plan, buf, 0, 0))) return rc;
+  if ((rc = fft_pass_col(ctx, plan, buf, 1, 0))) return rc;
+  ctx->bz = 3;
+  for (int s = 0; s < ns; s++)
+    if ((rc = fft_pass_z(ctx, plan, buf + 3 * s * nl, 0, out[s], nullptr, np * sizeof(float)))) return rc;
+  return MGPU_OK;
 }

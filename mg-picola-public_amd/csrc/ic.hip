@@ -438,25 +438,30 @@ __global__ __launch_bounds__(kBlock) void k_lpt_fold(const float2 *__restrict__ 
 }
 
 // growth from the shared-grid ln k slices of NS slots (node-major float4s,
-// copied once per block into LDS).  The blocks stride over the Nsample^2 rows;
-// the interior kz of a row first, then the kz = 0 and Nsample/2 modes of all
-// rows.  Output spectrum (slot s, component a) at out + (3 s + a) nl.
+// copied once per block into LDS).  The blocks stride over the Nsample^2 rows, lpw
+// (a power of two) lanes to a row and kFoldNT/lpw rows at a time; the interior kz of
+// the rows first, then the kz = 0 and Nsample/2 modes of all rows.  Output spectrum
+// (slot s, component a) at out + (3 s + a) nl.
+// What bounds it: the slices of 1000 nodes take 48 KB, so blocks of 256 threads left
+// three waves per SIMD, and a row of a 128 lattice 63 of the 256 lanes.
+constexpr int kFoldNT = 512;
+constexpr unsigned kFoldRounds = 2;
 template <int MF, int NS>
-__global__ __launch_bounds__(kBlock) void k_lpt_fold_gs(const float2 *__restrict__ cd1,
-                                                        const float2 *__restrict__ cd2,
-                                                        const float4 *__restrict__ nodes, GShared<NS> gs,
-                                                        float lnkf, int N, int HP, int Np, int HPn, int m_rt,
-                                                        float ikf, float2 *__restrict__ out, size_t nl) {
+__global__ __launch_bounds__(kFoldNT, 4) void k_lpt_fold_gs(const float2 *__restrict__ cd1,
+                                                            const float2 *__restrict__ cd2,
+                                                            const float4 *__restrict__ nodes, GShared<NS> gs,
+                                                            float lnkf, int N, int HP, int Np, int HPn, int m_rt,
+                                                            float ikf, int lpw, float2 *__restrict__ out, size_t nl) {
   extern __shared__ float4 sl[];
   const int nn = gs.ny * (1 + NS);
-  for (int e = threadIdx.x; e < nn; e += blockDim.x) sl[e] = nodes[e];
+  for (int e = threadIdx.x; e < nn; e += kFoldNT) sl[e] = nodes[e];
   __syncthreads();
   gs.sl = sl;
-  const unsigned rows = (unsigned)Np * (unsigned)Np;
-  const int H = Np / 2;
-  for (unsigned row = blockIdx.x; row < rows; row += gridDim.x) {
+  const unsigned rows = (unsigned)Np * (unsigned)Np, rpb = kFoldNT / lpw;
+  const int H = Np / 2, l0 = (int)threadIdx.x & (lpw - 1);
+  for (unsigned row = blockIdx.x * rpb + threadIdx.x / lpw; row < rows; row += gridDim.x * rpb) {
     const int jp = (int)(row % (unsigned)Np), ip = (int)(row / (unsigned)Np);
-    for (int lp = 1 + (int)threadIdx.x; lp < H; lp += blockDim.x) {
+    for (int lp = l0 ? l0 : lpw; lp < H; lp += lpw) {
       float acc[NS][6];
       fold_mode<MF, NS, GShared<NS>, false>(ip, jp, lp, N, HP, Np, m_rt, ikf, lnkf, cd1, cd2, gs, acc);
       const size_t o = (size_t)row * HPn + lp;
@@ -466,7 +471,7 @@ __global__ __launch_bounds__(kBlock) void k_lpt_fold_gs(const float2 *__restrict
         for (int a = 0; a < 3; a++) out[(3 * s + a) * nl + o] = make_float2(acc[s][2 * a], acc[s][2 * a + 1]);
     }
   }
-  for (unsigned q = blockIdx.x * blockDim.x + threadIdx.x; q < 2 * rows; q += gridDim.x * blockDim.x) {
+  for (unsigned q = blockIdx.x * kFoldNT + threadIdx.x; q < 2 * rows; q += gridDim.x * kFoldNT) {
     const unsigned row = q >> 1;
     const int lp = (q & 1) ? H : 0;
     const int jp = (int)(row % (unsigned)Np), ip = (int)(row / (unsigned)Np);
@@ -776,10 +781,14 @@ int launch_fold_gs(mgpu_ctx *ctx, const SliceFold &f, float lnkf, float ikf, flo
   gs.ny = f.ny;
   const int Np = ctx->Np;
   const size_t lds = sizeof(float4) * (size_t)f.ny * (1 + NS);
-  const unsigned nb = (unsigned)std::min<size_t>((size_t)Np * Np, 2048);
-  hipLaunchKernelGGL((k_lpt_fold_gs<MF, NS>), dim3(nb), dim3(kBlock), lds, ctx->stream, ctx->cdelta[0],
+  int lpw = 16;
+  while (lpw < Np / 2 && lpw < kFoldNT) lpw *= 2;
+  // as many blocks as the LDS and the registers keep resident, each copying the slices once
+  const unsigned per_cu = (unsigned)std::max<size_t>(1, std::min<size_t>(2, ctx->lds_max / std::max<size_t>(lds, 1)));
+  const unsigned nb = (unsigned)std::min<size_t>(cdiv((size_t)Np * Np, kFoldNT / lpw), 256 * per_cu * kFoldRounds);
+  hipLaunchKernelGGL((k_lpt_fold_gs<MF, NS>), dim3(nb), dim3(kFoldNT), lds, ctx->stream, ctx->cdelta[0],
                      ctx->cdelta[1], (const float4 *)ctx->slice_buf, gs, lnkf, ctx->N, ctx->HP, Np,
-                     ctx->fft_lattice.hp, ctx->N / Np, ikf, out, nl);
+                     ctx->fft_lattice.hp, ctx->N / Np, ikf, lpw, out, nl);
   MGPU_HIP(ctx, hipGetLastError());
   return MGPU_OK;
 }
@@ -818,12 +827,9 @@ static int lattice_fields(mgpu_ctx *ctx, int ns, const int *slots, const SliceFo
       if (rc) return rc;
     }
     MGPU_HIP(ctx, hipGetLastError());
-    for (int s = 0; s < ns; s++)
-      for (int a = 0; a < 3; a++)
-        if ((rc = fft_c2r_3d(ctx, &ctx->fft_lattice, ctx->lattice_slot + (3 * s + a) * nl,
-                             ctx->lpt[slots[s]] + (size_t)a * ctx->np)))
-          return rc;
-    return MGPU_OK;
+    // the 3 ns fields' transforms, one launch per pass (the z pass one per slot)
+    float *out[2] = {ctx->lpt[slots[0]], ns > 1 ? ctx->lpt[slots[1]] : nullptr};
+    return fft_c2r_fields(ctx, &ctx->fft_lattice, ctx->lattice_slot, nl, ns, out, ctx->np);
   }
   if (ns != 1) return mgpu_fail(ctx, MGPU_E_INVALID, "several LPT slots at once need the lattice fold");
   for (int a = 0; a < 3; a++) {

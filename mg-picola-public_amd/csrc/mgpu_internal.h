@@ -220,7 +220,7 @@ size_t fft_col_lds(int n, int T);
 static inline size_t pofk_lds(int n, int nbins, int copies) {
   return copies * sizeof(double) * (size_t)nbins + sizeof(float) * (size_t)(n / 2 + 1) + sizeof(int) * (size_t)(nbins + 1);
 }
-int fft_autotune(mgpu_ctx *ctx, FFTPlan *plan, float2 *buf, double ms[2]);
+int fft_autotune(mgpu_ctx *ctx, FFTPlan *plan, float2 *buf, bool force, double ms[2]);
 bool fft_size_supported(int n);
 // in-place 3D transforms on a slot with the padded layout above
 // in != nullptr: the real input is read from in (same padded layout) and buf only written
@@ -228,8 +228,11 @@ int fft_r2c_3d(mgpu_ctx *ctx, const FFTPlan *plan, float2 *buf, const float *in 
 // c2r; with out != nullptr the real result goes to a compact [N][N][N] array
 int fft_c2r_3d(mgpu_ctx *ctx, const FFTPlan *plan, float2 *buf, float *out = nullptr);
 // individual passes (used by fused paths and tests)
+// (ozs: byte stride of out between the launch's grid z, where it is not buf's)
 int fft_pass_z(mgpu_ctx *ctx, const FFTPlan *plan, float2 *buf, int forward, float *out = nullptr,
-               const float *in = nullptr);
+               const float *in = nullptr, size_t ozs = 0);
+// c2r of the fields (s, a), s < ns, a < 3, at buf + (3 s + a) nl, to out[s] + a np
+int fft_c2r_fields(mgpu_ctx *ctx, const FFTPlan *plan, float2 *buf, size_t nl, int ns, float *const out[2], size_t np);
 int fft_pass_col(mgpu_ctx *ctx, const FFTPlan *plan, float2 *buf, int axis, int forward);
 
 // z c2r of the three force components in place, of the third with X(k) -> i kz X(k) first

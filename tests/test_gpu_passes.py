@@ -70,3 +70,59 @@ def test_pofk_bins_by_edges(nbins, bintype, kmin, kmax):
         # one lost or misplaced mode changes a sparse bin by its share of the power
         np.testing.assert_allclose(pk[ok], rp[ok], rtol=1e-3)
     g.close()
+
+
+@pytest.mark.parametrize("ns,n", [(1, 8), (7, 16), (64, 96), (65, 96), (81, 96), (102, 128), (40, 384)])
+def test_means_and_bins_over_particle_counts(ns, n):
+    """The means for every number of particles per thread (up to 1024 blocks: 64^3, 65^3,
+    81^3 and 102^3 take 1, 2, 4 and 8) against the particles' own FP64 means, and two
+    deposits in a row, with a redshift-space one between, to the bit: the bin scan (one
+    launch up to the 256 mesh, two beyond) leaves its counters cleared."""
+    pos = lattice_particles(ns, BOX, amp=1.5, seed=ns, clustered=ns > 4)
+    rng = np.random.default_rng(ns)
+    vel = rng.normal(size=pos.shape).astype(np.float32)
+    g = M.MGPU(n, ns, BOX, OM)
+    g.set_particles(pos, vel)
+    g.pm_deposit()
+    first = g.get_mesh(M.MESH_DENSITY_X)
+    g.rsd_power_spectrum(2, 0.1)
+    g.pm_deposit()
+    assert np.array_equal(first, g.get_mesh(M.MESH_DENSITY_X))
+    sum_d, _ = g.get_displacements()
+    d = g.get_disp().astype(np.float64)
+    scale = np.abs(d).max() + 1e-30
+    # FP64 sums of np FP32 values in another order
+    assert np.abs(sum_d - d.mean(1)).max() < 1e-12 * scale
+    sum_v = g.kick(0.3, 0.7, 0.1, 0.2, sum_d)
+    v = g.get_particles()[1].astype(np.float64)
+    assert np.abs(sum_v - v.mean(1)).max() < 1e-12 * np.abs(v).max()
+    g.close()
+
+
+@pytest.mark.parametrize("n,ns", [(8, 8), (16, 8), (32, 32), (48, 24), (96, 48), (96, 32), (128, 32), (128, 128)])
+def test_two_slot_fold_with_constant_growth(n, ns):
+    """Both LPT slots by the ln k slices against the per-|n|^2 tables, one slot at a time,
+    with a growth that does not depend on k (so the slices are exact): the fold's lanes per
+    row from 16 up, m = 1, 2, 3 and 4.  The slices form 1/den with a 1-ulp reciprocal and
+    the sums of up to 2 m^3 aliases round in another order: 4e-6 of the field maximum."""
+    import ctypes as C
+
+    g = M.MGPU(n, ns, BOX, OM, scale_dependent=1)
+    pk = 100.0 / (1.0 + np.arange(M.n2_table_len(n), dtype=np.float64))
+    g.ic_displacement_fields(11, pk)
+    nk, keep = 50, []
+
+    def kslice(value, den, norm):
+        a = [np.full(nk, value), np.zeros(nk), np.full(nk, den), np.zeros(nk)]
+        keep.append(a)
+        return M.KSlice(-6.0, 0.25, nk, *[x.ctypes.data_as(C.POINTER(C.c_double)) for x in a], norm)
+
+    norm2 = -3.0 / 7.0 / n ** 3
+    grow = [(0.8, 0.5), (0.3, 0.2)]
+    M.lpt_fields_slices2(g, *[(kslice(2 * a, 2.0, 1.0), kslice(4 * b, 4.0, norm2)) for a, b in grow])
+    got = [g.get_lpt(s) for s in (0, 1)]
+    ones = np.ones(M.n2_table_len(n))
+    for s, (a, b) in enumerate(grow):
+        g.lpt_fields(s, a * ones, norm2 * b * ones)
+        assert rel_err(got[s], g.get_lpt(s)) < 4e-6
+    g.close()
