@@ -364,8 +364,8 @@ int mgpu_density_feature(mgpu_ctx *ctx, double *s); /* s of the last deposit */
  * transforms of the scale-dependent LPT fields. */
 int mgpu_set_fft_tile(mgpu_ctx *ctx, int which, int tcols); /* 16 only where the tile fits a workgroup */
 int mgpu_get_fft_tile(mgpu_ctx *ctx, int which, int *tcols);
-/* Measure both widths on this device (a forward and an inverse y pass, an x pass
- * and, for the Nmesh transforms, the y passes of the force; best of three) and
+/* Measure both widths on this device (a forward x pass and the y passes of the
+ * force, or an inverse y pass of the lattice transforms; the better of two) and
  * keep the faster, for both plans.  It uses the force meshes and the
  * lattice spectra as scratch: call it before the initial conditions.
  * ms: 4 doubles (main 8, main 16, lattice 8, lattice 16; -1 where not run). */

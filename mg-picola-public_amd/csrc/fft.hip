@@ -225,14 +225,13 @@ int fft_plan_init(mgpu_ctx *ctx, FFTPlan *plan, int n, int tcols) {
   return MGPU_OK;
 }
 
-// The column passes' tile width measured on this device: a forward and an
-// inverse y pass, a forward x pass and (force: the Nmesh plan) the y passes of
-// the force tail, over buf (a scratch mesh of the plan's size) and the force
-// slots, with each width that fits, one warm-up and the best of three; the
-// faster becomes plan->tcols.  The width changes no column's arithmetic, only
-// the schedule.  The y pair alone does not tell the widths apart at 1024 (3.51
-// against 3.47 ms for 8 and 16), where the dual pass takes 3.18 against 2.75 ms
-// and the density pair with P(k) 6.0 against 4.1 ms.
+// The column passes' tile width measured on this device: a forward x pass, and the y
+// passes of the force tail over the force slots (force: the Nmesh plan) or an inverse
+// y pass over buf (a scratch mesh of the plan's size), with each width that fits, one
+// warm-up and the better of two; the faster becomes plan->tcols.  The width changes no
+// column's arithmetic, only the schedule.  The y passes alone do not tell the widths
+// apart at 1024 (3.51 against 3.47 ms a pair for 8 and 16), where the dual pass takes
+// 3.18 against 2.75 ms and the density pair with P(k) 6.0 against 4.1 ms.
 int fft_autotune(mgpu_ctx *ctx, FFTPlan *plan, float2 *buf, bool force, double ms[2]) {
   const bool can16 = fft_tile16_fits(ctx, plan->n);
   hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -246,12 +245,10 @@ int fft_autotune(mgpu_ctx *ctx, FFTPlan *plan, float2 *buf, bool force, double m
     ms[w] = -1.0;
     if (widths[w] == 16 && !can16) continue;
     plan->tcols = widths[w];
-    for (int rep = 0; rep < 4 && !rc; rep++) {
+    for (int rep = 0; rep < 3 && !rc; rep++) {
       if (hipEventRecord(e0, ctx->stream) != hipSuccess) rc = MGPU_E_HIP;
-      if (!rc) rc = fft_pass_col(ctx, plan, buf, 1, 1);
-      if (!rc) rc = fft_pass_col(ctx, plan, buf, 1, 0);
       if (!rc) rc = fft_pass_col(ctx, plan, buf, 0, 1);
-      if (!rc && force) rc = fused_force_y(ctx, ctx->slot[1], ctx->slot[2], ctx->slot[3]);
+      if (!rc) rc = force ? fused_force_y(ctx, ctx->slot[1], ctx->slot[2], ctx->slot[3]) : fft_pass_col(ctx, plan, buf, 1, 0);
       float t = 0.f;
       if (!rc && (hipEventRecord(e1, ctx->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
                   hipEventElapsedTime(&t, e0, e1) != hipSuccess))

@@ -11,6 +11,7 @@
 //                      mean removal (src/2LPT.c:1493-1508, 1713-1729).
 #include "mgpu_internal.h"
 #include "ranlux.h"
+#include "ranlux_jump.h"
 
 #include <algorithm>
 #include <cmath>
@@ -31,15 +32,54 @@ constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 unsigned *g_scratch_ptr[kMaxDevices] = {};
 
+// Seed table (src/2LPT.c:259-271): the N^2 values of one RANLUX stream, in the
+// reference's order of shells.  Shell i holds 4 (2 i + 1) values from draw 4 i^2 on:
+// for each of four sign quadrants i values along one axis and i + 1 along the other.
+// Thread t generates the draws [12 adv t, 12 adv (t + 1)) from its own state of the
+// stream, which the host jumped ahead to (state q of thread t at st[q n + t], the
+// carry as the 13th).  The stream itself is one serial chain of 17 dependent steps per
+// draw: the host took 10.5 ms for the table of a 384 mesh, the chunks take 0.3 ms
+// there and 60 us here.
+// With flag, st[13 n] (a realization's inversion) goes behind the table.
+__global__ __launch_bounds__(64) void k_seed_table(const double *__restrict__ st, unsigned n, unsigned adv, int N,
+                                                   int flag, unsigned *__restrict__ table, size_t zs) {
+  st = zbuf(st, zs);
+  table = zbuf(table, zs);
+  const unsigned t = blockIdx.x * 64 + threadIdx.x;
+  if (t >= n) return;
+  Ranlxd1 r;
+#pragma unroll
+  for (int q = 0; q < 12; q++) r.y[q] = st[(size_t)q * n + t];
+  r.carry = st[(size_t)12 * n + t];
+  const unsigned total = (unsigned)N * (unsigned)N;
+  if (flag && t == 0) table[total] = (unsigned)st[(size_t)13 * n];
+  unsigned d = 12 * adv * t;
+  for (unsigned a = 0; a < adv && d < total; a++) {
+    r.advance();
+#pragma unroll
+    for (int q = 0; q < 12; q++, d++) {
+      if (d >= total) break;
+      unsigned i = (unsigned)(0.5f * sqrtf((float)d));  // the shell: 4 i^2 <= d < 4 (i + 1)^2
+      while (4 * i * i > d) i--;
+      while (4 * (i + 1) * (i + 1) <= d) i++;
+      const unsigned e = d - 4 * i * i, g = e / (2 * i + 1), k = e % (2 * i + 1);
+      unsigned x = k < i ? i : k - i, y = k < i ? k : i;
+      if (g & 1) x = (unsigned)N - 1 - x;
+      if (g & 2) y = (unsigned)N - 1 - y;
+      table[(size_t)x * N + y] = (unsigned)(0x7fffffff * r.y[q]);
+    }
+  }
+}
+
 // one thread per column (i, j) of the N x N grid
 __global__ __launch_bounds__(kBlock) void k_ic_delta(const unsigned *__restrict__ seedtable, int N, int Np, int HP,
                                                      double box, int sphere_mode, int amp_fixed, int inverted,
                                                      const double *__restrict__ pk_n2, float2 *__restrict__ cd,
-                                                     size_t zs, size_t seed_stride, const int *__restrict__ inv_z) {
+                                                     size_t zs, const int *__restrict__ inv_z) {
   // a batch: realization blockIdx.z's seed table and inversion flag
   cd = zbuf(cd, zs);
-  seedtable += (size_t)blockIdx.z * seed_stride;
-  if (inv_z) inverted = inv_z[blockIdx.z];
+  seedtable = zbuf(seedtable, zs);
+  if (inv_z) inverted = *zbuf(inv_z, zs);
   const int col = blockIdx.x * blockDim.x + threadIdx.x;
   if (col >= N * N) return;
   const int i = col / N, j = col % N;
@@ -558,22 +598,38 @@ __global__ __launch_bounds__(kBlock) void k_nu_add(float2 *__restrict__ dk, cons
   dk[e] = make_float2((float)(cdmfac * (double)v.x + f * (double)c.x), (float)(cdmfac * (double)v.y + f * (double)c.y));
 }
 
-// seed table on the host (a single serial stream), src/2LPT.c:259-271
-void seedtable_host(int N, unsigned long seed, std::vector<unsigned> &t) {
-  Ranlxd1 r;
-  r.seed(seed);
-  t.assign((size_t)N * N, 0u);
-  auto draw = [&]() { return (unsigned)(0x7fffffff * r.uniform()); };
-  for (int i = 0; i < N / 2; i++) {
-    for (int j = 0; j < i; j++) t[i * N + j] = draw();
-    for (int j = 0; j < i + 1; j++) t[j * N + i] = draw();
-    for (int j = 0; j < i; j++) t[(N - 1 - i) * N + j] = draw();
-    for (int j = 0; j < i + 1; j++) t[(N - 1 - j) * N + i] = draw();
-    for (int j = 0; j < i; j++) t[i * N + (N - 1 - j)] = draw();
-    for (int j = 0; j < i + 1; j++) t[j * N + (N - 1 - i)] = draw();
-    for (int j = 0; j < i; j++) t[(N - 1 - i) * N + (N - 1 - j)] = draw();
-    for (int j = 0; j < i + 1; j++) t[(N - 1 - j) * N + (N - 1 - i)] = draw();
+// The seed tables of count realizations (ctx's, at the batch stride) into table (on the
+// device): the states the chunks of each stream start from go to slot 1, which the
+// initial conditions overwrite afterwards.  A chunk is 16 advances of 12 values, or
+// what makes 2048 chunks: the host's jump takes 0.35 us, a thread's advance 3.4 us.
+// inverted (or nullptr): the realizations' inversion flags, one behind each table.
+int seed_tables(mgpu_ctx *ctx, int count, const unsigned long *seeds, const int *inverted, unsigned *table,
+                std::vector<double> &st) {
+  const int N = ctx->N;
+  const unsigned advances = cdiv((size_t)N * N, 12), adv = std::max(16u, cdiv(advances, 2048)), n = cdiv(advances, adv);
+  const size_t len = 13 * (size_t)n + 1;
+  if (len * sizeof(double) > ctx->slot_elems * sizeof(float2))
+    return mgpu_fail(ctx, MGPU_E_INVALID, "seed states do not fit a mesh slot");
+  const rlx::Num jump = rlx::step_power(202ull * adv);
+  st.resize(len * count);
+  for (int r = 0; r < count; r++) {
+    double *o = st.data() + len * r;
+    Ranlxd1 g;
+    g.seed(seeds[r]);
+    rlx::Num X = rlx::from_state(g);
+    for (unsigned t = 0; t < n; t++) {
+      for (int q = 0; q < 12; q++) o[(size_t)q * n + t] = g.y[q];
+      o[(size_t)12 * n + t] = g.carry;
+      if (t + 1 < n) rlx::to_state(X = rlx::mul(X, jump), g);
+    }
+    o[len - 1] = inverted && inverted[r] ? 1.0 : 0.0;
+    MGPU_HIP(ctx, hipMemcpyAsync((char *)ctx->slot[1] + ctx->zs * r, o, len * sizeof(double), hipMemcpyHostToDevice,
+                                 ctx->stream));
   }
+  hipLaunchKernelGGL(k_seed_table, dim3(cdiv(n, 64), 1, count), dim3(64), 0, ctx->stream, (const double *)ctx->slot[1],
+                     n, adv, N, inverted != nullptr, table, ctx->zs);
+  MGPU_HIP(ctx, hipGetLastError());
+  return MGPU_OK;
 }
 
 int spectrum(mgpu_ctx *ctx, int mode, const float2 *cd, const float2 *cd2, float2 *out, int a, int b,
@@ -638,29 +694,27 @@ int ic_scratch_init(mgpu_ctx *ctx) {
   return MGPU_OK;
 }
 
-// displacement_fields.  seed_dev == nullptr: the seed table goes to a buffer
-// allocated for the call; otherwise to seed_dev (the per-device scratch), and
-// nothing is allocated on the device.
+// displacement_fields.  The seed table goes to seed_dev (the per-device scratch) or,
+// with nullptr, to slot 2 (work space of the initial conditions); nothing is
+// allocated on the device either way.
 int ic_displacement_fields(mgpu_ctx *ctx, unsigned long seed, int sphere_mode, int amp_fixed, int inverted,
                            const double *pk_n2, unsigned *seed_dev) {
   PhaseTimer pt(ctx, &ctx->t.ic);
   const int N = ctx->N;
   int rc;
-  std::vector<unsigned> st;
-  seedtable_host(N, seed, st);
-  unsigned *dseed = seed_dev;
-  if (!dseed) MGPU_HIP(ctx, hipMalloc(&dseed, st.size() * sizeof(unsigned)));
-  MGPU_HIP(ctx, hipMemcpyAsync(dseed, st.data(), st.size() * sizeof(unsigned), hipMemcpyHostToDevice, ctx->stream));
+  std::vector<double> st;
+  unsigned *dseed = seed_dev ? seed_dev : (unsigned *)ctx->slot[2];
+  if ((rc = seed_tables(ctx, 1, &seed, nullptr, dseed, st))) return rc;
   if ((rc = upload_n2(ctx, 0, pk_n2))) return rc;
   float2 *cd = ctx->p.scale_dependent ? ctx->cdelta[0] : ctx->slot[0];
   MGPU_HIP(ctx, hipMemsetAsync(cd, 0, ctx->slot_elems * sizeof(float2), ctx->stream));
   hipLaunchKernelGGL(k_ic_delta, dim3(cdiv((size_t)N * N, kBlock)), dim3(kBlock), 0, ctx->stream, dseed, N, ctx->Np,
-                     ctx->HP, ctx->p.box, sphere_mode, amp_fixed, inverted, ctx->n2tab[0], cd, (size_t)0, (size_t)0,
+                     ctx->HP, ctx->p.box, sphere_mode, amp_fixed, inverted, ctx->n2tab[0], cd, (size_t)0,
                      (const int *)nullptr);
   MGPU_HIP(ctx, hipGetLastError());
-  MGPU_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  if (!seed_dev) MGPU_HIP(ctx, hipFree(dseed));
-  return ic_lpt_from_delta(ctx, cd);
+  if ((rc = ic_lpt_from_delta(ctx, cd))) return rc;
+  MGPU_HIP(ctx, hipStreamSynchronize(ctx->stream));  // the uploads' host memory goes out of scope
+  return MGPU_OK;
 }
 
 // From delta(k) in cd on: the 2LPT source and the ZA and 2LPT lattice
@@ -717,21 +771,10 @@ int ic_displacement_fields_batch(mgpu_ctx *const *m, int count, const unsigned l
     return mgpu_fail(ctx, MGPU_E_STATE, "batched initial conditions: not for scale-dependent runs");
   const int N = ctx->N;
   const size_t nn = (size_t)N * N;
-  // all seed tables, then the inversion flags, in one upload
-  std::vector<unsigned> all(count * nn + count), st;
-  for (int r = 0; r < count; r++) {
-    seedtable_host(N, seeds[r], st);
-    std::copy(st.begin(), st.end(), all.begin() + r * nn);
-    all[count * nn + r] = inverted[r] ? 1u : 0u;
-  }
-  unsigned *dbuf = nullptr;
-  MGPU_HIP(ctx, hipMalloc(&dbuf, all.size() * sizeof(unsigned)));
-  struct Free {
-    unsigned *p;
-    ~Free() { (void)hipFree(p); }
-  } free_dbuf{dbuf};
-  MGPU_HIP(ctx, hipMemcpyAsync(dbuf, all.data(), all.size() * sizeof(unsigned), hipMemcpyHostToDevice, ctx->stream));
   int rc;
+  std::vector<double> st;
+  // the seed tables, and behind them the inversion flags, in the members' slot 2
+  if ((rc = seed_tables(ctx, count, seeds, inverted, (unsigned *)ctx->slot[2], st))) return rc;
   for (int r = 0; r < count; r++) {
     // every member holds the table (later calls on a member alone read its own)
     if ((rc = upload_n2(m[r], 0, pk_n2))) return rc;
@@ -743,9 +786,9 @@ int ic_displacement_fields_batch(mgpu_ctx *const *m, int count, const unsigned l
   } restore{ctx};
   ctx->bz = (unsigned)count;
   float2 *cd = ctx->slot[0];
-  hipLaunchKernelGGL(k_ic_delta, dim3(cdiv(nn, kBlock), 1, count), dim3(kBlock), 0, ctx->stream, dbuf, N, ctx->Np,
-                     ctx->HP, ctx->p.box, sphere_mode, amp_fixed, 0, ctx->n2tab[0], cd, ctx->zs, nn,
-                     (const int *)(dbuf + count * nn));
+  hipLaunchKernelGGL(k_ic_delta, dim3(cdiv(nn, kBlock), 1, count), dim3(kBlock), 0, ctx->stream,
+                     (const unsigned *)ctx->slot[2], N, ctx->Np, ctx->HP, ctx->p.box, sphere_mode, amp_fixed, 0,
+                     ctx->n2tab[0], cd, ctx->zs, (const int *)ctx->slot[2] + nn);
   MGPU_HIP(ctx, hipGetLastError());
   if ((rc = ic_lpt_from_delta(ctx, cd))) return rc;
   MGPU_HIP(ctx, hipStreamSynchronize(ctx->stream));

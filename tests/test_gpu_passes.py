@@ -126,3 +126,18 @@ def test_two_slot_fold_with_constant_growth(n, ns):
         g.lpt_fields(s, a * ones, norm2 * b * ones)
         assert rel_err(got[s], g.get_lpt(s)) < 4e-6
     g.close()
+
+
+@pytest.mark.parametrize("n", [8, 12, 16, 24, 48, 64, 96, 128])
+def test_seed_table_by_chunks(n):
+    """The jumped-ahead chunks of the RANLUX stream give the oracle's serial seed table: with
+    fixed amplitudes every mode's phase is its column stream's draw, so one wrong seed moves
+    a whole column of delta(k).  Sizes with one chunk (8-24), a part-filled last one (48, 96)
+    and several waves' worth; FP32 storage of the same FP64 products: 1e-6."""
+    pk = 100.0 / (1.0 + np.arange(M.n2_table_len(n), dtype=np.float64))
+    for seed in (1, 5001, 2147483647):
+        g = M.MGPU(n, n // 2, BOX, OM, scale_dependent=1)
+        g.ic_displacement_fields(seed, pk, amplitude_fixed=1)
+        want = O.complex_view(O.ic_delta(O.cfg(n, n // 2, BOX, OM), seed, pk, 0, 1, 0), n)
+        assert rel_err(g.get_mesh(M.MESH_CDELTA1), want) < 1e-6
+        g.close()
