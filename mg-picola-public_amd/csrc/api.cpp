@@ -289,6 +289,11 @@ int create_ctx(const mgpu_params *p, mgpu_ctx **out, mgpu_arena *arena, char *sh
       if ((rc = alloc(ctx, (void **)&ctx->lattice_slot, 6 * nl * sizeof(float2), "lattice spectra"))) return fail(rc);
     }
   }
+  // the initial conditions' lattice fields, folded into the mesh slots
+  if (!p->scale_dependent && ctx->N % ctx->Np == 0 && ctx->N > ctx->Np && fft_size_supported(ctx->Np)) {
+    if ((rc = fft_plan_init(ctx, &ctx->fft_read, ctx->Np, MGPU_FFT_TCOLS))) return fail(rc);
+    ctx->fft_read.kcat = MGPU_K_LPT;
+  }
   ctx->partial_len = 3 * (size_t)std::max<size_t>(cdiv(ctx->np, 256), (size_t)ctx->N) + 3 * 1024;
   if ((rc = alloc(ctx, (void **)&ctx->partial, ctx->partial_len * sizeof(double), "reduction scratch"))) return fail(rc);
   if ((rc = alloc(ctx, (void **)&ctx->dsum, 8 * sizeof(double), "sums"))) return fail(rc);
@@ -416,6 +421,7 @@ void mgpu_destroy(mgpu_ctx *ctx) {
   if (ctx->slice_ev) (void)hipEventDestroy(ctx->slice_ev);
   fft_plan_free(&ctx->fft);
   fft_plan_free(&ctx->fft_lattice);
+  fft_plan_free(&ctx->fft_read);
   if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
   if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
   if (arena) {

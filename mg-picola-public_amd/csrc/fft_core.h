@@ -327,6 +327,17 @@ __device__ __forceinline__ void xcd_tile(int &bx, int &by) {
   by = (int)(lin / nbx);
 }
 
+// Integer wavenumber of index i as the LPT fields take it (src/2LPT.c:339-366: the
+// Nyquist index counts as -N/2), and 1/n2 in FP64: the reciprocal estimate and two
+// Newton steps, within a rounding of the quotient at a third of a division's instructions.
+__device__ __forceinline__ int kint(int i, int N) { return i < N / 2 ? i : i - N; }
+__device__ __forceinline__ double recip(int n2) {
+  const double x = (double)n2;
+  double y = __builtin_amdgcn_rcp(x);
+  y = fma(fma(-x, y, 1.0), y, y);
+  return fma(fma(-x, y, 1.0), y, y);
+}
+
 // ---------------------------------------------------------------- strided column pass
 constexpr int col_ept(int L, int T) { return elems_per_thread(L); }
 constexpr int col_threads(int L, int T) { return L * T / col_ept(L, T); }

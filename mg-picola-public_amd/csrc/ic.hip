@@ -3,13 +3,16 @@
 //   k_ic_delta         displacement_fields' Gaussian mode loop (src/2LPT.c:337-495):
 //                      one thread per (i, j) column re-seeds RANLUX from the seed
 //                      table and draws (phase, amplitude) for kz < N/2 in order.
-//   k_lpt_spectrum     i k_a/k^2 delta(k) g(|k|) and the displacement-gradient
-//                      spectra (src/2LPT.c:1224-1277, 1311-1373, 1583-1629),
-//                      2LPT.c wavenumbers (Nyquist = -N/2).
+//   k_lpt_spectrum     i k_a/k^2 delta(k) g(|k|) of the scale-dependent fields
+//                      (src/2LPT.c:1583-1629), 2LPT.c wavenumbers (Nyquist = -N/2);
+//                      the displacements' and the gradients' spectra ride on their
+//                      x passes (lpt_passes.hip).
+//   k_disp_fold        the displacement spectra folded onto the particle lattice
 //   k_lattice_read     trilinear read-out at the Lagrangian lattice
 //                      (src/2LPT.c:1407-1476, 1657-1702) + per-block sums for the
 //                      mean removal (src/2LPT.c:1493-1508, 1713-1729).
 #include "mgpu_internal.h"
+#include "fft_core.h"
 #include "ranlux.h"
 #include "ranlux_jump.h"
 
@@ -26,6 +29,9 @@
 static __device__ __align__(256) unsigned scratch[MGPU_IC_SCRATCH_SEEDS];
 
 namespace {
+
+using fftc::kint;
+using fftc::recip;
 
 constexpr int kBlock = 256;
 constexpr int kMaxDevices = 64;
@@ -133,17 +139,14 @@ __global__ __launch_bounds__(kBlock) void k_ic_delta(const unsigned *__restrict_
 __device__ __forceinline__ double kc(int i, int N, double kf) { return (i < N / 2 ? i : -(N - i)) * kf; }
 __device__ __forceinline__ int nabs(int i, int N) { return i < N / 2 ? i : N - i; }
 
-enum { SPEC_DISP = 0, SPEC_GRAD = 1, SPEC_DISP2 = 2, SPEC_FIELD = 3, SPEC_NEG = 4 };
+enum { SPEC_FIELD = 0, SPEC_NEG = 1 };
 
-// Spectral kernels of the IC / LPT fields.  mode:
-//   SPEC_DISP   out = i k_a/k^2 cd                           (cdisp, src/2LPT.c:417-490)
-//   SPEC_GRAD   out = i k_b (i k_a/k^2 cd) = -k_a k_b/k^2 cd  (cdigrad, src/2LPT.c:1247-1271)
-//   SPEC_DISP2  out = -i k_a/k^2 src                        (cdisp2, src/2LPT.c:1359-1370)
+// Spectral kernel of the scale-dependent LPT fields.  mode:
 //   SPEC_FIELD  out = i k_a/k^2 (g1 cd + g2 cd2)            (from_cdisp_store_to_ZA, both orders)
 //   SPEC_NEG    out = -src, 0 at k = 0                      (cdelta_cdm2, src/2LPT.c:1336-1345)
 __global__ __launch_bounds__(kBlock) void k_lpt_spectrum(int mode, const float2 *__restrict__ cd,
                                                          const float2 *__restrict__ cd2, float2 *__restrict__ out,
-                                                         int N, int HP, double kf, int a, int b,
+                                                         int N, int HP, double kf, int a,
                                                          const double *__restrict__ g1,
                                                          const double *__restrict__ g2, size_t zs) {
   cd = zbuf(cd, zs);
@@ -160,21 +163,7 @@ __global__ __launch_bounds__(kBlock) void k_lpt_spectrum(int mode, const float2 
     const double k2 = kv[0] * kv[0] + kv[1] * kv[1] + kv[2] * kv[2];
     if (k2 > 0.0) {
       double re = 0, im = 0;
-      if (mode == SPEC_DISP || mode == SPEC_GRAD) {
-        const float2 d = cd[e];
-        // cdisp = (-k_a/k2 * im, k_a/k2 * re)
-        re = -kv[a] / k2 * d.y;
-        im = kv[a] / k2 * d.x;
-        if (mode == SPEC_GRAD) {  // times i k_b
-          const double r2 = -im * kv[b], i2 = re * kv[b];
-          re = r2;
-          im = i2;
-        }
-      } else if (mode == SPEC_DISP2) {
-        const float2 s = cd[e];
-        re = s.y * kv[a] / k2;
-        im = -s.x * kv[a] / k2;
-      } else if (mode == SPEC_FIELD) {
+      if (mode == SPEC_FIELD) {
         const int n2 = nabs(i, N) * nabs(i, N) + nabs(j, N) * nabs(j, N) + nabs(k, N) * nabs(k, N);
         const float2 d = cd[e];
         double dr = d.x * g1[n2], di = d.y * g1[n2];
@@ -194,31 +183,6 @@ __global__ __launch_bounds__(kBlock) void k_lpt_spectrum(int mode, const float2 
     }
   }
   out[e] = r;
-}
-
-// 2LPT source on padded real meshes: src = d00 (d11 + d22) + d11 d22 (first
-// call), src -= d*d (off-diagonal calls).  src/2LPT.c:1282-1290
-// src may be d00 (each element is read before it is written)
-__global__ __launch_bounds__(kBlock) void k_source_diag(const float *d00, const float *__restrict__ d11,
-                                                        const float *__restrict__ d22, float *src, size_t n,
-                                                        size_t zs) {
-  d00 = zbuf(d00, zs);
-  d11 = zbuf(d11, zs);
-  d22 = zbuf(d22, zs);
-  src = zbuf(src, zs);
-  size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
-  const double a = d00[e], b = d11[e], c = d22[e];
-  src[e] = (float)(a * (b + c) + b * c);
-}
-__global__ __launch_bounds__(kBlock) void k_source_off(const float *__restrict__ d, float *__restrict__ src,
-                                                       size_t n, size_t zs) {
-  d = zbuf(d, zs);
-  src = zbuf(src, zs);
-  size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
-  const double v = d[e];
-  src[e] = (float)((double)src[e] - v * v);
 }
 
 // trilinear lattice read-out, src/2LPT.c:1407-1476.  out[q] = scale * value
@@ -525,6 +489,76 @@ __global__ __launch_bounds__(kFoldNT, 4) void k_lpt_fold_gs(const float2 *__rest
   }
 }
 
+// The fold of scale i n_a/n^2 X, a = 0..2, with the multipliers and the sums in FP64:
+// component a's spectrum at out + a nl.  One thread per output mode, first the kz
+// between the planes, row by row, then the kz = 0 and Nsample/2 modes of all rows, so
+// that a wave takes one path.  Bound by the read of the mesh's spectrum, row segments
+// of the m^2 aliases up and down (384 to 192: 105 us, 2.9 TB/s).
+template <int MF, bool PLANES>
+__device__ __forceinline__ void disp_fold(int ip, int jp, int lp, const float2 *__restrict__ X, int N, int HP, int Np,
+                                          int m_rt, double acc[6]) {
+  const int m = MF > 0 ? MF : m_rt;
+#pragma unroll
+  for (int q = 0; q < 6; q++) acc[q] = 0.0;
+  if (ip == 0 && jp == 0 && lp == 0) return;
+  // (re, im) += (wr, wi) (i n_a/n^2 X(i, j, l)), component by component
+  auto add = [&](int i, int j, int l, double wr, double wi) {
+    const float2 d = X[((size_t)i * N + j) * HP + l];
+    const int n[3] = {kint(i, N), kint(j, N), kint(l, N)}, n2 = n[0] * n[0] + n[1] * n[1] + n[2] * n[2];
+    const double w = n2 > 0 ? recip(n2) : 0.0, x = wr * w * d.y, y = wi * w * d.x;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      acc[2 * a] -= (double)n[a] * x;
+      acc[2 * a + 1] += (double)n[a] * y;
+    }
+  };
+#pragma unroll
+  for (int a = 0; a < m; a++) {
+    const int i = ip + a * Np, mi = i == 0 ? 0 : N - i;
+#pragma unroll
+    for (int b = 0; b < m; b++) {
+      const int j = jp + b * Np, mj = j == 0 ? 0 : N - j;
+#pragma unroll
+      for (int c = 0; c < m; c++) {
+        const int l = lp + c * Np;
+        if (l > 0 && l < N / 2) {
+          add(i, j, l, 1.0, 1.0);
+        } else if (l > N / 2) {
+          add(mi, mj, N - l, 1.0, -1.0);
+        } else if (PLANES) {  // kz = 0 or N/2 plane: (X(k) + conj X(-k)) / 2
+          add(i, j, l, 0.5, 0.5);
+          add(mi, mj, l, 0.5, -0.5);
+        }
+      }
+    }
+  }
+}
+template <int MF>
+__global__ __launch_bounds__(kBlock) void k_disp_fold(const float2 *__restrict__ X, int N, int HP, int Np, int HPn,
+                                                      int m_rt, double scale, float2 *__restrict__ out, size_t nl,
+                                                      size_t zs) {
+  X = zbuf(X, zs);
+  out = zbuf(out, zs);
+  const size_t rows = (size_t)Np * Np, H = Np / 2, inner = rows * (H - 1);
+  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  double acc[6];
+  size_t row;
+  int lp;
+  if (e < inner) {
+    row = e / (H - 1);
+    lp = 1 + (int)(e % (H - 1));
+    disp_fold<MF, false>((int)(row / Np), (int)(row % Np), lp, X, N, HP, Np, m_rt, acc);
+  } else {
+    if (e >= inner + 2 * rows) return;
+    row = (e - inner) >> 1;
+    lp = (e - inner) & 1 ? (int)H : 0;
+    disp_fold<MF, true>((int)(row / Np), (int)(row % Np), lp, X, N, HP, Np, m_rt, acc);
+  }
+#pragma unroll
+  for (int a = 0; a < 3; a++)
+    out[a * nl + row * HPn + lp] = make_float2((float)(scale * acc[2 * a]), (float)(scale * acc[2 * a + 1]));
+}
+
 __global__ __launch_bounds__(kBlock) void k_d2f(size_t n, const double *__restrict__ a, float *__restrict__ b) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) b[i] = (float)a[i];
@@ -632,14 +666,14 @@ int seed_tables(mgpu_ctx *ctx, int count, const unsigned long *seeds, const int 
   return MGPU_OK;
 }
 
-int spectrum(mgpu_ctx *ctx, int mode, const float2 *cd, const float2 *cd2, float2 *out, int a, int b,
+int spectrum(mgpu_ctx *ctx, int mode, const float2 *cd, const float2 *cd2, float2 *out, int a,
              const double *g1 = nullptr, const double *g2 = nullptr) {
   const double kf = 2 * MGPU_PI / ctx->p.box;
   const double modes = (double)ctx->N * ctx->N * (ctx->N / 2 + 1);
   {
     KScope ks(ctx, MGPU_K_LPT, 8.0 * modes * (cd2 ? 3 : 2));
     hipLaunchKernelGGL(k_lpt_spectrum, dim3(cdiv(ctx->slot_elems, kBlock), 1, ctx->bz), dim3(kBlock), 0, ctx->stream,
-                       mode, cd, cd2, out, ctx->N, ctx->HP, kf, a, b, g1, g2, ctx->zs);
+                       mode, cd, cd2, out, ctx->N, ctx->HP, kf, a, g1, g2, ctx->zs);
   }
   MGPU_HIP(ctx, hipGetLastError());
   return MGPU_OK;
@@ -717,48 +751,73 @@ int ic_displacement_fields(mgpu_ctx *ctx, unsigned long seed, int sphere_mode, i
   return MGPU_OK;
 }
 
+// The lattice displacements i k_a/k^2 X scale of spectrum X in slot in (0 or 1), mean
+// removed, into LPT slot o; slots 2 and 3 are work space.  Where the mesh is a multiple
+// of the lattice the read-out has weight 1 on one node, and the spectra are folded onto
+// the lattice's own (192 of 384: three
+// fields in 205 us with their transforms, where each took 500 us on the mesh); else, and at Nmesh =
+// Nsample where there is nothing to fold, the mesh's transform is read out.
+static int ic_read_displacements(mgpu_ctx *ctx, const float2 *X, double scale, int o) {
+  int rc;
+  if (ctx->fft_read.n > 0) {
+    const FFTPlan *plan = &ctx->fft_read;
+    const int Np = ctx->Np, m = ctx->N / Np;
+    const size_t nl = (size_t)Np * Np * plan->hp;  // 3 nl <= N^2 HP: m >= 2
+    float2 *buf = ctx->slot[2];
+    {
+      KScope ks(ctx, MGPU_K_LPT, ctx->bz * 8.0 * ((double)ctx->N * ctx->N * (ctx->N / 2 + 1) + 3.0 * Np * Np * (Np / 2 + 1)));
+      auto kern = m == 2 ? k_disp_fold<2> : m == 3 ? k_disp_fold<3> : k_disp_fold<0>;
+      hipLaunchKernelGGL(kern, dim3(cdiv((size_t)Np * Np * (Np / 2 + 1), kBlock), 1, ctx->bz), dim3(kBlock), 0,
+                         ctx->stream, X, ctx->N, ctx->HP, Np, plan->hp, m, scale * ctx->p.box / (2 * MGPU_PI), buf, nl,
+                         ctx->zs);
+    }
+    MGPU_HIP(ctx, hipGetLastError());
+    if (ctx->bz == 1) {
+      float *out[2] = {ctx->lpt[o], nullptr};
+      return fft_c2r_fields(ctx, plan, buf, nl, 1, out, ctx->np);
+    }
+    for (int a = 0; a < 3; a++)
+      if ((rc = fft_c2r_3d(ctx, plan, buf + a * nl, ctx->lpt[o] + a * ctx->np))) return rc;
+    return MGPU_OK;
+  }
+  for (int a = 0; a < 3; a++) {
+    if ((rc = lpt_x_pass(ctx, X, ctx->slot[3], nullptr, nullptr, LptFields{1, {a}, {-1}, 1.0}))) return rc;
+    if ((rc = fft_pass_col(ctx, &ctx->fft, ctx->slot[3], 1, 0))) return rc;
+    if ((rc = fft_pass_z(ctx, &ctx->fft, ctx->slot[3], 0))) return rc;
+    if ((rc = readout(ctx, ctx->slot[3], scale, ctx->lpt[o] + (size_t)a * ctx->np))) return rc;
+  }
+  return MGPU_OK;
+}
+
 // From delta(k) in cd on: the 2LPT source and the ZA and 2LPT lattice
 // displacements (or, scale-dependent, the stored -source).  Every launch covers
 // ctx->bz realizations (a batch's member 0 with bz = count).
 int ic_lpt_from_delta(mgpu_ctx *ctx, float2 *cd) {
   int rc;
-  const int N = ctx->N;
-  // displacement gradient -> 2LPT source (real), built in slot 1 over the
-  // psi_00 gradient (the diagonal gradients in slots 1-3)
-  const size_t nr = 2 * ctx->slot_elems;
-  const unsigned gr = cdiv(nr, kBlock);
-  static const int ga[3] = {0, 1, 2};
-  for (int g = 0; g < 3; g++) {
-    if ((rc = spectrum(ctx, SPEC_GRAD, cd, nullptr, ctx->slot[1 + g], ga[g], ga[g]))) return rc;
-    if ((rc = fft_c2r_3d(ctx, &ctx->fft, ctx->slot[1 + g]))) return rc;
-  }
-  hipLaunchKernelGGL(k_source_diag, dim3(gr, 1, ctx->bz), dim3(kBlock), 0, ctx->stream, (const float *)ctx->slot[1],
-                     (const float *)ctx->slot[2], (const float *)ctx->slot[3], (float *)ctx->slot[1], nr, ctx->zs);
-  MGPU_HIP(ctx, hipGetLastError());
-  static const int oa[3] = {0, 0, 1}, ob[3] = {1, 2, 2};
-  for (int g = 0; g < 3; g++) {
-    if ((rc = spectrum(ctx, SPEC_GRAD, cd, nullptr, ctx->slot[3], oa[g], ob[g]))) return rc;
-    if ((rc = fft_c2r_3d(ctx, &ctx->fft, ctx->slot[3]))) return rc;
-    hipLaunchKernelGGL(k_source_off, dim3(gr, 1, ctx->bz), dim3(kBlock), 0, ctx->stream, (const float *)ctx->slot[3],
-                       (float *)ctx->slot[1], nr, ctx->zs);
-    MGPU_HIP(ctx, hipGetLastError());
-  }
-  if ((rc = fft_r2c_3d(ctx, &ctx->fft, ctx->slot[1]))) return rc;
+  const FFTPlan *plan = &ctx->fft;
+  float2 *s = ctx->slot[1], *d1 = ctx->slot[2], *d2 = ctx->slot[3];
+  // displacement gradients -> 2LPT source, built in slot 1 with two more slots of work
+  // space: the diagonal ones, two off the diagonal, the last one and the r2c
+  if ((rc = lpt_x_pass(ctx, cd, s, d1, d2, LptFields{3, {0, 1, 2}, {0, 1, 2}, 1.0}))) return rc;
+  for (float2 *d : {s, d1, d2})
+    if ((rc = fft_pass_col(ctx, plan, d, 1, 0))) return rc;
+  if ((rc = lpt_source_pass(ctx, LPT_DIAG, s, d1, d2))) return rc;
+  if ((rc = lpt_x_pass(ctx, cd, d1, d2, nullptr, LptFields{2, {0, 0}, {1, 2}, 1.0}))) return rc;
+  for (float2 *d : {d1, d2})
+    if ((rc = fft_pass_col(ctx, plan, d, 1, 0))) return rc;
+  if ((rc = lpt_source_pass(ctx, LPT_OFF2, s, d1, d2))) return rc;
+  if ((rc = lpt_x_pass(ctx, cd, d1, nullptr, nullptr, LptFields{1, {1}, {2}, 1.0}))) return rc;
+  if ((rc = fft_pass_col(ctx, plan, d1, 1, 0))) return rc;
+  if ((rc = lpt_source_pass(ctx, LPT_OFF1, s, d1, nullptr))) return rc;
+  if ((rc = fft_pass_col(ctx, plan, s, 1, 1))) return rc;
+  if ((rc = fft_pass_col(ctx, plan, s, 0, 1))) return rc;
 
-  if (ctx->p.scale_dependent) {
-    if ((rc = spectrum(ctx, SPEC_NEG, ctx->slot[1], nullptr, ctx->cdelta[1], 0, 0))) return rc;
-    return MGPU_OK;
-  }
-  // ZA and 2LPT displacements at the lattice, mean removed
-  const double inv_n3 = 1.0 / ((double)N * N * N);
-  for (int a = 0; a < 3; a++) {
-    if ((rc = spectrum(ctx, SPEC_DISP, cd, nullptr, ctx->slot[3], a, 0))) return rc;
-    if ((rc = fft_c2r_3d(ctx, &ctx->fft, ctx->slot[3]))) return rc;
-    if ((rc = readout(ctx, ctx->slot[3], 1.0, ctx->lpt[0] + (size_t)a * ctx->np))) return rc;
-    if ((rc = spectrum(ctx, SPEC_DISP2, ctx->slot[1], nullptr, ctx->slot[2], a, 0))) return rc;
-    if ((rc = fft_c2r_3d(ctx, &ctx->fft, ctx->slot[2]))) return rc;
-    if ((rc = readout(ctx, ctx->slot[2], -3. / 7. * inv_n3, ctx->lpt[1] + (size_t)a * ctx->np))) return rc;
-  }
+  if (ctx->p.scale_dependent) return spectrum(ctx, SPEC_NEG, s, nullptr, ctx->cdelta[1], 0);
+  // ZA and 2LPT displacements at the lattice, mean removed (cdisp, src/2LPT.c:417-490;
+  // cdisp2 = -i k_a/k^2 src, src/2LPT.c:1359-1370, read out with -3/7 N^-3)
+  const double inv_n3 = 1.0 / ((double)ctx->N * ctx->N * ctx->N);
+  if ((rc = ic_read_displacements(ctx, cd, 1.0, 0))) return rc;
+  if ((rc = ic_read_displacements(ctx, s, 3. / 7. * inv_n3, 1))) return rc;
   MGPU_HIP(ctx, hipStreamSynchronize(ctx->stream));
   return MGPU_OK;
 }
@@ -876,7 +935,7 @@ static int lattice_fields(mgpu_ctx *ctx, int ns, const int *slots, const SliceFo
   }
   if (ns != 1) return mgpu_fail(ctx, MGPU_E_INVALID, "several LPT slots at once need the lattice fold");
   for (int a = 0; a < 3; a++) {
-    if ((rc = spectrum(ctx, SPEC_FIELD, ctx->cdelta[0], ctx->cdelta[1], ctx->slot[3], a, 0, ctx->n2tab[0],
+    if ((rc = spectrum(ctx, SPEC_FIELD, ctx->cdelta[0], ctx->cdelta[1], ctx->slot[3], a, ctx->n2tab[0],
                        ctx->n2tab[1])))
       return rc;
     if ((rc = fft_c2r_3d(ctx, &ctx->fft, ctx->slot[3]))) return rc;

@@ -123,6 +123,7 @@ struct mgpu_ctx {
   FFTPlan fft;
   FFTPlan fft_lattice;  // Nsample-sized plan for folded LPT fields (when N % Ns == 0)
   float2 *lattice_slot = nullptr;  // 3 Nsample^3 half spectra
+  FFTPlan fft_read;     // Nsample-sized plan of the initial conditions' read-out (N a multiple of Nsample, not equal)
   double *slice_buf = nullptr;     // growth slices uploaded by mgpu_lpt_fields_slices
   size_t slice_len = 0;
   double *slice_host = nullptr;    // pinned staging buffer of the slices
@@ -209,6 +210,16 @@ struct PhaseTimer {
   PhaseTimer(mgpu_ctx *c, double *f);
   ~PhaseTimer();
 };
+
+// ---------------------------------------------------------------- LPT spectra in FFT passes (lpt_passes.hip)
+// n <= 3 fields sign i k_a/k^2 X, or with b >= 0 i k_b times that
+struct LptFields {
+  int n, a[3], b[3];
+  double sign;
+};
+enum { LPT_DIAG, LPT_OFF2, LPT_OFF1 };
+int lpt_x_pass(mgpu_ctx *ctx, const float2 *cd, float2 *o0, float2 *o1, float2 *o2, const LptFields &f);
+int lpt_source_pass(mgpu_ctx *ctx, int mode, float2 *s, const float2 *d1, const float2 *d2);
 
 // ---------------------------------------------------------------- FFT (fft.hip)
 int fft_plan_init(mgpu_ctx *ctx, FFTPlan *plan, int n, int tcols = 16);

@@ -141,3 +141,25 @@ def test_seed_table_by_chunks(n):
         want = O.complex_view(O.ic_delta(O.cfg(n, n // 2, BOX, OM), seed, pk, 0, 1, 0), n)
         assert rel_err(g.get_mesh(M.MESH_CDELTA1), want) < 1e-6
         g.close()
+
+
+@pytest.mark.parametrize("tcols", [8, 16])
+@pytest.mark.parametrize("n,ns", [(8, 4), (8, 8), (16, 8), (24, 8), (32, 8), (48, 20), (64, 16), (96, 24), (96, 48),
+                                  (128, 128), (192, 64)])
+def test_lpt_passes_and_fold(n, ns, tcols):
+    """Lattice displacements from the fused spectrum, source and read-out against the oracle:
+    fold factors 2, 3 and 4, none (Nmesh = Nsample), and lattices that do not divide the mesh
+    or have no transform of their own (4, 20).  FP32 rounding of 3 log2(n)-stage transforms:
+    the bounds of the oracle comparisons of the separate passes, 1e-5 and, through the
+    products of the source, 2e-5 of the field maximum."""
+    pk = 1000.0 / (1.0 + np.arange(M.n2_table_len(n), dtype=np.float64)) ** 1.5
+    pk[0] = 0.0
+    print("n, ns, tcols =", n, ns, tcols, flush=True)
+    g = M.MGPU(n, ns, BOX, OM)
+    g.set_fft_tile(0, tcols)
+    g.ic_displacement_fields(4001, pk)
+    c = O.cfg(n, ns, BOX, OM)
+    za, lp = O.ic_displacements(c, O.ic_delta(c, 4001, pk), 0)
+    assert rel_err(g.get_lpt(0), za) < 1e-5
+    assert rel_err(g.get_lpt(1), lp) < 2e-5
+    g.close()
