@@ -98,6 +98,29 @@ __device__ __forceinline__ unsigned bin_key(const float *__restrict__ pos, const
 // scatter forms the key again from the position.
 constexpr int kBinU = 4;
 
+// Particle u of this thread.  ns > 0 (a multiple of 32): the workgroup takes the block of
+// 4 x 8 x 32 particles of the ns^3 lattice that the particles started from, which spread
+// over fewer bins than 1024 in a row do: fewer global atomics here and longer runs of
+// records in the scatter (512^3 particles on 1024^3: binning 1249 -> 809 us with the
+// runs' shared atomics of k_dep_bin, scatter 1503 -> 1263 us; 256^3 on 256^3: 138 -> 98
+// and 133 -> 131 us).  It is an order only: any particles may be in any place.
+struct BinIndex {
+  size_t i0;
+  unsigned step;
+  __device__ __forceinline__ BinIndex(int ns) {
+    if (ns > 0) {
+      const unsigned nz = ns / 32, ny = ns / 8, bz = blockIdx.x % nz, by = blockIdx.x / nz % ny, bx = blockIdx.x / (nz * ny);
+      i0 = ((size_t)(4 * bx) * ns + 8 * by + (threadIdx.x >> 5)) * ns + 32 * bz + (threadIdx.x & 31);
+      step = (unsigned)ns * (unsigned)ns;
+    } else {
+      i0 = (size_t)blockIdx.x * (kBinU * kTB) + threadIdx.x;
+      step = kTB;
+    }
+  }
+  __device__ __forceinline__ size_t operator()(int u) const { return i0 + (size_t)u * step; }
+};
+static_assert(kBinU * kTB == 4 * 8 * 32 && kTB == 256, "lattice block of a workgroup");
+
 // LDS hash slots of a workgroup's keys (kBinU kTB particles: at most half full, so
 // every probe sequence ends at a free or matching slot)
 constexpr int kBinHBits = 11, kBinH = 1 << kBinHBits;
@@ -105,7 +128,7 @@ static_assert(kBinH >= 2 * kBinU * kTB, "hash table too small for a workgroup's 
 template <bool RSD>
 __global__ __launch_bounds__(kTB) void k_dep_bin(const float *__restrict__ pos, const float4 *__restrict__ crd,
                                                  size_t np, TileGeom g, double scale, unsigned *__restrict__ count,
-                                                 unsigned *__restrict__ rank, size_t zs) {
+                                                 unsigned *__restrict__ rank, int ns, size_t zs) {
   pos = zbuf(pos, zs);
   crd = zbuf(crd, zs);
   count = zbuf(count, zs);
@@ -117,31 +140,41 @@ __global__ __launch_bounds__(kTB) void k_dep_bin(const float *__restrict__ pos, 
     hcnt[s] = 0u;
   }
   __syncthreads();
-  const size_t i0 = (size_t)blockIdx.x * (kBinU * kTB) + threadIdx.x;
+  const BinIndex at(ns);
   unsigned t[kBinU], loc[kBinU];
   int slot[kBinU];
 #pragma unroll
   for (int u = 0; u < kBinU; u++) {
-    const size_t i = i0 + (size_t)u * kTB;
-    t[u] = i < np ? bin_key<RSD>(pos, crd, np, i, g, scale) : 0u;
-    slot[u] = -1;
-    loc[u] = 0u;
+    const size_t i = at(u);
+    t[u] = i < np ? bin_key<RSD>(pos, crd, np, i, g, scale) : kEmpty;
   }
-  // the workgroup's keys into the LDS table (linear probing), a local rank per key
+  // the workgroup's keys into the LDS table (linear probing), a local rank per key; the
+  // first lane of each run of equal keys does it for the run
+  const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int u = 0; u < kBinU; u++) {
-    if (i0 + (size_t)u * kTB < np) {
+    const unsigned before = __shfl_up(t[u], 1);
+    const bool head = lane == 0 || t[u] != before;
+    const unsigned long long heads = __ballot(head), upto = heads & (~0ull >> (63 - lane));
+    const int first = 63 - __clzll((long long)upto);
+    int sl = -1;
+    unsigned lo = 0u;
+    if (head && t[u] != kEmpty) {
+      const unsigned long long after = heads & ~(~0ull >> (63 - lane));
+      const unsigned len = (unsigned)((after ? __ffsll((long long)after) - 1 : 64) - lane);
       unsigned h = (t[u] * 2654435761u) >> (32 - kBinHBits);
       for (int p = 0; p < kBinH; ++p) {
         const unsigned prev = atomicCAS(&hkey[h], kEmpty, t[u]);
         if (prev == kEmpty || prev == t[u]) {
-          slot[u] = (int)h;
+          sl = (int)h;
           break;
         }
         h = (h + 1) & (kBinH - 1);
       }
-      if (slot[u] >= 0) loc[u] = atomicAdd(&hcnt[slot[u]], 1u);
+      if (sl >= 0) lo = atomicAdd(&hcnt[sl], len);
     }
+    slot[u] = __shfl(sl, first);
+    loc[u] = __shfl(lo, first) + (unsigned)(lane - first);
   }
   __syncthreads();
   // one global atomic per distinct key of the workgroup: its base replaces the count
@@ -152,7 +185,7 @@ __global__ __launch_bounds__(kTB) void k_dep_bin(const float *__restrict__ pos, 
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < kBinU; u++) {
-    const size_t i = i0 + (size_t)u * kTB;
+    const size_t i = at(u);
     if (i < np) rank[i] = slot[u] >= 0 ? hcnt[slot[u]] + loc[u] : atomicAdd(&count[t[u]], 1u);
   }
 }
@@ -248,22 +281,22 @@ template <bool RSD>
 __global__ __launch_bounds__(kTB) void k_dep_scatter(const unsigned *__restrict__ rank,
                                                      const unsigned *__restrict__ off, const float *__restrict__ pos,
                                                      const float4 *__restrict__ crd, size_t np, TileGeom g,
-                                                     double scale, float4 *__restrict__ rec, size_t zs) {
+                                                     double scale, float4 *__restrict__ rec, int ns, size_t zs) {
   rank = zbuf(rank, zs);
   off = zbuf(off, zs);
   pos = zbuf(pos, zs);
   crd = zbuf(crd, zs);
   rec = zbuf(rec, zs);
-  const size_t i0 = (size_t)blockIdx.x * (kBinU * kTB) + threadIdx.x;
+  const BinIndex at(ns);
   unsigned o[kBinU];
 #pragma unroll
   for (int u = 0; u < kBinU; u++) {
-    const size_t i = i0 + (size_t)u * kTB;
+    const size_t i = at(u);
     o[u] = i < np ? off[bin_key<RSD>(pos, crd, np, i, g, scale)] + rank[i] : 0u;
   }
 #pragma unroll
   for (int u = 0; u < kBinU; u++) {
-    const size_t i = i0 + (size_t)u * kTB;
+    const size_t i = at(u);
     if (i < np)
       rec[o[u]] = RSD ? crd[i] : make_float4(pos[i], pos[np + i], pos[2 * np + i], __uint_as_float((unsigned)i));
   }
@@ -606,6 +639,7 @@ int deposit_tiled(mgpu_ctx *ctx, float *d, const float4 *rsd) {
   const size_t zs = ctx->zs;
   // the scan leaves the counters at zero; a context's first deposit, or one after a failed
   // one, clears them (by a kernel, not hipMemsetAsync, so that the step can be captured)
+  const int ns = ctx->Np % 32 == 0 ? ctx->Np : 0;  // lattice blocks fill the particles exactly
   if (!ctx->dep_counts_zero)
     hipLaunchKernelGGL(k_zero_u32, dim3((unsigned)std::min<size_t>(cdiv(nb + 1, 1024), 65535), 1, bz), dim3(256), 0,
                        ctx->stream, count, nb + 1, zs);
@@ -613,7 +647,7 @@ int deposit_tiled(mgpu_ctx *ctx, float *d, const float4 *rsd) {
   if (np) {
     KScope ks(ctx, MGPU_K_DEP_SORT, 16.0 * np);
     hipLaunchKernelGGL(rsd ? k_dep_bin<true> : k_dep_bin<false>, dim3(cdiv(np, kBinU * kTB), 1, bz), dim3(kTB), 0,
-                       ctx->stream, ctx->pos, rsd, np, g, scale, count, rank, zs);
+                       ctx->stream, ctx->pos, rsd, np, g, scale, count, rank, ns, zs);
   }
   MGPU_HIP(ctx, hipGetLastError());
   if (nb <= kScanOne) {
@@ -627,7 +661,7 @@ int deposit_tiled(mgpu_ctx *ctx, float *d, const float4 *rsd) {
   if (np) {
     KScope ks(ctx, MGPU_K_DEP_SORT, 32.0 * np);
     hipLaunchKernelGGL(rsd ? k_dep_scatter<true> : k_dep_scatter<false>, dim3(cdiv(np, kBinU * kTB), 1, bz),
-                       dim3(kTB), 0, ctx->stream, rank, off, ctx->pos, rsd, np, g, scale, rec, zs);
+                       dim3(kTB), 0, ctx->stream, rank, off, ctx->pos, rsd, np, g, scale, rec, ns, zs);
   }
   MGPU_HIP(ctx, hipGetLastError());
   const size_t shmem = sizeof(unsigned long long) * g.tx * g.ty * g.tz;
