@@ -289,8 +289,11 @@ int create_ctx(const mgpu_params *p, mgpu_ctx **out, mgpu_arena *arena, char *sh
       if ((rc = alloc(ctx, (void **)&ctx->lattice_slot, 6 * nl * sizeof(float2), "lattice spectra"))) return fail(rc);
     }
   }
-  // the initial conditions' lattice fields, folded into the mesh slots
-  if (!p->scale_dependent && ctx->N % ctx->Np == 0 && ctx->N > ctx->Np && fft_size_supported(ctx->Np)) {
+  // the initial conditions' lattice fields, folded into the mesh slots.  Up to a quarter
+  // of the mesh: a mode's m^3 aliases are one thread's work, which for small lattices in
+  // large meshes leaves the chip idle.
+  if (!p->scale_dependent && ctx->N % ctx->Np == 0 && ctx->N > ctx->Np && ctx->N <= 4 * ctx->Np &&
+      fft_size_supported(ctx->Np)) {
     if ((rc = fft_plan_init(ctx, &ctx->fft_read, ctx->Np, MGPU_FFT_TCOLS))) return fail(rc);
     ctx->fft_read.kcat = MGPU_K_LPT;
   }

@@ -28,7 +28,7 @@ __device__ __forceinline__ void anew(V &v) {
 // 384, in launches of three, two and one: 0.55 ms, where six sweeps took 0.80 ms and
 // their x passes 0.58 ms.
 template <int L, int T>
-__global__ __launch_bounds__(col_threads(L, T), 4) void k_lpt_x(const float2 *__restrict__ cd, float2 *o0, float2 *o1,
+__global__ __launch_bounds__(col_threads(L, T), tw_in_lds(L) ? 4 : 1) void k_lpt_x(const float2 *__restrict__ cd, float2 *o0, float2 *o1,
                                                              float2 *o2, LptFields f, size_t ls, size_t os,
                                                              const float2 *__restrict__ tw, double kf, size_t zs) {
   cd = zbuf(cd, zs);

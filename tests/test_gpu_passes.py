@@ -144,11 +144,11 @@ def test_seed_table_by_chunks(n):
 
 
 @pytest.mark.parametrize("tcols", [8, 16])
-@pytest.mark.parametrize("n,ns", [(8, 4), (8, 8), (16, 8), (24, 8), (32, 8), (48, 20), (64, 16), (96, 24), (96, 48),
+@pytest.mark.parametrize("n,ns", [(8, 4), (8, 8), (16, 8), (24, 8), (32, 8), (48, 20), (64, 16), (96, 16), (96, 24), (96, 48),
                                   (128, 128), (192, 64)])
 def test_lpt_passes_and_fold(n, ns, tcols):
     """Lattice displacements from the fused spectrum, source and read-out against the oracle:
-    fold factors 2, 3 and 4, none (Nmesh = Nsample), and lattices that do not divide the mesh
+    fold factors 2, 3 and 4, none (Nmesh = Nsample, or 6), and lattices that do not divide the mesh
     or have no transform of their own (4, 20).  FP32 rounding of 3 log2(n)-stage transforms:
     the bounds of the oracle comparisons of the separate passes, 1e-5 and, through the
     products of the source, 2e-5 of the field maximum."""
