@@ -321,15 +321,14 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_pofk(float2 *buf, siz
 //                with delta(k) read from dk (as k_col_green adds them).
 //   FWD_PLAIN    the same without the epilogue (DGP: phi(k) is the transform).
 // Then S times the MODE multiplier and the inverse x transform(s), as
-// k_col_green.  The forward's last stage stores its outputs into LDS in the
-// tile layout (after a barrier), from where each thread takes its first-stage
-// operands of the inverse.
+// k_col_green.  The forward's outputs reach the inverse in registers or through LDS
+// (see kHand).
 // What bounds it: with one workgroup per CU its load, transform and store phases add
 // up.  At most 128 VGPRs (four waves per SIMD, two 512-thread workgroups per CU at
 // 1024) let one tile's loads and stores run under another's transforms; the stage
 // twiddles in LDS free the registers and the vector-memory queue for that.  Force
-// pair 6.45 -> 4.68 ms at 1024 (2.8 -> 3.8 TB/s), 316 -> 254 us at 384; density pair
-// with the Green's force (LCDM) 7.2 -> 5.2 ms at 1024, 340 -> 293 us at 384.
+// pair 6.45 -> 4.55 ms at 1024 (2.7 -> 3.8 TB/s), 316 -> 239 us at 384; density pair
+// with P(k) 4.81 -> 4.19 ms at 1024, with the Green's force (LCDM) 7.2 -> 5.2 ms.
 enum { FWD_DENSITY = 0, FWD_EPI = 1, FWD_PLAIN = 2 };
 template <int L, int T, int FWD, int MODE>
 __global__ __launch_bounds__(col_threads(L, T), tw_in_lds(L) ? 4 : 1) void k_col_fused(
@@ -421,8 +420,9 @@ __global__ __launch_bounds__(col_threads(L, T), tw_in_lds(L) ? 4 : 1) void k_col
 enum { SCREEN_POTENTIAL = 0, SCREEN_DENSITY = 1 };
 
 // z pass: c2r of the row (potential Phi_N or smoothed density delta_R), the
-// screening against the delta(x) row, r2c of the effective density; the row
-// stays in LDS between the three steps.
+// screening against the delta(x) row, r2c of the effective density.  The screened row
+// goes from the one's last stage to the other's first, of the same radix, in registers:
+// 3.53 -> 3.02 ms at 1024 (4.3 TB/s), 213 -> 183 us at 384 with the potential.
 //   SCREEN_POTENTIAL (f(R), m-beta; src/mg.h:169-171, src/user_defined_functions.h:725-752):
 //       delta_eff = delta * min(1, |p0 / Phi|) where Phi < 0, else delta       (p0 = phi_crit)
 //   SCREEN_DENSITY (DGP; src/mg.h:235-244, src/user_defined_functions.h:757-773):

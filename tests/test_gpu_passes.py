@@ -144,8 +144,8 @@ def test_seed_table_by_chunks(n):
 
 
 @pytest.mark.parametrize("tcols", [8, 16])
-@pytest.mark.parametrize("n,ns", [(8, 4), (8, 8), (16, 8), (24, 8), (32, 8), (48, 20), (64, 16), (96, 16), (96, 24), (96, 48),
-                                  (128, 128), (192, 64)])
+@pytest.mark.parametrize("n,ns", [(8, 4), (8, 8), (16, 8), (24, 8), (32, 8), (48, 20), (64, 16), (96, 16), (96, 24),
+                                  (96, 48), (128, 128), (192, 64)])
 def test_lpt_passes_and_fold(n, ns, tcols):
     """Lattice displacements from the fused spectrum, source and read-out against the oracle:
     fold factors 2, 3 and 4, none (Nmesh = Nsample, or 6), and lattices that do not divide the mesh
