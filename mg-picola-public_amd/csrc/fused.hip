@@ -27,6 +27,21 @@ namespace {
 
 using namespace fftc;
 
+// Stores of the passes that write more than one mesh: past the caches from 384 on, where a
+// mesh is larger than they keep until the next pass reads it, and with full 128-byte lines
+// (16 columns; half lines cost more than they gain).  Dual y pass / density pair: 146 / 165
+// -> 137 / 143 us at 384, 1.38 / 1.93 -> 1.20 / 1.80 ms at 768, 2.84 / 4.19 -> 2.80 / 4.15
+// ms at 1024; up to 256 the next pass finds the meshes in the caches.
+template <int L, int T>
+__device__ __forceinline__ void put(float2 &p, float2 v) {
+  if constexpr (L >= 384 && T == 16) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    __builtin_nontemporal_store(f2{v.x, v.y}, reinterpret_cast<f2 *>(&p));
+  } else {
+    p = v;
+  }
+}
+
 __device__ __forceinline__ int nsgn(int i, int N) { return i > N / 2 ? i - N : i; }
 
 enum { GREEN_FORCE = FUSED_GREEN_FORCE, GREEN_LAPLACE = FUSED_GREEN_LAPLACE, GREEN_SMOOTH = FUSED_GREEN_SMOOTH };
@@ -149,11 +164,11 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_dual(float2 *buf, flo
     }
   }
   auto ld = [&](int, int, int) { return make_float2(0.f, 0.f); };
-  auto st0 = [&](int c, int j, int o, float2 v) { col_at<L, T>(oy + tile, ls, c, j, o) = v; };
+  auto st0 = [&](int c, int j, int o, float2 v) { put<L, T>(col_at<L, T>(oy + tile, ls, c, j, o), v); };
   const float2 *twl = stw.to_lds(lds, tid);
   fft_stages<L, T, NT, +1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ld, st0, p1);
   __syncthreads();
-  auto st1 = [&](int c, int j, int o, float2 v) { col_at<L, T>(buf + tile, ls, c, j, o) = v; };
+  auto st1 = [&](int c, int j, int o, float2 v) { put<L, T>(col_at<L, T>(buf + tile, ls, c, j, o), v); };
   fft_stages<L, T, NT, +1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ld, st1, p2);
 }
 
@@ -364,7 +379,7 @@ __global__ __launch_bounds__(col_threads(L, T), tw_in_lds(L) ? 4 : 1) void k_col
   auto st = [&](int c, int j, int o, float2 v) {
     const int kx = j + o, kz = kz0 + c;
     if (FWD == FWD_DENSITY) {
-      if (kout) col_at<L, T>(kout + tile, ls, c, j, o) = v;
+      if (kout) put<L, T>(col_at<L, T>(kout + tile, ls, c, j, o), v);
       if (bin) pl.add(v, kx, d1, kz, fn, copies, tid);
     }
     if (FWD == FWD_EPI) {
@@ -405,10 +420,10 @@ __global__ __launch_bounds__(col_threads(L, T), tw_in_lds(L) ? 4 : 1) void k_col
     }
   }
   auto ldz = [&](int, int, int) { return make_float2(0.f, 0.f); };
-  auto st0 = [&](int c, int j, int o, float2 v) { col_at<L, T>(out0 + tile, ls, c, j, o) = v; };
+  auto st0 = [&](int c, int j, int o, float2 v) { put<L, T>(col_at<L, T>(out0 + tile, ls, c, j, o), v); };
   fft_stages<L, T, NT, +1, 1, T, true, true, 1, false, true, kHand>(lds, twl, 1, tid, ldz, st0, p1);
   if (MODE == GREEN_FORCE) {
-    auto st1 = [&](int c, int j, int o, float2 v) { col_at<L, T>(out1 + tile, ls, c, j, o) = v; };
+    auto st1 = [&](int c, int j, int o, float2 v) { put<L, T>(col_at<L, T>(out1 + tile, ls, c, j, o), v); };
     fft_stages<L, T, NT, +1, 1, T, true, true, 1, false, true, kHand>(lds, twl, 1, tid, ldz, st1, p2);
   }
   if (bin) {

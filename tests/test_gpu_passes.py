@@ -195,3 +195,25 @@ def test_bins_do_not_depend_on_particle_order(ns, n):
     g.get_displacements()
     np.testing.assert_array_equal(g.get_disp(), d[:, perm])
     g.close()
+
+
+@pytest.mark.parametrize("model", ["lcdm", "dgp"])
+@pytest.mark.parametrize("n", [192, 384])
+def test_tile_widths_and_stores_give_the_same_forces(model, n):
+    """8- and 16-column tiles (from 384 on with stores past the caches in the passes of more
+    than one mesh) change no column's arithmetic: the force meshes are equal to the bit."""
+    pos = lattice_particles(32, BOX, amp=1.5, seed=n)
+    kw = dict(model=M.DGP, mg_active=1, include_screening=1, filter=O.FILTER_GAUSSIAN) if model == "dgp" else {}
+    mg = M.MG(a=0.7, coupling=0.12, dgp_fac=0.05, rsmooth=2.0, geff=1.0) if model == "dgp" else None
+    print("model, n =", model, n, flush=True)
+    out = []
+    for tcols in (8, 16):
+        g = M.MGPU(n, 32, BOX, OM, **kw)
+        g.set_fft_tile(0, tcols)
+        g.set_particles(pos)
+        g.get_displacements(mg=mg)
+        out.append([g.get_mesh(m) for m in (M.MESH_FORCE_X, M.MESH_FORCE_Y, M.MESH_FORCE_Z)])
+        g.close()
+    for a, b in zip(*out):
+        assert np.abs(a).max() > 0
+        np.testing.assert_array_equal(a, b)
