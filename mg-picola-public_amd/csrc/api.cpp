@@ -762,12 +762,20 @@ int run_step(mgpu_ctx *ctx, const mgpu_mg *mg, double dda, double A, double s1k,
   if (graph && ctx->step_warm) {
     hipGraph_t g = nullptr;
     MGPU_HIP(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeRelaxed));
+    // until the graph is launched nothing of the step has run: what the captured deposit
+    // noted (cleared counters, sorted records) does not hold when a call fails before that
+    struct NotRun {
+      mgpu_ctx *c;
+      ~NotRun() {
+        if (!c) return;
+        c->dep_counts_zero = c->sorted_valid = false;
+        (void)hipGetLastError();  // reported by the call that failed
+      }
+    } not_run{ctx};
     rc = device_step_body(ctx, mg, dda, A, s1k, s2k, dyyy, s1d, s2d);
     const hipError_t e = hipStreamEndCapture(ctx->stream, &g);
     if (rc || e != hipSuccess || !g) {
       if (g) (void)hipGraphDestroy(g);
-      (void)hipGetLastError();
-      ctx->dep_counts_zero = false;  // nothing of the capture has run
       return rc ? rc : mgpu_fail(ctx, MGPU_E_HIP, std::string("step capture failed: ") + hipGetErrorString(e));
     }
     if (ctx->step_exec) {
@@ -783,11 +791,11 @@ int run_step(mgpu_ctx *ctx, const mgpu_mg *mg, double dda, double A, double s1k,
     if (!ctx->step_exec && hipGraphInstantiate(&ctx->step_exec, g, nullptr, nullptr, 0) != hipSuccess) {
       ctx->step_exec = nullptr;
       (void)hipGraphDestroy(g);
-      ctx->dep_counts_zero = false;
       return mgpu_fail(ctx, MGPU_E_HIP, "step graph instantiation failed");
     }
     (void)hipGraphDestroy(g);
     MGPU_HIP(ctx, hipGraphLaunch(ctx->step_exec, ctx->stream));
+    not_run.c = nullptr;
   } else {
     if ((rc = device_step_body(ctx, mg, dda, A, s1k, s2k, dyyy, s1d, s2d))) return rc;
     ctx->step_warm = true;
@@ -916,7 +924,7 @@ int mgpu_batch_step(mgpu_ctx *const *members, int count, const mgpu_mg *mg, doub
   rc = run_step(m0, mg, dda, A, s1k, s2k, dyyy, s1d, s2d, graph);
   m0->bz = 1;
   if (rc) {
-    for (int r = 0; r < count; r++) members[r]->dep_counts_zero = false;
+    for (int r = 0; r < count; r++) members[r]->dep_counts_zero = members[r]->sorted_valid = false;
     return rc;
   }
   const size_t rec_off = (const char *)m0->dep_rec - (const char *)m0->dep_scratch;

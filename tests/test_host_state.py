@@ -1,0 +1,80 @@
+"""The host side of libmgpu.so on a stand-in runtime (fake_hip.cpp): which kernels a call
+launches, and what a context believes after a launch, a capture or a copy has failed.  Each
+case runs in a process of its own, so that the stand-in is there before libmgpu.so.  No GPU."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+PRELUDE = """
+import ctypes as C, sys
+import numpy as np
+F = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+sys.path[:0] = sys.argv[2:]
+import mgpicola as M
+
+ran = lambda kernel: F.fake_ran(kernel.encode())
+
+def fails(what, call, *args, **kw):
+    F.fake_fail(what.encode())
+    try:
+        call(*args, **kw)
+    except M.MGPUError:
+        return
+    raise AssertionError(what + " did not fail the call")
+
+def context(n=32, ns=16, **kw):
+    g = M.MGPU(n, ns, 64.0, 0.3, **kw)
+    g.set_particles(np.zeros((3, ns**3), np.float32), np.zeros((3, ns**3), np.float32))
+    return g
+
+def forces_at_hand(g):
+    for m in (M.MESH_FORCE_X, M.MESH_FORCE_Y, M.MESH_FORCE_Z):
+        g.set_mesh(m, np.zeros((g.n,) * 3))
+"""
+
+
+@pytest.fixture(scope="session")
+def fake(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-o", so, os.path.join(HERE, "fake_hip.cpp")], check=True)
+
+    def run(code):
+        p = subprocess.run([sys.executable, "-c", PRELUDE + code, so, os.path.join(HERE, "..", "mg-picola-public_amd")],
+                           stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
+        assert p.returncode == 0, p.stdout
+
+    return run
+
+
+@pytest.mark.parametrize("call", ["k_gather_tile", "hipStreamEndCapture", "hipGraphInstantiate", "hipGraphLaunch"])
+@pytest.mark.parametrize("members", [1, 3])
+def test_bins_after_a_step_graph_that_never_ran(fake, call, members):
+    """A deposit fails half-way (its counters hold counts), then the graph of the next step,
+    which would have cleared them, fails before it runs: the step after that clears them, and
+    a gather in between does not take the records that the graph would have sorted."""
+    fake(f"""
+members, call = {members}, "{call}"
+ms = M.MGPU.batch(members, 32, 16, 64.0, 0.3) if members > 1 else [M.MGPU(32, 16, 64.0, 0.3)]
+for g in ms:
+    g.set_particles(np.zeros((3, 16**3), np.float32), np.zeros((3, 16**3), np.float32))
+    g.kick(0.1, 1.0, 0.0, 0.0, g.get_displacements()[0])
+a = (0.1, 1.0, 0.0, 0.0, 0.1, 0.0, 0.0)
+step = lambda: M.MGPU.batch_step(ms, *a, graph=True) if members > 1 else ms[0].step(*a, graph=True)
+F.fake_reset()
+step()
+assert ran("k_dep_bin") == 1 and ran("k_zero_u32") == 0
+fails("k_dep_bin", ms[-1].pm_deposit)
+F.fake_reset()
+fails(call, step)
+assert ran("k_dep_bin") == 0
+forces_at_hand(ms[0])
+ms[0].mesh_to_particles()
+assert ran("k_gather_tile") == 0 and ran("k_gather") == 1
+F.fake_reset()
+step()
+assert ran("k_dep_bin") == 1 and ran("k_zero_u32") == 1
+""")
