@@ -632,7 +632,7 @@ int deposit_tiled(mgpu_ctx *ctx, float *d, const float4 *rsd) {
   // redshift-space positions)
   ctx->dep_rec = rec;
   ctx->dep_off = off;
-  ctx->sorted_valid = np > 0 && !rsd;
+  ctx->sorted_valid = false;
   const double scale = (double)N / ctx->p.box;
   const double wpar = std::pow((double)N / (double)ctx->Np, 3);
   const unsigned bz = ctx->bz;
@@ -687,6 +687,7 @@ int deposit_tiled(mgpu_ctx *ctx, float *d, const float4 *rsd) {
                        2 * ctx->HP, d, zs);
   }
   MGPU_HIP(ctx, hipGetLastError());
+  ctx->sorted_valid = np > 0 && !rsd;
   return MGPU_OK;
 }
 

@@ -78,3 +78,17 @@ F.fake_reset()
 step()
 assert ran("k_dep_bin") == 1 and ran("k_zero_u32") == 1
 """)
+
+
+@pytest.mark.parametrize("kernel", ["k_dep_bin", "k_scan_one", "k_dep_scatter", "k_dep_tiles"])
+def test_no_gather_by_the_records_of_a_failed_deposit(fake, kernel):
+    """A context's first deposit fails before its records and bin offsets are written: the
+    gather takes the particles one by one and not by what the memory holds."""
+    fake(f"""
+g = context()
+fails("{kernel}", g.pm_deposit)
+forces_at_hand(g)
+F.fake_reset()
+g.mesh_to_particles()
+assert ran("k_gather_tile") == 0 and ran("k_gather") == 1
+""")
