@@ -366,8 +366,10 @@ int mgpu_set_fft_tile(mgpu_ctx *ctx, int which, int tcols); /* 16 only where the
 int mgpu_get_fft_tile(mgpu_ctx *ctx, int which, int *tcols);
 /* Measure both widths on this device (a forward x pass and the y passes of the
  * force, or an inverse y pass of the lattice transforms; the better of two) and
- * keep the faster, for both plans.  It uses the force meshes and the
- * lattice spectra as scratch: call it before the initial conditions.
+ * keep the faster, for both plans.  It uses the force meshes and the lattice
+ * spectra as scratch: call it before the initial conditions.  With a density or
+ * forces at hand it times plain passes over the F_x mesh alone: densities and
+ * phi(k) stay, the forces are to be made again.
  * ms: 4 doubles (main 8, main 16, lattice 8, lattice 16; -1 where not run). */
 int mgpu_autotune_fft(mgpu_ctx *ctx, double ms[4]);
 

@@ -647,7 +647,12 @@ int mgpu_get_fft_tile(mgpu_ctx *ctx, int which, int *tcols) {
 int mgpu_autotune_fft(mgpu_ctx *ctx, double ms[4]) {
   if (check_ctx(ctx) || !ms) return MGPU_E_INVALID;
   ms[0] = ms[1] = ms[2] = ms[3] = -1.0;
-  int rc = fft_autotune(ctx, &ctx->fft, ctx->slot[3], true, ms);
+  // the force passes are timed over slots 1 to 3 while no mesh is in use; a delta(x) (slot
+  // 1), a phi(k) (slot 2) or force meshes leave only slot 3 to plain passes, which takes
+  // F_x from the force meshes
+  const bool idle = !ctx->have_deposit && !ctx->have_density && !ctx->have_forces && !ctx->have_phik;
+  ctx->have_forces = false;
+  int rc = fft_autotune(ctx, &ctx->fft, ctx->slot[3], idle, ms);
   if (!rc && ctx->fft_lattice.n > 0 && ctx->lattice_slot) rc = fft_autotune(ctx, &ctx->fft_lattice, ctx->lattice_slot, false, ms + 2);
   return rc;
 }

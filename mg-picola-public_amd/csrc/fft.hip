@@ -226,9 +226,9 @@ int fft_plan_init(mgpu_ctx *ctx, FFTPlan *plan, int n, int tcols) {
 }
 
 // The column passes' tile width measured on this device: a forward x pass, and the y
-// passes of the force tail over the force slots (force: the Nmesh plan) or an inverse
-// y pass over buf (a scratch mesh of the plan's size), with each width that fits, one
-// warm-up and the better of two; the faster becomes plan->tcols.  The width changes no
+// passes of the force tail over the force slots (force: the Nmesh plan, no mesh in use) or
+// an inverse y pass over buf (a scratch mesh of the plan's size), with each width that
+// fits, one warm-up and the better of two; the faster becomes plan->tcols.  The width changes no
 // column's arithmetic, only the schedule.  The y passes alone do not tell the widths
 // apart at 1024 (3.51 against 3.47 ms a pair for 8 and 16), where the dual pass takes
 // 3.18 against 2.75 ms and the density pair with P(k) 6.0 against 4.1 ms.

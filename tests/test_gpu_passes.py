@@ -217,3 +217,36 @@ def test_tile_widths_and_stores_give_the_same_forces(model, n):
     for a, b in zip(*out):
         assert np.abs(a).max() > 0
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("after", ["deposit", "density", "fifth"])
+@pytest.mark.parametrize("model,n", [("fofr", 48), ("dgp", 48), ("dgp", 384)])
+def test_autotune_leaves_the_meshes_in_use(model, n, after):
+    """The autotuner between the calls of a force computation: the delta(x) of slot 1 and the
+    phi(k) of slot 2 stay what they were (up to 256 and beyond the y passes of the force are
+    one launch and two), so the displacements are equal to the bit; force meshes, which it
+    uses, are refused afterwards."""
+    pos = lattice_particles(24, BOX, amp=1.5, seed=n)
+    kw = dict(model=M.FOFR if model == "fofr" else M.DGP, mg_active=1, include_screening=1,
+              filter=O.FILTER_NONE if model == "fofr" else O.FILTER_GAUSSIAN)
+    mg = M.MG(a=0.7, coupling=1 / 3 if model == "fofr" else 0.12, mass2=2e4, phi_crit=3e-8, dgp_fac=0.05, rsmooth=2.0,
+              geff=1.0)
+    print("model, n, after =", model, n, after, flush=True)
+    out = []
+    for tune in (False, True):
+        g = M.MGPU(n, 24, BOX, OM, **kw)
+        g.set_particles(pos)
+        for name, call in (("deposit", g.pm_deposit), ("density", g.pm_transform), ("fifth", lambda: g.fifth_force(mg)),
+                           ("forces", g.forces)):
+            call()
+            if tune and name == after:
+                g.autotune_fft()
+        g.mesh_to_particles()
+        out.append(g.get_disp())
+        if tune:
+            g.autotune_fft()
+            with pytest.raises(M.MGPUError, match="no force meshes"):
+                g.mesh_to_particles()
+        g.close()
+    assert np.abs(out[0]).max() > 0
+    np.testing.assert_array_equal(out[0], out[1])
