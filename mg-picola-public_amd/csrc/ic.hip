@@ -632,6 +632,15 @@ __global__ __launch_bounds__(kBlock) void k_nu_add(float2 *__restrict__ dk, cons
   dk[e] = make_float2((float)(cdmfac * (double)v.x + f * (double)c.x), (float)(cdmfac * (double)v.y + f * (double)c.y));
 }
 
+// Waits for the stream on every way out of the block: the host memory that it copies
+// from stays until the copies are done, also where a later call fails.
+struct StreamWait {
+  mgpu_ctx *ctx;
+  ~StreamWait() {
+    if (ctx) (void)hipStreamSynchronize(ctx->stream);
+  }
+};
+
 // The seed tables of count realizations (ctx's, at the batch stride) into table (on the
 // device): the states the chunks of each stream start from go to slot 1, which the
 // initial conditions overwrite afterwards.  A chunk is 16 advances of 12 values, or
@@ -737,6 +746,7 @@ int ic_displacement_fields(mgpu_ctx *ctx, unsigned long seed, int sphere_mode, i
   const int N = ctx->N;
   int rc;
   std::vector<double> st;
+  StreamWait wait{ctx};
   unsigned *dseed = seed_dev ? seed_dev : (unsigned *)ctx->slot[2];
   if ((rc = seed_tables(ctx, 1, &seed, nullptr, dseed, st))) return rc;
   if ((rc = upload_n2(ctx, 0, pk_n2))) return rc;
@@ -747,6 +757,7 @@ int ic_displacement_fields(mgpu_ctx *ctx, unsigned long seed, int sphere_mode, i
                      (const int *)nullptr);
   MGPU_HIP(ctx, hipGetLastError());
   if ((rc = ic_lpt_from_delta(ctx, cd))) return rc;
+  wait.ctx = nullptr;
   MGPU_HIP(ctx, hipStreamSynchronize(ctx->stream));  // the uploads' host memory goes out of scope
   return MGPU_OK;
 }
@@ -832,6 +843,7 @@ int ic_displacement_fields_batch(mgpu_ctx *const *m, int count, const unsigned l
   const size_t nn = (size_t)N * N;
   int rc;
   std::vector<double> st;
+  StreamWait wait{ctx};
   // the seed tables, and behind them the inversion flags, in the members' slot 2
   if ((rc = seed_tables(ctx, count, seeds, inverted, (unsigned *)ctx->slot[2], st))) return rc;
   for (int r = 0; r < count; r++) {
@@ -850,6 +862,7 @@ int ic_displacement_fields_batch(mgpu_ctx *const *m, int count, const unsigned l
                      ctx->n2tab[0], cd, ctx->zs, (const int *)ctx->slot[2] + nn);
   MGPU_HIP(ctx, hipGetLastError());
   if ((rc = ic_lpt_from_delta(ctx, cd))) return rc;
+  wait.ctx = nullptr;
   MGPU_HIP(ctx, hipStreamSynchronize(ctx->stream));
   return MGPU_OK;
 }

@@ -243,10 +243,9 @@ def test_autotune_leaves_the_meshes_in_use(model, n, after):
                 g.autotune_fft()
         g.mesh_to_particles()
         out.append(g.get_disp())
-        if tune:
-            g.autotune_fft()
-            with pytest.raises(M.MGPUError, match="no force meshes"):
-                g.mesh_to_particles()
-        g.close()
     assert np.abs(out[0]).max() > 0
     np.testing.assert_array_equal(out[0], out[1])
+    g.autotune_fft()
+    with pytest.raises(M.MGPUError, match="no force meshes"):
+        g.mesh_to_particles()
+    g.close()

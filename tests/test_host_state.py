@@ -92,3 +92,21 @@ F.fake_reset()
 g.mesh_to_particles()
 assert ran("k_gather_tile") == 0 and ran("k_gather") == 1
 """)
+
+
+@pytest.mark.parametrize("kernel", ["k_seed_table", "k_ic_delta", "k_lpt_x", "k_lpt_source"])
+@pytest.mark.parametrize("sd", [0, 1])
+def test_initial_conditions_that_fail_wait_for_their_uploads(fake, kernel, sd):
+    """No copy from the call's own states or the caller's table is in flight on return."""
+    fake(f"""
+pk = np.ones(M.n2_table_len(32))
+g = M.MGPU(32, 16, 64.0, 0.3, scale_dependent={sd})
+fails("{kernel}", g.ic_displacement_fields, 1, pk)
+assert F.fake_pending() == 0
+g.ic_displacement_fields(1, pk)
+assert F.fake_pending() == 0 and ran("k_seed_table") >= 1
+if not {sd}:
+    ms = M.MGPU.batch(2, 32, 16, 64.0, 0.3)
+    fails("{kernel}", M.MGPU.batch_ic, ms, [1, 2], pk)
+    assert F.fake_pending() == 0
+""")
