@@ -343,6 +343,8 @@ int create_ctx(const mgpu_params *p, mgpu_ctx **out, mgpu_arena *arena, char *sh
     if ((rc = alloc(ctx, (void **)&ctx->pk_bin, tab.size() * sizeof(int16_t), "P(k) bin table"))) return fail(rc);
     if (hipMemcpy(ctx->pk_bin, tab.data(), tab.size() * sizeof(int16_t), hipMemcpyHostToDevice) != hipSuccess)
       return fail(mgpu_fail(ctx, MGPU_E_HIP, "bin table upload failed"));
+    ctx->pk_fn.table = ctx->pk_bin;
+    ctx->pk_fn.nbins = p->pofk_nbins;
     // the bins by their first |n|^2: below the first bin and past the last one the table
     // holds -1 (bins of unusual kmin, kmax that do not rise with |n|^2 keep the table)
     const int nbk = p->pofk_nbins;
@@ -363,7 +365,6 @@ int create_ctx(const mgpu_params *p, mgpu_ctx **out, mgpu_arena *arena, char *sh
       ctx->pk_fn.edge = dev;
       if (hipMemcpy(dev, edge.data(), edge.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess)
         return fail(mgpu_fail(ctx, MGPU_E_HIP, "bin edge upload failed"));
-      ctx->pk_fn.nbins = nbk;
       ctx->pk_fn.logbins = p->pofk_bintype == 1;
       if (p->pofk_bintype == 1) {
         ctx->pk_fn.a = (float)(0.5 * std::log(2.0) * nbk / lnrange);

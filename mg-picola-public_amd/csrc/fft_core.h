@@ -365,18 +365,18 @@ constexpr bool tw_in_lds(int L) { return L < 1536; }
 constexpr size_t col_lds_elems(int L, int T) { return (size_t)L * T + (tw_in_lds(L) ? L : 0); }
 // Construct before the tile's loads (so the table's loads are the older ones), then
 // to_lds() after them: the table's LDS writes wait for its own loads only.
-template <int L, int T, int NT>
+template <int L, int T, int NT, bool LDS = tw_in_lds(L)>
 struct StageTwiddles {
-  static constexpr int K = tw_in_lds(L) ? (L + NT - 1) / NT : 1;
+  static constexpr int K = LDS ? (L + NT - 1) / NT : 1;
   float2 r[K];
   const float2 *tw;
   __device__ __forceinline__ StageTwiddles(const float2 *t, int tid) : tw(t) {
-    if constexpr (tw_in_lds(L))
+    if constexpr (LDS)
 #pragma unroll
       for (int i = 0; i < K; ++i) r[i] = tw[tid + i * NT < L ? tid + i * NT : 0];
   }
   __device__ __forceinline__ const float2 *to_lds(float2 *lds, int tid) {
-    if constexpr (!tw_in_lds(L)) return tw;
+    if constexpr (!LDS) return tw;
     float2 *t = lds + (size_t)L * T;
 #pragma unroll
     for (int i = 0; i < K; ++i)

@@ -245,10 +245,10 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_epi(float2 *buf, size
 
 // P(k) sums of an x pass in LDS: copies sets of bin sums (lanes take them in turn, so
 // fewer lanes of a wave add to one address: most of a wave's modes share a few bins),
-// the per-axis window and the bin edges.  init() goes behind the tile's loads, so that
-// it costs no latency of its own, and in front of the twiddles' barrier (or, without
-// one, of the stages' barriers).
-template <int L, int NT>
+// the per-axis window and, with EDGES, the bin edges (see fused_pofk_by).  init() goes
+// behind the tile's loads, so that it costs no latency of its own, and in front of the
+// twiddles' barrier (without one, a barrier of its own or the stages' barriers).
+template <int L, int NT, bool EDGES>
 struct PofkLds {
   double *bins;
   float *wv;
@@ -261,21 +261,23 @@ struct PofkLds {
     edge = (int *)(wv + L / 2 + 1);
     for (int b = tid; b < copies * f.nbins; b += NT) bins[b] = 0.0;
     for (int d = tid; d <= L / 2; d += NT) wv[d] = winv[d];
-    for (int b = tid; b <= f.nbins; b += NT) edge[b] = f.edge[b];
+    if (EDGES)
+      for (int b = tid; b <= f.nbins; b += NT) edge[b] = f.edge[b];
   }
   // after a barrier
   __device__ __forceinline__ void begin(const PkBinFn &f) {
+    if (!EDGES) return;
     e0 = edge[0];
     e1 = edge[f.nbins];
   }
   // mode (kx, d1 = |ky|, kz) of power |v|^2: weight 1 (kz = 0, N/2) or 2, CIC deconvolution
   __device__ __forceinline__ void add(float2 v, int kx, int d1, int kz, const PkBinFn &f, int copies, int tid) const {
     if (kz > L / 2) return;
-    const int d0 = kx > L / 2 ? L - kx : kx;
-    const int nk = pk_bin_of(d0 * d0 + d1 * d1 + kz * kz, f, edge, e0, e1);
+    const int d0 = kx > L / 2 ? L - kx : kx, n2 = d0 * d0 + d1 * d1 + kz * kz;
+    const int nk = EDGES ? pk_bin_of(n2, f, edge, e0, e1) : f.table[n2];
     if (nk < 0) return;
     const float w = (kz == 0 || kz == L / 2) ? 1.f : 2.f;
-    atomicAdd(&bins[nk + f.nbins * (tid & (copies - 1))],
+    atomicAdd(&bins[EDGES ? nk + f.nbins * (tid & (copies - 1)) : nk],
               (double)((v.x * v.x + v.y * v.y) * (w * wv[d0] * wv[d1] * wv[kz])));
   }
   // into the workgroup's set of MGPU_PK_SETS global sums (adds to one address are
@@ -295,7 +297,7 @@ struct PofkLds {
 // weight 1 (kz = 0, N/2) or 2, CIC deconvolution winv[d0] winv[d1] winv[d2]
 // (1/N^6 folded in), |n| binned linearly (bintype 0) or logarithmically.
 // Bin sums go to LDS doubles, then one global atomic per bin and block.
-template <int L, int T>
+template <int L, int T, bool EDGES>
 __global__ __launch_bounds__(col_threads(L, T)) void k_col_pofk(float2 *buf, size_t ls, size_t os,
                                                                   const float2 *__restrict__ tw,
                                                                   const float *__restrict__ winv, PkBinFn fn,
@@ -304,7 +306,7 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_pofk(float2 *buf, siz
   constexpr int NT = col_threads(L, T);
   constexpr int N = L;
   const int tid = threadIdx.x;
-  PofkLds<L, NT> pl;
+  PofkLds<L, NT, EDGES> pl;
   int bx, ky;
   xcd_tile(bx, ky);
   const int kz0 = bx * T;
@@ -315,10 +317,11 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_pofk(float2 *buf, siz
     col_at<L, T>(buf + tile, ls, c, j, o) = v;
     pl.add(v, j + o, d1, kz0 + c, fn, copies, tid);
   };
-  StageTwiddles<L, T, NT> stw(tw, tid);
+  StageTwiddles<L, T, NT, EDGES && tw_in_lds(L)> stw(tw, tid);
   float2 pre[col_ept(L, T)];
   first_loads<L, T, NT, true>(pre, tid, ld);
-  pl.init(lds + col_lds_elems(L, T), fn, copies, winv, tid);
+  pl.init(lds + (EDGES ? col_lds_elems(L, T) : (size_t)L * T), fn, copies, winv, tid);
+  if (!EDGES) __syncthreads();  // up to 16 points the only stage adds to the sums
   const float2 *twl = stw.to_lds(lds, tid);
   fft_stages<L, T, NT, -1, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ld, st, pre, [&]() { pl.begin(fn); });
   __syncthreads();
@@ -345,8 +348,8 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_pofk(float2 *buf, siz
 // pair 6.45 -> 4.55 ms at 1024 (2.7 -> 3.8 TB/s), 316 -> 239 us at 384; density pair
 // with P(k) 4.81 -> 4.19 ms at 1024, with the Green's force (LCDM) 7.2 -> 5.2 ms.
 enum { FWD_DENSITY = 0, FWD_EPI = 1, FWD_PLAIN = 2 };
-template <int L, int T, int FWD, int MODE>
-__global__ __launch_bounds__(col_threads(L, T), tw_in_lds(L) ? 4 : 1) void k_col_fused(
+template <int L, int T, int FWD, int MODE, bool EDGES = true>
+__global__ __launch_bounds__(col_threads(L, T), tw_in_lds(L) && EDGES ? 4 : 1) void k_col_fused(
     const float2 *in, float2 *kout, const float2 *__restrict__ dk, float2 *out0, float2 *out1, size_t ls, size_t os,
     const float2 *__restrict__ tw, GreenArgs ga, float coupling, float m2, const float *__restrict__ winv,
     PkBinFn fn, int copies, double *__restrict__ pk, size_t zs) {
@@ -371,7 +374,7 @@ __global__ __launch_bounds__(col_threads(L, T), tw_in_lds(L) ? 4 : 1) void k_col
   const size_t tile = (size_t)ky * os + kz0;
   const int ny = nsgn(ky, N), d1 = ky > N / 2 ? N - ky : ky;
   const bool bin = FWD == FWD_DENSITY && pk != nullptr;
-  PofkLds<L, NT> pl;
+  PofkLds<L, NT, EDGES> pl;
   // forward transform; its outputs stay in the registers of the threads that form them
   float2 p1[E], p2[E];
   auto ld = [&](int c, int j, int o) { return col_at<L, T>(in + tile, ls, c, j, o); };
@@ -390,9 +393,10 @@ __global__ __launch_bounds__(col_threads(L, T), tw_in_lds(L) ? 4 : 1) void k_col
     if constexpr (kHand) p1[oi++] = v;
     else lds[c + kx * T] = v;
   };
-  StageTwiddles<L, T, NT> stw(tw, tid);
+  StageTwiddles<L, T, NT, EDGES && tw_in_lds(L)> stw(tw, tid);
   first_loads<L, T, NT, true>(p1, tid, ld);
-  if (bin) pl.init(lds + col_lds_elems(L, T), fn, copies, winv, tid);
+  if (bin) pl.init(lds + (EDGES ? col_lds_elems(L, T) : (size_t)L * T), fn, copies, winv, tid);
+  if (!EDGES) __syncthreads();  // as in k_col_pofk
   const float2 *twl = stw.to_lds(lds, tid);
   // delta(k) to add, in the layout of the inverse's first stage: requested before the
   // forward's last stage, or after it where the registers are short
@@ -536,23 +540,33 @@ int pofk_copies(const mgpu_ctx *ctx, size_t tile_lds) {
   // not at the price of a workgroup per CU
   return l2 <= ctx->lds_max && (ctx->lds_max / l2 == ctx->lds_max / l1 || ctx->lds_max / l2 >= 4) ? 2 : 1;
 }
+// LDS of an x pass that bins P(k) by the table: the tile, the bin sums and the window
+size_t pofk_table_lds(const mgpu_ctx *ctx, int T) {
+  return (size_t)ctx->N * T * sizeof(float2) + sizeof(double) * (size_t)ctx->p.pofk_nbins + sizeof(float) * (size_t)(ctx->N / 2 + 1);
+}
 
-template <int N, int T, int FWD, int MODE>
-int fused_x_launch_k(mgpu_ctx *ctx, const FusedXArgs &a) {
+template <int N, int T, int FWD, int MODE, bool EDGES>
+int fused_x_launch_by(mgpu_ctx *ctx, const FusedXArgs &a, size_t lds, int copies) {
   const size_t HP = ctx->fft.hp, ls = (size_t)N * HP, os = HP;
-  const size_t tile_lds = col_lds_elems(N, T) * sizeof(float2);
-  const int copies = a.pk ? pofk_copies(ctx, tile_lds) : 1;
-  const size_t lds = tile_lds + (a.pk ? pofk_lds(N, ctx->p.pofk_nbins, copies) : 0);
-  if (lds > ctx->lds_max) return mgpu_fail(ctx, MGPU_E_INVALID, "P(k) bins do not fit the LDS of the x pass");
-  if (a.pk && !ctx->pk_fn.edge) return mgpu_fail(ctx, MGPU_E_INVALID, "no P(k) bin table");
   int rc;
-  auto kern = k_col_fused<N, T, FWD, MODE>;
+  auto kern = k_col_fused<N, T, FWD, MODE, EDGES>;
   if ((rc = set_lds(ctx, kern, lds))) return rc;
   hipLaunchKernelGGL(kern, dim3(HP / T, N, ctx->bz), dim3(col_threads(N, T)), lds, ctx->stream, a.in, a.kout, a.dk,
                      a.o0, a.o1, ls, os, ctx->fft.tw, a.ga, a.coupling, a.m2, ctx->winvf, ctx->pk_fn, copies, a.pk,
                      ctx->zs);
   MGPU_HIP(ctx, hipGetLastError());
   return MGPU_OK;
+}
+template <int N, int T, int FWD, int MODE>
+int fused_x_launch_k(mgpu_ctx *ctx, const FusedXArgs &a) {
+  const size_t tile_lds = col_lds_elems(N, T) * sizeof(float2);
+  if (FWD != FWD_DENSITY || !a.pk) return fused_x_launch_by<N, T, FWD, MODE, true>(ctx, a, tile_lds, 1);
+  const int by = fused_pofk_by(ctx, T);
+  if (by == POFK_NONE) return mgpu_fail(ctx, MGPU_E_INVALID, "P(k) bins do not fit the LDS of the x pass");
+  if constexpr (FWD == FWD_DENSITY)
+    if (by == POFK_TABLE) return fused_x_launch_by<N, T, FWD, MODE, false>(ctx, a, pofk_table_lds(ctx, T), 1);
+  const int copies = pofk_copies(ctx, tile_lds);
+  return fused_x_launch_by<N, T, FWD, MODE, true>(ctx, a, tile_lds + pofk_lds(N, ctx->p.pofk_nbins, copies), copies);
 }
 
 template <int N, int T>
@@ -604,20 +618,24 @@ int epi_launch(mgpu_ctx *ctx, float2 *buf, float coupling, float m2) {
   return MGPU_OK;
 }
 
-template <int N, int T>
-int pofk_launch(mgpu_ctx *ctx, float2 *buf, double *pk) {
+template <int N, int T, bool EDGES>
+int pofk_launch_by(mgpu_ctx *ctx, float2 *buf, double *pk, size_t lds, int copies) {
   const size_t HP = ctx->fft.hp, ls = (size_t)N * HP, os = HP;
-  const size_t tile_lds = col_lds_elems(N, T) * sizeof(float2);
-  const int copies = pofk_copies(ctx, tile_lds);
-  const size_t lds = tile_lds + pofk_lds(N, ctx->p.pofk_nbins, copies);
-  if (lds > ctx->lds_max) return mgpu_fail(ctx, MGPU_E_INVALID, "P(k) bins do not fit the LDS of the x pass");
-  if (!ctx->pk_fn.edge) return mgpu_fail(ctx, MGPU_E_INVALID, "no P(k) bin table");
   int rc;
-  if ((rc = set_lds(ctx, k_col_pofk<N, T>, lds))) return rc;
-  hipLaunchKernelGGL((k_col_pofk<N, T>), dim3(HP / T, N), dim3(col_threads(N, T)), lds, ctx->stream, buf, ls, os,
+  if ((rc = set_lds(ctx, k_col_pofk<N, T, EDGES>, lds))) return rc;
+  hipLaunchKernelGGL((k_col_pofk<N, T, EDGES>), dim3(HP / T, N), dim3(col_threads(N, T)), lds, ctx->stream, buf, ls, os,
                      ctx->fft.tw, ctx->winvf, ctx->pk_fn, copies, pk);
   MGPU_HIP(ctx, hipGetLastError());
   return MGPU_OK;
+}
+template <int N, int T>
+int pofk_launch(mgpu_ctx *ctx, float2 *buf, double *pk) {
+  const int by = fused_pofk_by(ctx, T);
+  if (by == POFK_NONE) return mgpu_fail(ctx, MGPU_E_INVALID, "P(k) bins do not fit the LDS of the x pass");
+  if (by == POFK_TABLE) return pofk_launch_by<N, T, false>(ctx, buf, pk, pofk_table_lds(ctx, T), 1);
+  const size_t tile_lds = col_lds_elems(N, T) * sizeof(float2);
+  const int copies = pofk_copies(ctx, tile_lds);
+  return pofk_launch_by<N, T, true>(ctx, buf, pk, tile_lds + pofk_lds(N, ctx->p.pofk_nbins, copies), copies);
 }
 
 template <int N>
@@ -679,6 +697,21 @@ struct EpiF {
 }  // namespace
 
 // ---------------------------------------------------------------- host entry points
+
+// The edges' and the twiddles' LDS pays while the edges are at most a sixth of the tile
+// (every workgroup copies them) and no workgroup per CU is lost to them.  By the edges / by
+// the table: density and P(k) 8.87 / 9.29 ms at 1024 with 16 columns and 1024 bins (a 32nd),
+// 1.53 / 1.51 ms at 512, 16 columns and 4000 bins (a quarter), an LCDM step 1.65 / 1.74 ms at
+// 384 with 1024 bins (8 columns: a sixth); with a workgroup less 661 / 589 us at 384, 16
+// columns and 2500 bins.
+int fused_pofk_by(const mgpu_ctx *ctx, int T) {
+  const size_t max = ctx->lds_max, l = pofk_table_lds(ctx, T);
+  if (ctx->pk_fn.edge && (size_t)ctx->p.pofk_nbins <= (size_t)ctx->N * T / 3) {
+    const size_t le = fft_col_lds(ctx->N, T) + pofk_lds(ctx->N, ctx->p.pofk_nbins, 1);
+    if (le <= max && (max / le == max / l || max / le >= 4)) return POFK_EDGES;
+  }
+  return ctx->pk_fn.table && l <= max ? POFK_TABLE : POFK_NONE;
+}
 
 int fused_green_x(mgpu_ctx *ctx, int mode, const float2 *a, const float2 *b, float2 *o0, float2 *o1, double p0,
                   double p1, int filter) {

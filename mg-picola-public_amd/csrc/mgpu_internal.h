@@ -99,7 +99,7 @@ struct mgpu_ctx {
   double *winv = nullptr;     // P(k) deconvolution per axis: 1/sinc(pi d/N)^4 N^-2, d = 0..N/2
   float *winvf = nullptr;     // FP32 copy of winv
   int16_t *pk_bin = nullptr;  // P(k) bin of each |n|^2 (-1: outside the bins); null when nbins > 32767
-  PkBinFn pk_fn;              // the same bins by their edges; edge null when pk_bin is, or does not rise with |n|^2
+  PkBinFn pk_fn;              // the same bins by their edges (null when pk_bin is, or does not rise with |n|^2) and pk_bin
   float4 *rsd_crd = nullptr;  // redshift-space particle records (allocated on the first RSD call)
   // massive neutrinos: PtoMesh's term delta = cdmfac delta + fac(|n|^2) cdelta_IC while nu_on
   bool nu_on = false;
@@ -231,6 +231,11 @@ size_t fft_col_lds(int n, int T);
 static inline size_t pofk_lds(int n, int nbins, int copies) {
   return copies * sizeof(double) * (size_t)nbins + sizeof(float) * (size_t)(n / 2 + 1) + sizeof(int) * (size_t)(nbins + 1);
 }
+// How an x pass of T columns bins P(k): by the bin edges, which share the LDS with the
+// bin sums, the tile and the twiddles, or by the table in global memory with the twiddles
+// there too, up to 3839 bins at 1024 with 16 columns and 12031 with 8.
+enum { POFK_NONE, POFK_EDGES, POFK_TABLE };
+int fused_pofk_by(const mgpu_ctx *ctx, int T);
 int fft_autotune(mgpu_ctx *ctx, FFTPlan *plan, float2 *buf, bool force, double ms[2]);
 bool fft_size_supported(int n);
 // in-place 3D transforms on a slot with the padded layout above

@@ -19,10 +19,8 @@ constexpr int kBlock = 256;
 // Only bins [b0, b0 + nb) are accumulated (in LDS), so a bin count beyond
 // the LDS takes several launches over bin ranges.
 __global__ __launch_bounds__(kBlock) void k_pofk(const float2 *__restrict__ dk, int N, int HP,
-                                                 const double *__restrict__ winv, const int16_t *__restrict__ pbin,
-                                                 PkBinFn fn, int nbins, int bintype, double kmin, double kmax, int b0,
-                                                 int nb,
-                                                 double *__restrict__ out) {
+                                                 const double *__restrict__ winv, PkBinFn fn, int nbins, int bintype,
+                                                 double kmin, double kmax, int b0, int nb, double *__restrict__ out) {
   extern __shared__ double sh[];  // 3*nb
   for (int b = threadIdx.x; b < 3 * nb; b += blockDim.x) sh[b] = 0.0;
   __syncthreads();
@@ -39,7 +37,7 @@ __global__ __launch_bounds__(kBlock) void k_pofk(const float2 *__restrict__ dk, 
     const double kmag = sqrt((double)n2);
     int nk;
     if (fn.edge) nk = pk_bin_of(n2, fn, fn.edge, e0, e1);
-    else if (pbin) nk = pbin[n2];  // the same formula, evaluated by the host
+    else if (fn.table) nk = fn.table[n2];  // the same formula, evaluated by the host
     else if (bintype == 0) nk = (int)((kmag - kmin) / (kmax - kmin) * nbins + 0.5);
     else nk = kmag <= 0.0 ? -1 : (int)(log(kmag / kmin) / lnrange * nbins + 0.5);
     if (nk < 0 || nk >= nbins || nk < b0 || nk >= b0 + nb) continue;
@@ -90,8 +88,7 @@ __global__ __launch_bounds__(kBlock) void k_rsd_coords(const float *__restrict__
 // weighted |delta|^2 (deconvolved, 1/N^6), its mu^2 and mu^4 moments with
 // mu^2 = n_z^2/n^2, and the mode count; weights 1 (kz = 0, N/2) or 2.
 __global__ __launch_bounds__(kBlock) void k_rsd_bins(const float2 *__restrict__ dk, int N, int HP,
-                                                     const double *__restrict__ winv,
-                                                     const int16_t *__restrict__ pbin, PkBinFn fn, int nbins,
+                                                     const double *__restrict__ winv, PkBinFn fn, int nbins,
                                                      double *__restrict__ out) {
   extern __shared__ double sh[];  // 4*nbins
   for (int b = threadIdx.x; b < 4 * nbins; b += blockDim.x) sh[b] = 0.0;
@@ -105,7 +102,7 @@ __global__ __launch_bounds__(kBlock) void k_rsd_bins(const float2 *__restrict__ 
     const int j = (int)(rowi % N), i = (int)(rowi / N);
     const int d0 = i > N / 2 ? N - i : i, d1 = j > N / 2 ? N - j : j;
     const int n2 = d0 * d0 + d1 * d1 + k * k;
-    const int nk = fn.edge ? pk_bin_of(n2, fn, fn.edge, e0, e1) : pbin[n2];
+    const int nk = fn.edge ? pk_bin_of(n2, fn, fn.edge, e0, e1) : fn.table[n2];
     if (nk < 0) continue;
     const double kmag = sqrt((double)n2);
     const double mu2 = k == 0 ? 0.0 : (double)(k * k) / kmag / kmag;
@@ -496,18 +493,13 @@ int pm_pofk(mgpu_ctx *ctx, const float2 *dk, mgpu_pofk *out) {
     const int nb = std::min(chunk, nbins - b0);
     KScope ks(ctx, MGPU_K_POFK, 8.0 * modes);
     hipLaunchKernelGGL(k_pofk, dim3(grid), dim3(kBlock), 3 * (size_t)nb * sizeof(double), ctx->stream, dk, N, ctx->HP,
-                       dwin, ctx->pk_bin, ctx->pk_fn, nbins, ctx->p.pofk_bintype, ctx->p.pofk_kmin, ctx->p.pofk_kmax, b0, nb,
+                       dwin, ctx->pk_fn, nbins, ctx->p.pofk_bintype, ctx->p.pofk_kmin, ctx->p.pofk_kmax, b0, nb,
                        ctx->pk);
     MGPU_HIP(ctx, hipGetLastError());
   }
   if ((rc = pofk_queue(ctx, false))) return rc;
   MGPU_HIP(ctx, hipStreamSynchronize(ctx->stream));
   return pofk_finish(ctx, out, false);
-}
-
-// The x pass that bins P(k) holds its tile of T columns and the bins in LDS.
-static bool pofk_fused_fits(const mgpu_ctx *ctx, int T) {
-  return ctx->pk_fn.edge && fft_col_lds(ctx->N, T) + pofk_lds(ctx->N, ctx->p.pofk_nbins, 1) <= ctx->lds_max;
 }
 
 // PtoMesh's r2c of delta(x) (slot dx_slot) into slot 0, with P(k) when out != NULL.
@@ -518,7 +510,7 @@ int pm_transform(mgpu_ctx *ctx, mgpu_pofk *out) {
   const float *dx = (const float *)ctx->slot[ctx->dx_slot];
   int rc;
   if (!out || ctx->pk_geom.size() != 2 * (size_t)ctx->p.pofk_nbins ||
-      !pofk_fused_fits(ctx, ctx->fft.tcols)) {
+      fused_pofk_by(ctx, ctx->fft.tcols) == POFK_NONE) {
     {
       PhaseTimer pt(ctx, &ctx->t.ptomesh);
       if ((rc = fft_r2c_3d(ctx, &ctx->fft, dk, dx))) return rc;
@@ -644,7 +636,7 @@ bool pm_step_fusable(const mgpu_ctx *ctx, const mgpu_mg *mg, const mgpu_pofk *ou
   if (out && ctx->pk_geom.size() != 2 * (size_t)ctx->p.pofk_nbins) return false;
   // the density pair bins P(k) in LDS: 8-column tiles with the Green's force (LCDM), else the plan's width
   const bool lcdm = !ctx->p.mg_active || ctx->p.model == MGPU_LCDM;
-  if (out && !pofk_fused_fits(ctx, lcdm ? 8 : ctx->fft.tcols)) return false;
+  if (out && fused_pofk_by(ctx, lcdm ? 8 : ctx->fft.tcols) == POFK_NONE) return false;
   if (lcdm) return true;
   if (!mg || !ctx->p.include_screening) return false;
   return ctx->p.model == MGPU_FOFR || ctx->p.model == MGPU_MBETA || ctx->p.model == MGPU_DGP;
@@ -876,7 +868,7 @@ int pm_rsd_pofk(mgpu_ctx *ctx, int axis, double vnorm, double s1, double s2, mgp
   {
     KScope ks(ctx, MGPU_K_POFK, 8.0 * modes);
     hipLaunchKernelGGL(k_rsd_bins, dim3(std::min<size_t>(cdiv(modes, kBlock), 4096)), dim3(kBlock), shmem, ctx->stream,
-                       dk, N, ctx->HP, ctx->winv, ctx->pk_bin, ctx->pk_fn, nbins, ctx->pk);
+                       dk, N, ctx->HP, ctx->winv, ctx->pk_fn, nbins, ctx->pk);
   }
   MGPU_HIP(ctx, hipGetLastError());
   const double *h = ctx->host_pk;

@@ -7,12 +7,14 @@
 // formula's bin.  The edges are a few KB, read from LDS; a table of the bin of every
 // |n|^2 (1.5 MB at 1024) costs a gather whose 64 lanes touch up to 64 cache lines:
 // the density x pass that bins P(k) at 1024 took 4.79 ms with it against 3.78 ms
-// without binning.
+// without binning.  Bins too many for their edges to share the LDS, or that do not rise
+// with |n|^2 (a last bin below the first), are taken from the table.
 #pragma once
 #include <hip/hip_runtime.h>
 
 struct PkBinFn {
-  const int *edge = nullptr;  // nbins + 1 first |n|^2 of the bins (device memory)
+  const int *edge = nullptr;       // nbins + 1 first |n|^2 of the bins (device memory)
+  const int16_t *table = nullptr;  // bin of every |n|^2, -1 outside (device memory)
   int nbins = 0, logbins = 0;
   float a = 0.f, b = 0.f;  // estimate: a |n| + b, or a log2 |n|^2 + b
 };

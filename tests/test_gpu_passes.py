@@ -249,3 +249,44 @@ def test_autotune_leaves_the_meshes_in_use(model, n, after):
     with pytest.raises(M.MGPUError, match="no force meshes"):
         g.mesh_to_particles()
     g.close()
+
+
+@pytest.mark.parametrize("tcols", [8, 16])
+@pytest.mark.parametrize("n", [8, 12, 16, 24, 48, 64, 96, 128])
+@pytest.mark.parametrize("bins", ["most", "more", "many", "falling"])
+def test_pofk_bins_by_table(n, tcols, bins, monkeypatch):
+    """The x passes with the bins' table, on both sides of its line (a third of columns times
+    points by the edges, one more by the table), far beyond it (16 n + 1) and for bins that
+    fall with |n|^2 (last bin below the first).
+    Mode counts equal the oracle's formula; the sizes with one transform stage (8, 12, 16)
+    have no other barrier between the cleared sums and the first of them added."""
+    ns = n // 2
+    nbins = {"most": n * tcols // 3, "more": n * tcols // 3 + 1, "many": 16 * n + 1, "falling": n // 2}[bins]
+    kmin, kmax = (n / 2.0, 1.0) if bins == "falling" else (0.0, float(n))
+    plain = M.make_params
+
+    def with_range(*a):  # the binding itself asks for no last bin below the first
+        p = plain(*a)
+        p.pofk_kmin, p.pofk_kmax = kmin, kmax
+        return p
+
+    monkeypatch.setattr(M, "make_params", with_range)
+    pos = lattice_particles(ns, BOX, amp=1.5, seed=n, clustered=ns > 4)
+    print("n, tcols, bins =", n, tcols, bins, flush=True)
+    mg = dict(a=0.7, coupling=1 / 3, mass2=2e4, phi_crit=3e-8, dgp_fac=0.0, rsmooth=2.0, geff=1.0)
+    c = O.cfg(n, ns, BOX, OM)
+    dk = O.deposit(c, pos)
+    O.fft_r2c_3d(n, dk)
+    rp, rk, rn = O.pofk(c, dk, nbins, 0, kmin, kmax, 0)
+    ok = (rn > 0) & (rk > 0)
+    assert ok.any()
+    for mkw in ({}, dict(model=M.FOFR, mg_active=1, include_screening=1)):
+        g = M.MGPU(n, ns, BOX, OM, pofk_nbins=nbins, pofk_subtract_shotnoise=0, **mkw)
+        g.set_fft_tile(0, tcols)
+        g.set_particles(pos)
+        g.pm_density(pofk=True)
+        for pk, kk, nm in (g.pm_density(pofk=True), g.get_displacements(mg=M.MG(**mg) if mkw else None, pofk=True)[1]):
+            assert np.array_equal(nm, rn)
+            np.testing.assert_allclose(kk[ok], rk[ok], rtol=1e-12)
+            np.testing.assert_allclose(pk[ok], rp[ok], rtol=1e-3)
+        g.close()

@@ -110,3 +110,47 @@ if not {sd}:
     fails("{kernel}", M.MGPU.batch_ic, ms, [1, 2], pk)
     assert F.fake_pending() == 0
 """)
+
+
+@pytest.mark.parametrize("n,tcols,nbins", [(1024, 16, 512), (1024, 16, 1876), (1024, 16, 3800), (1024, 8, 12000), (2048, 8, 3500),
+                                           (128, 16, 18000), (64, 8, 19800)])
+def test_pofk_stays_in_the_x_pass(fake, n, tcols, nbins):
+    """Every number of bins whose sums fit the LDS beside the tile of columns is binned by the x
+    pass, alone and in the fused step of every model (unscreened LCDM's takes 8 columns)."""
+    fake(f"""
+n, tcols, nbins = {n}, {tcols}, {nbins}
+mg = M.MG(a=0.7, coupling=0.3, mass2=2e4, phi_crit=3e-8, dgp_fac=0.05, rsmooth=2.0, geff=1.0)
+plain = M.make_params
+def falling(*a):  # the last bin below the first, which the binding itself does not ask for
+    p = plain(*a)
+    p.pofk_kmin, p.pofk_kmax = float(n), 1.0
+    return p
+for kw, params in ((dict(), plain), (dict(model=M.FOFR, mg_active=1, include_screening=1), plain), (dict(), falling)):
+    M.make_params = params
+    g = context(n, 16, pofk_nbins=nbins, **kw)
+    assert (g.p.pofk_kmax < g.p.pofk_kmin) == (params is falling)
+    g.set_fft_tile(0, tcols)
+    m = mg if kw.get("mg_active") else None
+    g.pm_density(pofk=True)
+    assert ran("k_pofk") >= 1
+    for call in (lambda: g.pm_density(pofk=True), lambda: g.get_displacements(mg=m, pofk=True)):
+        F.fake_reset()
+        call()
+        assert ran("k_pofk") == 0, (kw, nbins)
+    assert ran("k_col_fused") == (2 if m else 1)
+    g.close()
+""")
+
+
+def test_pofk_of_more_bins_than_the_x_pass_holds(fake):
+    """Beyond that, and without the table (more than 32767 bins), by a pass of its own."""
+    fake("""
+for n, nbins in ((1024, 13000), (32, 33000)):
+    g = context(n, 16, pofk_nbins=nbins)
+    g.pm_density(pofk=True)
+    for call in (lambda: g.pm_density(pofk=True), lambda: g.get_displacements(pofk=True)):
+        F.fake_reset()
+        call()
+        assert ran("k_pofk") >= 1 and ran("k_col_pofk") + ran("k_col_fused") == 0
+    g.close()
+""")
