@@ -19,6 +19,7 @@ std::vector<std::string> *capture = nullptr; // where a capture puts them
 std::vector<const void *> pending;           // pageable host memory of copies in flight
 std::string fail_at;                         // call or kernel to fail, once
 hipError_t last = hipSuccess;
+size_t to_host = 0;                          // bytes copied from the device
 struct Cfg { dim3 g, b; size_t sh; hipStream_t st; };
 std::vector<Cfg> cfgs;
 
@@ -54,13 +55,14 @@ hipError_t handle(T *h) {
 
 extern "C" {
 // ---- the tests' handles
-void fake_reset() { ran.clear(); }
+void fake_reset() { ran.clear(); to_host = 0; }
 void fake_fail(const char *what) { fail_at = what; }
 int fake_ran(const char *kernel) {
   int n = 0;
   for (auto &s : ran) n += s.find(kernel) != std::string::npos;
   return n;
 }
+long fake_to_host() { return (long)to_host; }
 int fake_pending() { return (int)pending.size(); }
 
 // ---- registration and launches
@@ -122,6 +124,7 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hip
   if (fails("hipMemcpyAsync")) return last;
   const void *host = k == hipMemcpyHostToDevice ? s : d;
   if (!inside(host, pinned)) pending.push_back(host);
+  if (k == hipMemcpyDeviceToHost) to_host += n;
   memcpy(d, s, n);
   return hipSuccess;
 }

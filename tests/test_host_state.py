@@ -154,3 +154,17 @@ for n, nbins in ((1024, 13000), (32, 33000)):
         assert ran("k_pofk") >= 1 and ran("k_col_pofk") + ran("k_col_fused") == 0
     g.close()
 """)
+
+
+@pytest.mark.parametrize("nbins", [16, 500, 5000])
+def test_pofk_comes_back_without_a_copy(fake, nbins):
+    """The bin sums of P(k) and of the multipoles are stored to the host by a kernel, which
+    adds the x pass's sets first: no copy that grows with the sets."""
+    fake(f"""
+g = context(64, 32, pofk_nbins={nbins})
+for call in (lambda: g.pm_density(pofk=True), lambda: g.pm_density(pofk=True), lambda: g.get_displacements(pofk=True),
+             g.power_spectrum, lambda: g.rsd_power_spectrum(2, 0.1)):
+    F.fake_reset()
+    call()
+    assert F.fake_to_host() == 0 and ran("k_bins_to_host") == 1
+""")
