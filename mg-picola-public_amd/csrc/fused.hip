@@ -698,19 +698,18 @@ struct EpiF {
 
 // ---------------------------------------------------------------- host entry points
 
-// The edges' and the twiddles' LDS pays while the edges are at most a sixth of the tile
-// (every workgroup copies them) and no workgroup per CU is lost to them.  By the edges / by
-// the table: density and P(k) 8.87 / 9.29 ms at 1024 with 16 columns and 1024 bins (a 32nd),
-// 1.53 / 1.51 ms at 512, 16 columns and 4000 bins (a quarter), an LCDM step 1.65 / 1.74 ms at
-// 384 with 1024 bins (8 columns: a sixth); with a workgroup less 661 / 589 us at 384, 16
-// columns and 2500 bins.
+// The edges' and the twiddles' LDS pays while the edges are at most a sixth of the tile:
+// every workgroup copies them, and they cost workgroups per CU.  By the edges / by the
+// table: density and P(k) 8.87 / 9.29 ms at 1024 with 16 columns and 1024 bins (a 32nd),
+// 661 / 589 us at 384, 16 columns and 2500 bins (a fifth), 1.53 / 1.51 ms at 512, 16
+// columns and 4000 bins (a quarter); an LCDM step (8 columns) 28.2 / 28.5 ms at 1024 with
+// 1024 bins (a 16th), 1.65 / 1.74 ms at 384 with 1024 (a sixth), 4.63 / 4.04 ms at 512 with
+// 4000 (a half).
 int fused_pofk_by(const mgpu_ctx *ctx, int T) {
-  const size_t max = ctx->lds_max, l = pofk_table_lds(ctx, T);
-  if (ctx->pk_fn.edge && (size_t)ctx->p.pofk_nbins <= (size_t)ctx->N * T / 3) {
-    const size_t le = fft_col_lds(ctx->N, T) + pofk_lds(ctx->N, ctx->p.pofk_nbins, 1);
-    if (le <= max && (max / le == max / l || max / le >= 4)) return POFK_EDGES;
-  }
-  return ctx->pk_fn.table && l <= max ? POFK_TABLE : POFK_NONE;
+  if (ctx->pk_fn.edge && (size_t)ctx->p.pofk_nbins <= (size_t)ctx->N * T / 3 &&
+      fft_col_lds(ctx->N, T) + pofk_lds(ctx->N, ctx->p.pofk_nbins, 1) <= ctx->lds_max)
+    return POFK_EDGES;
+  return ctx->pk_fn.table && pofk_table_lds(ctx, T) <= ctx->lds_max ? POFK_TABLE : POFK_NONE;
 }
 
 int fused_green_x(mgpu_ctx *ctx, int mode, const float2 *a, const float2 *b, float2 *o0, float2 *o1, double p0,
