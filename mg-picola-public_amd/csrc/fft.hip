@@ -26,6 +26,15 @@ namespace {
 using namespace fftc;
 
 
+// col_at, but by a lane's own pointer where a stage's offsets need 64 bits: beside the
+// next tile's loads there are no registers for 64-bit offsets (2048: 22 to 32 of them went
+// to scratch, 19.4 and 21.4 ms a pass against 15.3 and 16.5).
+template <int L, int T, class P>
+__device__ __forceinline__ P &pass_at(P *base, size_t ls, int c, int j, int o) {
+  if constexpr (sizeof(typename ColOff<L, T>::type) > 4) return (base + (size_t)j * ls + c)[(size_t)o * ls];
+  else return col_at<L, T>(base, ls, c, j, o);
+}
+
 // TPB tiles per block, at outer indices blockIdx.y*TPB + i: the first-stage
 // loads of tile i+1 are issued before the stages of tile i run, so HBM reads
 // overlap the LDS exchanges of the previous tile.
@@ -47,7 +56,7 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_fft_col(float2 *__restric
   {
     const float2 *base = tile(0);
     first_loads<L, T, NT, true>(
-        pre, tid, [&](int c, int j, int o) { return col_at<L, T>(base, line_stride, c, j, o); });
+        pre, tid, [&](int c, int j, int o) { return pass_at<L, T>(base, line_stride, c, j, o); });
   }
   const float2 *twl = stw.to_lds(lds, tid);
 #pragma unroll
@@ -58,11 +67,11 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_fft_col(float2 *__restric
     if (i + 1 < TPB) {
       const float2 *nb = tile(i + 1);
       first_loads<L, T, NT, true>(
-          pre, tid, [&](int c, int j, int o) { return col_at<L, T>(nb, line_stride, c, j, o); });
+          pre, tid, [&](int c, int j, int o) { return pass_at<L, T>(nb, line_stride, c, j, o); });
     }
     float2 *base = tile(i);
-    auto ld = [&](int c, int j, int o) { return col_at<L, T>(base, line_stride, c, j, o); };
-    auto st = [&](int c, int j, int o, float2 v) { col_at<L, T>(base, line_stride, c, j, o) = v; };
+    auto ld = [&](int c, int j, int o) { return pass_at<L, T>(base, line_stride, c, j, o); };
+    auto st = [&](int c, int j, int o, float2 v) { pass_at<L, T>(base, line_stride, c, j, o) = v; };
     fft_stages<L, T, NT, SIGN, 1, T, true, false, 1, false, true>(lds, twl, 1, tid, ld, st, cur);
     if (i + 1 < TPB) __syncthreads();  // the next tile's first exchange reuses the LDS
   }
