@@ -363,8 +363,10 @@ __global__ __launch_bounds__(col_threads(L, T), tw_in_lds(L) && EDGES ? 4 : 1) v
   constexpr int NT = col_threads(L, T), E = col_ept(L, T);
   // The forward's outputs are handed to the inverse in registers (its stages reversed);
   // with delta(k) to add at 16 elements per thread those registers spill (1024: 4.94
-  // against 4.69 ms, 256: 96 against 82 us), and the outputs go through LDS instead.
-  constexpr bool kHand = FWD == FWD_DENSITY || E <= 12;
+  // against 4.69 ms, 256: 96 against 82 us), and the outputs go through LDS instead.  24
+  // elements have twice the registers, and it is the way through LDS that spills (68 and
+  // more of them; 1536: 24.4 against 32.1 ms).
+  constexpr bool kHand = FWD == FWD_DENSITY || E != 16;
   constexpr int RX = stage_radix(L, E, 1, kHand), MX = L / RX;  // the inverse's first stage
   constexpr int N = L;
   const int tid = threadIdx.x;
