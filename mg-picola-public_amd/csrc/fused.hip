@@ -449,8 +449,15 @@ enum { SCREEN_POTENTIAL = 0, SCREEN_DENSITY = 1 };
 //   SCREEN_DENSITY (DGP; src/mg.h:235-244, src/user_defined_functions.h:757-773):
 //       delta_eff = delta * p0 * 2 (sqrt(1 + f) - 1) / f, f = p1 (1 + delta_R), 1 if f < 1e-5
 //                                                                   (p0 = coupling, p1 = dgp_fac)
+// Four waves per SIMD (128 registers) up to 1024; three where the row's last radix is 16
+// (512: 12 to 14 registers spilled at four, 473 -> 442 us with the potential, 517 -> 485
+// with the density), one beyond, where a row has a workgroup's registers.
+template <int N>
+constexpr int screen_waves() {
+  return N > 1024 ? 1 : last_radix(N / 2, elems_per_thread(N / 2)) == 16 ? 3 : 4;
+}
 template <int N, int KIND>
-__global__ __launch_bounds__(RowCfg<N>::NT, N <= 1024 ? 4 : 1) void k_z_screen(float2 *buf, const float2 *__restrict__ dx, int HP,
+__global__ __launch_bounds__(RowCfg<N>::NT, screen_waves<N>()) void k_z_screen(float2 *buf, const float2 *__restrict__ dx, int HP,
                                                              size_t nrows, const float2 *__restrict__ tw, float p0,
                                                              float p1, size_t zs) {
   buf = zbuf(buf, zs);

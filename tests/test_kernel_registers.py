@@ -33,6 +33,7 @@ def spilled(tmp_path_factory):
 @pytest.mark.parametrize("kernel,most", [
     (r"k_fft_col<2048, 8, -?1, 2>", 6),  # the plain column passes of the largest mesh
     (r"k_col_fused<1536, 8, [12], 0, true>", 2),  # the force pairs of screened models
+    (r"k_z_screen<512, [01]>", 0),  # the screening rows of the learned runs' coarse mesh
 ])
 def test_spilled_registers(spilled, kernel, most):
     found = {k: v for k, v in spilled.items() if re.fullmatch(kernel, k)}
