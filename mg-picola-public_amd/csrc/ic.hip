@@ -644,12 +644,17 @@ struct StreamWait {
 // The seed tables of count realizations (ctx's, at the batch stride) into table (on the
 // device): the states the chunks of each stream start from go to slot 1, which the
 // initial conditions overwrite afterwards.  A chunk is 16 advances of 12 values, or
-// what makes 2048 chunks: the host's jump takes 0.35 us, a thread's advance 3.4 us.
+// what makes 2048 chunks; in small tables, which the chunks' own length would hold up, as
+// many as balance the host's jumps (0.35 us each) with a thread's advances (3.4 us each):
+// scale-dependent initial conditions 236 -> 145 us at 16, 262 -> 180 us at 32 (202 and 231
+// us with the table made by the host).
 // inverted (or nullptr): the realizations' inversion flags, one behind each table.
 int seed_tables(mgpu_ctx *ctx, int count, const unsigned long *seeds, const int *inverted, unsigned *table,
                 std::vector<double> &st) {
   const int N = ctx->N;
-  const unsigned advances = cdiv((size_t)N * N, 12), adv = std::max(16u, cdiv(advances, 2048)), n = cdiv(advances, adv);
+  const unsigned advances = cdiv((size_t)N * N, 12);
+  const unsigned adv = std::max({1u, std::min(16u, (unsigned)std::lround(std::sqrt(advances / 9.7))), cdiv(advances, 2048)});
+  const unsigned n = cdiv(advances, adv);
   const size_t len = 13 * (size_t)n + 1;
   if (len * sizeof(double) > ctx->slot_elems * sizeof(float2))
     return mgpu_fail(ctx, MGPU_E_INVALID, "seed states do not fit a mesh slot");
