@@ -775,18 +775,19 @@ int fused_x_pair(mgpu_ctx *ctx, int fwd, int mode, const float2 *in, float2 *kou
   }
 }
 
-int fused_dual_y(mgpu_ctx *ctx, float2 *buf, float2 *oy) {
+// inverse y pass: buf <- Y[buf], oy <- Y[i n_y buf], for the meshes beyond kForceYOne
+static int fused_dual_y(mgpu_ctx *ctx, float2 *buf, float2 *oy) {
   const double modes = (double)ctx->N * ctx->N * (ctx->N / 2 + 1);
   KScope ks(ctx, MGPU_K_FFT_DUAL, 8.0 * modes * 3);
   switch (ctx->N) {
-#define X(S) \
-  case S:    \
-    return by_tile<S, DualF>(ctx, buf, oy);
+#define X(S)                                                                \
+  case S:                                                                   \
+    if constexpr (S > kForceYOne) return by_tile<S, DualF>(ctx, buf, oy);   \
+    break;
     MGPU_FFT_SIZES(X)
 #undef X
-    default:
-      return mgpu_fail(ctx, MGPU_E_INVALID, "unsupported FFT size");
   }
+  return mgpu_fail(ctx, MGPU_E_INVALID, "unsupported FFT size");
 }
 
 int fused_force_y(mgpu_ctx *ctx, float2 *buf, float2 *oy, float2 *other) {
@@ -796,14 +797,14 @@ int fused_force_y(mgpu_ctx *ctx, float2 *buf, float2 *oy, float2 *other) {
     const double modes = (double)ctx->N * ctx->N * (ctx->N / 2 + 1);
     KScope ks(ctx, MGPU_K_FFT_DUAL, 8.0 * modes * 5);
     switch (ctx->N) {
-#define X(S) \
-  case S:    \
-    if constexpr (S <= kForceYOne) return by_tile<S, ForceYF>(ctx, buf, oy, other);
+#define X(S)                                                                          \
+  case S:                                                                             \
+    if constexpr (S <= kForceYOne) return by_tile<S, ForceYF>(ctx, buf, oy, other);   \
+    break;
       MGPU_FFT_SIZES(X)
 #undef X
-      default:
-        return mgpu_fail(ctx, MGPU_E_INVALID, "unsupported FFT size");
     }
+    return mgpu_fail(ctx, MGPU_E_INVALID, "unsupported FFT size");
   }
   int rc = fused_dual_y(ctx, buf, oy);
   return rc ? rc : fft_pass_col(ctx, &ctx->fft, other, 1, 0);

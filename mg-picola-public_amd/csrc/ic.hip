@@ -797,7 +797,7 @@ static int ic_read_displacements(mgpu_ctx *ctx, const float2 *X, double scale, i
     return MGPU_OK;
   }
   for (int a = 0; a < 3; a++) {
-    if ((rc = lpt_x_pass(ctx, X, ctx->slot[3], nullptr, nullptr, LptFields{1, {a}, {-1}, 1.0}))) return rc;
+    if ((rc = lpt_x_pass(ctx, X, ctx->slot[3], nullptr, nullptr, LptFields{1, {a}, {-1}}))) return rc;
     if ((rc = fft_pass_col(ctx, &ctx->fft, ctx->slot[3], 1, 0))) return rc;
     if ((rc = fft_pass_z(ctx, &ctx->fft, ctx->slot[3], 0))) return rc;
     if ((rc = readout(ctx, ctx->slot[3], scale, ctx->lpt[o] + (size_t)a * ctx->np))) return rc;
@@ -814,15 +814,15 @@ int ic_lpt_from_delta(mgpu_ctx *ctx, float2 *cd) {
   float2 *s = ctx->slot[1], *d1 = ctx->slot[2], *d2 = ctx->slot[3];
   // displacement gradients -> 2LPT source, built in slot 1 with two more slots of work
   // space: the diagonal ones, two off the diagonal, the last one and the r2c
-  if ((rc = lpt_x_pass(ctx, cd, s, d1, d2, LptFields{3, {0, 1, 2}, {0, 1, 2}, 1.0}))) return rc;
+  if ((rc = lpt_x_pass(ctx, cd, s, d1, d2, LptFields{3, {0, 1, 2}, {0, 1, 2}}))) return rc;
   for (float2 *d : {s, d1, d2})
     if ((rc = fft_pass_col(ctx, plan, d, 1, 0))) return rc;
   if ((rc = lpt_source_pass(ctx, LPT_DIAG, s, d1, d2))) return rc;
-  if ((rc = lpt_x_pass(ctx, cd, d1, d2, nullptr, LptFields{2, {0, 0}, {1, 2}, 1.0}))) return rc;
+  if ((rc = lpt_x_pass(ctx, cd, d1, d2, nullptr, LptFields{2, {0, 0}, {1, 2}}))) return rc;
   for (float2 *d : {d1, d2})
     if ((rc = fft_pass_col(ctx, plan, d, 1, 0))) return rc;
   if ((rc = lpt_source_pass(ctx, LPT_OFF2, s, d1, d2))) return rc;
-  if ((rc = lpt_x_pass(ctx, cd, d1, nullptr, nullptr, LptFields{1, {1}, {2}, 1.0}))) return rc;
+  if ((rc = lpt_x_pass(ctx, cd, d1, nullptr, nullptr, LptFields{1, {1}, {2}}))) return rc;
   if ((rc = fft_pass_col(ctx, plan, d1, 1, 0))) return rc;
   if ((rc = lpt_source_pass(ctx, LPT_OFF1, s, d1, nullptr))) return rc;
   if ((rc = fft_pass_col(ctx, plan, s, 1, 1))) return rc;

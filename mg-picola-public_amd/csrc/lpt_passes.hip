@@ -46,7 +46,7 @@ __global__ __launch_bounds__(col_threads(L, T), tw_in_lds(L) ? 4 : 1) void k_lpt
   auto ld = [&](int, int, int) { return make_float2(0.f, 0.f); };
   for (int n = 0; n < f.n; ++n) {
     const int a = f.a[n], b = f.b[n];
-    const double scale = b < 0 ? f.sign / kf : f.sign;
+    const double scale = b < 0 ? 1.0 / kf : 1.0;
     int ny = kint(by, L);
     anew(ny);
     float2 p[E];

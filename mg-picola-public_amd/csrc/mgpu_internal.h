@@ -212,10 +212,9 @@ struct PhaseTimer {
 };
 
 // ---------------------------------------------------------------- LPT spectra in FFT passes (lpt_passes.hip)
-// n <= 3 fields sign i k_a/k^2 X, or with b >= 0 i k_b times that
+// n <= 3 fields i k_a/k^2 X, or with b >= 0 i k_b times that
 struct LptFields {
   int n, a[3], b[3];
-  double sign;
 };
 enum { LPT_DIAG, LPT_OFF2, LPT_OFF1 };
 int lpt_x_pass(mgpu_ctx *ctx, const float2 *cd, float2 *o0, float2 *o1, float2 *o2, const LptFields &f);
@@ -262,9 +261,7 @@ enum { FUSED_GREEN_FORCE = 0, FUSED_GREEN_LAPLACE = 1, FUSED_GREEN_SMOOTH = 2 };
 //   SMOOTH   o0 = X[S W(|n| p1) p0]                                  (p0 = 1/N^3, p1 = 2 pi R/Box)
 int fused_green_x(mgpu_ctx *ctx, int mode, const float2 *a, const float2 *b, float2 *o0, float2 *o1, double p0,
                   double p1, int filter);
-// inverse y pass: buf <- Y[buf], oy <- Y[i n_y buf]
-int fused_dual_y(mgpu_ctx *ctx, float2 *buf, float2 *oy);
-// fused_dual_y and the inverse y pass of other
+// inverse y passes of the force: buf <- Y[buf], oy <- Y[i n_y buf], other <- Y[other]
 int fused_force_y(mgpu_ctx *ctx, float2 *buf, float2 *oy, float2 *other);
 // forward x pass then times coupling n^2/(n^2 + massterm2)
 int fused_epi_phi_x(mgpu_ctx *ctx, float2 *buf, double coupling, double massterm2);
