@@ -261,7 +261,10 @@ int create_ctx(const mgpu_params *p, mgpu_ctx **out, mgpu_arena *arena, char *sh
   if (hipGetDevice(&ctx->device) != hipSuccess) return fail(mgpu_fail(ctx, MGPU_E_HIP, "hipGetDevice failed"));
   if ((rc = ic_scratch_init(ctx))) return fail(rc);
   hipDeviceProp_t pr;
-  if (hipGetDeviceProperties(&pr, ctx->device) == hipSuccess) ctx->lds_max = pr.sharedMemPerBlock;
+  if (hipGetDeviceProperties(&pr, ctx->device) == hipSuccess) {
+    ctx->lds_max = pr.sharedMemPerBlock;
+    ctx->cus = pr.multiProcessorCount;
+  }
   if (!ctx->stream && hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess)
     return fail(mgpu_fail(ctx, MGPU_E_HIP, "stream creation failed"));
   if ((rc = fft_plan_init(ctx, &ctx->fft, ctx->N, MGPU_FFT_TCOLS))) return fail(rc);

@@ -449,7 +449,6 @@ __global__ __launch_bounds__(kBlock) void k_lpt_fold(const float2 *__restrict__ 
 // What bounds it: the slices of 1000 nodes take 48 KB, so blocks of 256 threads left
 // three waves per SIMD, and a row of a 128 lattice 63 of the 256 lanes.
 constexpr int kFoldNT = 512;
-constexpr unsigned kFoldRounds = 2;
 template <int MF, int NS>
 __global__ __launch_bounds__(kFoldNT, 4) void k_lpt_fold_gs(const float2 *__restrict__ cd1,
                                                             const float2 *__restrict__ cd2,
@@ -904,8 +903,10 @@ int launch_fold_gs(mgpu_ctx *ctx, const SliceFold &f, float lnkf, float ikf, flo
   int lpw = 16;
   while (lpw < Np / 2 && lpw < kFoldNT) lpw *= 2;
   // as many blocks as the LDS and the registers keep resident, each copying the slices once
+  // (both slots at 512 / 768 with 256 particles a side: 912 / 1412 us; twice as many blocks
+  // 1004 / 1648 us, four times 929 / 1431; up to 256 the three are equal)
   const unsigned per_cu = (unsigned)std::max<size_t>(1, std::min<size_t>(2, ctx->lds_max / std::max<size_t>(lds, 1)));
-  const unsigned nb = (unsigned)std::min<size_t>(cdiv((size_t)Np * Np, kFoldNT / lpw), 256 * per_cu * kFoldRounds);
+  const unsigned nb = (unsigned)std::min<size_t>(cdiv((size_t)Np * Np, kFoldNT / lpw), (size_t)ctx->cus * per_cu);
   hipLaunchKernelGGL((k_lpt_fold_gs<MF, NS>), dim3(nb), dim3(kFoldNT), lds, ctx->stream, ctx->cdelta[0],
                      ctx->cdelta[1], (const float4 *)ctx->slice_buf, gs, lnkf, ctx->N, ctx->HP, Np,
                      ctx->fft_lattice.hp, ctx->N / Np, ikf, lpw, out, nl);

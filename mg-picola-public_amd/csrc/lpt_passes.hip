@@ -94,8 +94,11 @@ __device__ __forceinline__ void z_c2r_regs(float2 *lds, const float2 *f, int HP,
 // Bound by memory: the source and the fields cross it once; the c2r of each field and
 // the sweeps over real meshes that formed the products crossed it more often.  The three
 // launches at 384: 0.76 ms, where six c2r, four sweeps and the r2c took 1.52 ms.
+// Three waves per SIMD up to 1024: with none asked for / three / four, DIAG 82 / 73 / 114 us
+// at 256, 721 / 678 / 826 at 512 and 6.33 / 6.23 / 6.88 ms at 1024, OFF2 472 / 481 / 713 us
+// at 512, OFF1 411 / 415 / 409.  Beyond, rows have their workgroup's registers.
 template <int N, int MODE>
-__global__ __launch_bounds__(RowCfg<N>::NT, N > 1024 ? 1 : MODE == LPT_OFF1 && N <= 512 ? 4 : 3) void k_lpt_source(float2 *s, const float2 *d1,
+__global__ __launch_bounds__(RowCfg<N>::NT, N > 1024 ? 1 : 3) void k_lpt_source(float2 *s, const float2 *d1,
                                                                                 const float2 *d2, int HP, size_t nrows,
                                                                                 const float2 *__restrict__ tw,
                                                                                 size_t zs) {

@@ -70,6 +70,7 @@ struct mgpu_ctx {
   hipStream_t stream = nullptr;
   int device = 0;
   size_t lds_max = 65536;
+  int cus = 256;                    // compute units of the device
 
   // particles, SoA [3][np]
   float *pos = nullptr, *vel = nullptr, *disp = nullptr;
