@@ -290,3 +290,68 @@ def test_pofk_bins_by_table(n, tcols, bins, monkeypatch):
             np.testing.assert_allclose(kk[ok], rk[ok], rtol=1e-12)
             np.testing.assert_allclose(pk[ok], rp[ok], rtol=1e-3)
         g.close()
+
+
+@pytest.mark.parametrize("n,ns", [(256, 128), (384, 192)])
+def test_lpt_passes_against_the_oracle_at_larger_meshes(n, ns):
+    """As test_lpt_passes_and_fold, at the 16 and 12 elements per thread of 256 and 384."""
+    pk = 1000.0 / (1.0 + np.arange(M.n2_table_len(n), dtype=np.float64)) ** 1.5
+    pk[0] = 0.0
+    print("n, ns =", n, ns, flush=True)
+    g = M.MGPU(n, ns, BOX, OM)
+    g.ic_displacement_fields(4001, pk)
+    c = O.cfg(n, ns, BOX, OM)
+    za, lp = O.ic_displacements(c, O.ic_delta(c, 4001, pk), 0)
+    assert rel_err(g.get_lpt(0), za) < 1e-5
+    assert rel_err(g.get_lpt(1), lp) < 2e-5
+    g.close()
+
+
+@pytest.mark.parametrize("n,ns,tcols", [(256, 8, 8), (512, 8, 8), (512, 256, 16), (768, 8, 8), (768, 384, 16), (1024, 8, 8),
+                                        (1024, 512, 16), (1536, 8, 8), (1536, 512, 8), (2048, 8, 8)])
+def test_initial_conditions_of_a_few_modes(n, ns, tcols):
+    """Power in |n|^2 <= 3 alone: the displacements have |n_a| <= 1 and, through the products of
+    the source, <= 2, so every lattice of 8 points a side holds them exactly.  From the first
+    order field's modes (one delta(k) for all three components) the second order follows in
+    FP64, with numpy.  Read out of the mesh (ns = 8) or folded; the bounds are those of the
+    oracle comparisons, 1e-5 and 2e-5 of the field maximum."""
+    pk = np.zeros(M.n2_table_len(n))
+    pk[1:4] = 1000.0
+    print("n, ns, tcols =", n, ns, tcols, flush=True)
+    g = M.MGPU(n, ns, BOX, OM)
+    g.set_fft_tile(0, tcols)
+    g.ic_displacement_fields(4001, pk)
+    step = ns // 8
+    first, second = (np.ascontiguousarray(g.get_lpt(s).reshape(3, ns, ns, ns)[:, ::step, ::step, ::step]).astype(np.float64)
+                     for s in (0, 1))
+    g.close()
+    k1 = np.fft.fftfreq(8, 1 / 8.0) * 2 * np.pi / BOX
+    k = np.array(np.meshgrid(k1, k1, k1, indexing="ij"))
+    k2 = (k * k).sum(0)
+    k2[0, 0, 0] = 1.0
+    psi = np.fft.fftn(first, axes=(1, 2, 3))
+    delta = -1j * (k * psi).sum(0)
+    delta[np.round(k2 * (BOX / 2 / np.pi) ** 2) > 3] = 0
+    assert np.abs(delta).max() > 0
+    real = lambda x: np.fft.ifftn(x).real
+    want = np.array([real(1j * k[a] / k2 * delta) for a in range(3)])
+    assert rel_err(first, want) < 1e-5
+    phi = {(a, b): real(-k[a] * k[b] / k2 * delta) for a in range(3) for b in range(a, 3)}
+    source = np.fft.fftn(sum(phi[a, a] * phi[b, b] - phi[a, b] ** 2 for a, b in ((0, 1), (0, 2), (1, 2))))
+    want = np.array([real(3.0 / 7.0 * 1j * k[a] / k2 * source) for a in range(3)])
+    assert np.abs(want).max() > 0
+    assert rel_err(second, want) < 2e-5
+
+
+def test_seed_table_of_long_chunks():
+    """768: chunks of 27 advances (16 up to 512), with fixed amplitudes against the oracle's
+    delta(k); see test_seed_table_by_chunks."""
+    n = 768
+    pk = 100.0 / (1.0 + np.arange(M.n2_table_len(n), dtype=np.float64))
+    g = M.MGPU(n, n // 2, BOX, OM, scale_dependent=1)
+    g.ic_displacement_fields(5001, pk, amplitude_fixed=1)
+    got = g.get_mesh(M.MESH_CDELTA1)
+    g.close()
+    want = O.complex_view(O.ic_delta(O.cfg(n, n // 2, BOX, OM), 5001, pk, 0, 1, 0), n)
+    top = np.abs(want).max()
+    assert top > 0 and max(np.abs(got[i] - want[i]).max() for i in range(n)) < 1e-6 * top
