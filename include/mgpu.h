@@ -89,7 +89,11 @@ typedef struct {
   double geff;             /* GeffoverG(a, 0), JBD */
 } mgpu_mg;
 
-/* Binned power spectrum as compute_power_spectrum forms it (src/compute_pofk.c:71-236). */
+/* Binned power spectrum as compute_power_spectrum forms it (src/compute_pofk.c:71-236).
+ * Any number of bins is taken.  Where the sums fit the LDS beside a tile of columns the
+ * density's x pass bins them as it goes: at Nmesh 1024 up to 3839 bins with 16-column tiles
+ * and 12031 with 8 (mgpu_set_fft_tile; the fused step of LCDM always takes 8), at 2048 3583,
+ * and at most 32767.  More take unfused passes and one of their own over delta(k). */
 typedef struct {
   double *pofk;            /* [nbins] normalised P(k) [(Mpc/h)^3], shot noise handled */
   double *kmean;           /* [nbins] mean |k| of the bin [h/Mpc] */

@@ -1,6 +1,6 @@
 // FFT building blocks shared by the plain transforms (fft.hip) and the fused
-// spectral passes (fused.hip): radix 2/3/4/8/16 butterflies and the
-// register-resident Stockham stage recursion used by every pass kernel.
+// spectral passes (fused.hip, lpt_passes.hip): radix 2/3/4/8/12/16 butterflies
+// and the register-resident Stockham stage recursion used by every pass kernel.
 #pragma once
 
 #include "mgpu_internal.h"

@@ -13,7 +13,7 @@
 //   z screen pass            c2r of the potential (or smoothed density) row,
 //                            the real-space screening against the delta(x)
 //                            row, and the r2c of the effective density row, in
-//                            one kernel with the row kept in LDS;
+//                            one kernel, the row handed on in registers;
 //   epilogue x pass (fwd)    x transform followed by coupling n^2/(n^2 + m^2);
 //   z c2r with i n_z         (fft.hip) the z force component.
 // Integer wavenumbers follow the Forces convention n in (-N/2, N/2] (the
@@ -27,11 +27,12 @@ namespace {
 
 using namespace fftc;
 
-// Stores of the passes that write more than one mesh: past the caches from 384 on, where a
+// Stores of the dual y pass and of the x pass pairs: past the caches from 384 on, where a
 // mesh is larger than they keep until the next pass reads it, and with full 128-byte lines
-// (16 columns; half lines cost more than they gain).  Dual y pass / density pair: 146 / 165
-// -> 137 / 143 us at 384, 1.38 / 1.93 -> 1.20 / 1.80 ms at 768, 2.84 / 4.19 -> 2.80 / 4.15
-// ms at 1024; up to 256 the next pass finds the meshes in the caches.
+// (16 columns; half lines, as the 8 columns of the force pairs write, cost more than they
+// gain).  Dual y pass / density pair: 146 / 165 -> 137 / 143 us at 384, 1.38 / 1.93 -> 1.20 /
+// 1.80 ms at 768, 2.84 / 4.19 -> 2.80 / 4.15 ms at 1024; up to 256 the next pass finds the
+// meshes in the caches.
 template <int L, int T>
 __device__ __forceinline__ void put(float2 &p, float2 v) {
   if constexpr (L >= 384 && T == 16) {
@@ -328,8 +329,8 @@ __global__ __launch_bounds__(col_threads(L, T)) void k_col_pofk(float2 *buf, siz
   pl.flush(pk, fn, copies, tid);
 }
 
-// x pass pair: a forward x transform and, from its output in LDS, an inverse
-// x transform with a Green's / smoothing multiplier, so the spectrum between
+// x pass pair: a forward x transform and, from its output, an inverse x
+// transform with a Green's / smoothing multiplier, so the spectrum between
 // them is never written and read back.
 //   FWD_DENSITY  the density's forward x pass: delta(k) stored to kout (when
 //                not null) and its power binned into pk (when not null) as
