@@ -47,10 +47,10 @@ KERNEL_SYMBOL = {
     "fft_r2c": "k_fft_z_r2c<{N}>", "fft_c2r": "k_fft_z_c2r3<{N}>", "fft_col_fwd": "k_fft_col<{N}, 16, -1, 2>",
     "fft_col_inv": "k_fft_col<{N}, 16, 1, 2>", "fft_green": "k_col_green<{N}, 16, 0>",
     "fft_pot": "k_col_green<{N}, 16, 1>", "fft_dual": "k_col_dual<{N}, 16>", "fft_screen": "k_z_screen<{N}, 0>",
-    "fft_epi": "k_col_epi<{N}, 16>", "fft_pk": "k_col_pofk<{N}, 16>", "fold": "k_lpt_fold_gs<{m}, 2>",
+    "fft_epi": "k_col_epi<{N}, 16>", "fft_pk": "k_col_pofk<{N}, 16, true>", "fold": "k_lpt_fold_gs<{m}, 2>",
     "gather": "k_gather_tile<16>", "kick": "k_kick_drift<8>", "drift": "k_drift", "pofk": "k_pofk",
     "lpt": "k_fft_col<{Ns}, ...> + k_fft_z_c2r<{Ns}>",
-    "fft_xdens": "k_col_fused<{N}, 16, 0, 1>", "fft_xforce": "k_col_fused<{N}, 8, 1, 0>",
+    "fft_xdens": "k_col_fused<{N}, 16, 0, 1, true>", "fft_xforce": "k_col_fused<{N}, 8, 1, 0, true>",
 }
 
 
